@@ -23,12 +23,15 @@ extern "C" const char* afqmc_last_error(void) { return g_err; }
 
 namespace {
 
+// Every allocation ends with DEV_PAD unused bytes: the 16-byte operand loads of the
+// float64 GEMM and exchange may start on the last element of a row of odd length.
+constexpr size_t DEV_PAD = 16;
 template <typename T>
 int dalloc(afqmc_ctx* c, T** p, size_t count) {
   *p = nullptr;
   if (count == 0) return AFQMC_OK;
   const size_t bytes = count * sizeof(T);
-  HIP_TRY(hipMalloc((void**)p, bytes));
+  HIP_TRY(hipMalloc((void**)p, bytes + DEV_PAD));
   c->device_bytes += (int64_t)bytes;
   return AFQMC_OK;
 }

@@ -522,7 +522,7 @@ int launch_taylor_grouped(hipStream_t s, int kind, int nkgv, int ct, const Taylo
 // bm: 64 or 128 square tiles; out: 0 float64 C, 1 float32 C (split-bf16 only)
 int launch_gemm_bf16x3_grouped(hipStream_t s, int bm, int out, const GemmArgs* args,
                                const int* start, int nprob, int nblocks);
-int launch_gemm_f64_grouped(hipStream_t s, int bm, bool vec2, const GemmArgs* args,
-                            const int* start, int nprob, int nblocks);
+int launch_gemm_f64_grouped(hipStream_t s, int bm, const GemmArgs* args, const int* start,
+                            int nprob, int nblocks);
 int launch_gemm_f32_grouped(hipStream_t s, int bm, bool vec2, const GemmArgs* args,
                             const int* start, int nprob, int nblocks);

@@ -8,26 +8,32 @@
 //   B operand: lane l holds B[l / 16][l % 16]
 //   D (double4): lane l, element r holds D[l / 16 + 4 r][l % 16]
 //
-// Tiles of BM x BN with BK = 16, four waves (2 x 2), operands staged k-major in LDS
-// (double buffered, register prefetch of the next k-tile).  Optional split-K: grid.y
-// splits the K range and each split writes alpha * partial product to its own slice
-// C + split * c_split_stride (beta must be 0); consumers sum the slices in order.
+// Tiles of BM x BN with BK = 16, four waves (2 x 2), double buffered in LDS with the next
+// k-tile's loads in flight in registers.  Optional split-K: grid.y splits the K range and
+// each split writes alpha * partial product to its own slice C + split * c_split_stride
+// (beta must be 0); consumers sum the slices in order.
+//
+// What bounds it: one 16 x 16 x 4 MFMA takes 64 cycles, so four 4 x 4-tile waves need 4096
+// MFMA cycles per k-tile and everything else has to stay off that path.
+//   - Operand loads are 16-byte and unconditional, from clamped rows and k (a masked load
+//     compiles to a branch with its own wait, which serialised the loads of a k-tile); k
+//     past the range is zeroed on both operands when the registers go to LDS.
+//   - LDS tiles keep the row-major order of memory (16 doubles = 8 chunks of 16 bytes per
+//     row), so staging is one 16-byte store per load instead of a scatter of 8-byte ones,
+//     and an operand read is one 16-byte chunk per lane: k = 2 c and 2 c + 1 of chunk
+//     c = 4 ks + lane / 16, which feeds two MFMAs (any order of k serves, as long as both
+//     operands share it).  Chunk c of row r sits at c ^ ((r >> 1) & 7): the sixteen rows
+//     of one chunk then cover all 64 banks once.
 #include "common.h"
 
 namespace {
 
 constexpr int GEMM_BK = 16;
-constexpr int GEMM_PAD = 16;  // row stride == 16 (mod 32) doubles: k and k+1 rows hit disjoint bank halves
-// Element (k, m) of a k-major LDS tile sits at column m ^ gemm_swz<VEC>(k).  The MFMA
-// operand reads (16 consecutive m at k and k + 1 per 32 lanes) see the same banks as
-// without it: k and k + 1 share the swizzle, which keeps 16-aligned groups of m
-// together.  The staging stores (8 or 16 k rows x 4 or 2 m per 32 lanes) without it put
-// the rows of one k parity on one bank pair, an 8-way conflict; with it the 32 lanes
-// meet 32 bank pairs.
-template <int VEC>
-__device__ inline int gemm_swz(int k) { return ((k >> 1) & 7) << (VEC == 2 ? 2 : 1); }
+// 16 bytes at any 8-byte boundary (rows of odd length)
+typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
+typedef double d2_t __attribute__((ext_vector_type(2)));
 
-template <int BM, int BN, int WM, int WN, int VEC>
+template <int BM, int BN, int WM, int WN>
 __device__ __forceinline__ void gemm_nt_f64_body(
     int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
     const double* __restrict__ B, int ldb, double beta, double* __restrict__ C, int ldc,
@@ -35,17 +41,17 @@ __device__ __forceinline__ void gemm_nt_f64_body(
     const int by) {
   constexpr int NT = 256;
   constexpr int BK = GEMM_BK;
+  constexpr int CH = BK / 2;  // 16-byte chunks per row
   constexpr int TM = BM / WM / 16;
   constexpr int TN = BN / WN / 16;
-  constexpr int KT = BK / VEC;             // threads along k per row
-  constexpr int RSTEP = NT / KT;           // rows covered per load pass
-  constexpr int A_LD = BM / RSTEP;         // vector loads of A per thread per k-tile
+  constexpr int RSTEP = NT / CH;  // rows covered per load pass
+  constexpr int A_LD = BM / RSTEP;
   constexpr int B_LD = BN / RSTEP;
   static_assert(WM * WN == 4, "four waves");
   static_assert(A_LD >= 1 && B_LD >= 1, "tile too small");
 
-  __shared__ double As[2][BK][BM + GEMM_PAD];
-  __shared__ double Bs[2][BK][BN + GEMM_PAD];
+  __shared__ d2_t As[2][BM * CH];
+  __shared__ d2_t Bs[2][BN * CH];
 
   // XCD-aware block -> tile map (contiguous tile runs per XCD; the larger operand's
   // panels are the shared ones)
@@ -61,48 +67,35 @@ __device__ __forceinline__ void gemm_nt_f64_body(
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave % WM, wn = wave / WM;
-  const int lk = (t % KT) * VEC, lr = t / KT;
+  const int lch = t % CH, lr = t / CH;
 
-  double ra[A_LD][VEC], rb[B_LD][VEC];
+  // rows past M or N read the last row: their products are never stored
+  const double* Ab = A + (int64_t)m0 * lda;
+  const double* Bb = B + (int64_t)n0 * ldb;
+  int aoff[A_LD], boff[B_LD];
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) aoff[i] = min(lr + i * RSTEP, M - 1 - m0) * lda;
+#pragma unroll
+  for (int i = 0; i < B_LD; ++i) boff[i] = min(lr + i * RSTEP, N - 1 - n0) * ldb;
+  d2_t ra[A_LD], rb[B_LD];
+  // chunks past kend read elements kend - 1 and kend (the operands' allocations end with
+  // at least one element of padding)
   auto load_tile = [&](int k0) {
-    const int k = k0 + lk;
-    const bool kok = k < kend;  // VEC == 2 needs even k ranges (checked at launch)
+    const int k = min(k0 + 2 * lch, kend - 1);
 #pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      const int r = m0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < M && kok) v = *reinterpret_cast<const double2*>(A + (int64_t)r * lda + k);
-        ra[i][0] = v.x;
-        ra[i][VEC - 1] = v.y;
-      } else {
-        ra[i][0] = (r < M && kok) ? A[(int64_t)r * lda + k] : 0.0;
-      }
-    }
+    for (int i = 0; i < A_LD; ++i) ra[i] = *reinterpret_cast<const d2u_t*>(Ab + (aoff[i] + k));
 #pragma unroll
-    for (int i = 0; i < B_LD; ++i) {
-      const int r = n0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < N && kok) v = *reinterpret_cast<const double2*>(B + (int64_t)r * ldb + k);
-        rb[i][0] = v.x;
-        rb[i][VEC - 1] = v.y;
-      } else {
-        rb[i][0] = (r < N && kok) ? B[(int64_t)r * ldb + k] : 0.0;
-      }
-    }
+    for (int i = 0; i < B_LD; ++i) rb[i] = *reinterpret_cast<const d2u_t*>(Bb + (boff[i] + k));
   };
-  auto store_tile = [&](int buf) {
+  const int sidx = lr * CH + (lch ^ ((lr >> 1) & 7));  // (RSTEP is a multiple of 16 rows)
+  auto store_tile = [&](int buf, int k0) {
+    const bool ok0 = k0 + 2 * lch < kend, ok1 = k0 + 2 * lch + 1 < kend;
 #pragma unroll
     for (int i = 0; i < A_LD; ++i)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        As[buf][lk + v][(lr + i * RSTEP) ^ gemm_swz<VEC>(lk + v)] = ra[i][v];
+      As[buf][sidx + i * RSTEP * CH] = d2_t{ok0 ? ra[i].x : 0.0, ok1 ? ra[i].y : 0.0};
 #pragma unroll
     for (int i = 0; i < B_LD; ++i)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        Bs[buf][lk + v][(lr + i * RSTEP) ^ gemm_swz<VEC>(lk + v)] = rb[i][v];
+      Bs[buf][sidx + i * RSTEP * CH] = d2_t{ok0 ? rb[i].x : 0.0, ok1 ? rb[i].y : 0.0};
   };
 
   double4_t acc[TM][TN];
@@ -114,30 +107,36 @@ __device__ __forceinline__ void gemm_nt_f64_body(
   const int nk = (kend - kbeg + BK - 1) / BK;
   if (nk > 0) {
     load_tile(kbeg);
-    store_tile(0);
+    store_tile(0, kbeg);
   }
   __syncthreads();
-  const int am = wm * (BM / WM) + (lane & 15);
-  const int bn = wn * (BN / WN) + (lane & 15);
-  const int kq = lane >> 4;
+  const int am = (wm * (BM / WM) + (lane & 15)) * CH;
+  const int bn = (wn * (BN / WN) + (lane & 15)) * CH;
+  const int kq = lane >> 4, sw = (lane >> 1) & 7;
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    if (kt + 1 < nk) load_tile(kbeg + (kt + 1) * BK);
+    const int knext = kbeg + (kt + 1) * BK;
+    if (kt + 1 < nk) load_tile(knext);
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      double af[TM], bf[TN];
-      const int sw = gemm_swz<VEC>(ks * 4 + kq);
+    for (int ks = 0; ks < BK / 8; ++ks) {
+      d2_t af[TM], bf[TN];
+      const int co = (ks * 4 + kq) ^ sw;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = As[cur][ks * 4 + kq][(am + i * 16) ^ sw];
+      for (int i = 0; i < TM; ++i) af[i] = As[cur][am + i * 16 * CH + co];
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = Bs[cur][ks * 4 + kq][(bn + j * 16) ^ sw];
+      for (int j = 0; j < TN; ++j) bf[j] = Bs[cur][bn + j * 16 * CH + co];
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i].x, bf[j].x, acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i].y, bf[j].y, acc[i][j], 0, 0, 0);
     }
-    if (kt + 1 < nk) store_tile(cur ^ 1);
+    if (kt + 1 < nk) store_tile(cur ^ 1, knext);
     __syncthreads();
   }
 
@@ -159,24 +158,26 @@ __device__ __forceinline__ void gemm_nt_f64_body(
     }
 }
 
-template <int BM, int BN, int WM, int WN, int VEC>
-__global__ __launch_bounds__(256) void gemm_nt_f64_kernel(
+// two waves per SIMD (two 128 x 128 workgroups per CU): without the bound the 128-wide
+// tile takes 336 registers
+template <int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256, 2) void gemm_nt_f64_kernel(
     int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
     const double* __restrict__ B, int ldb, double beta, double* __restrict__ C, int ldc,
     int tiles_m, int tiles_n, int k_per_split, int64_t c_split_stride) {
-  gemm_nt_f64_body<BM, BN, WM, WN, VEC>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles_m,
+  gemm_nt_f64_body<BM, BN, WM, WN>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles_m,
                                         tiles_n, k_per_split, c_split_stride, blockIdx.x,
                                         blockIdx.y);
 }
 
 // grouped: problem p owns tiles [start[p], start[p + 1]), no split-K, beta = 0
-template <int BM, int BN, int VEC>
-__global__ __launch_bounds__(256) void gemm_f64_grouped_kernel(const GemmArgs* __restrict__ args,
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_f64_grouped_kernel(const GemmArgs* __restrict__ args,
                                                                const int* __restrict__ start,
                                                                int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
   const GemmArgs a = args[p];
-  gemm_nt_f64_body<BM, BN, 2, 2, VEC>(a.M, a.N, a.K, (double)a.alpha,
+  gemm_nt_f64_body<BM, BN, 2, 2>(a.M, a.N, a.K, (double)a.alpha,
                                       static_cast<const double*>(a.A), (int)a.lda,
                                       static_cast<const double*>(a.B), (int)a.ldb, 0.0,
                                       static_cast<double*>(a.C), (int)a.ldc, a.tiles_m, a.tiles_n,
@@ -187,19 +188,26 @@ __global__ __launch_bounds__(256) void gemm_f64_grouped_kernel(const GemmArgs* _
 template <int BM, int BN>
 int launch_tiles(hipStream_t s, int M, int N, int K, double alpha, const double* A, int lda,
                  const double* B, int ldb, double beta, double* C, int ldc, int splits,
-                 int k_per_split, int64_t c_split_stride, bool vec2) {
+                 int k_per_split, int64_t c_split_stride) {
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-  dim3 grid(tm * tn, splits);
-  if (vec2)
-    hipLaunchKernelGGL((gemm_nt_f64_kernel<BM, BN, 2, 2, 2>), grid, dim3(256), 0, s, M, N, K,
-                       alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, k_per_split,
-                       c_split_stride);
-  else
-    hipLaunchKernelGGL((gemm_nt_f64_kernel<BM, BN, 2, 2, 1>), grid, dim3(256), 0, s, M, N, K,
-                       alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, k_per_split,
-                       c_split_stride);
+  hipLaunchKernelGGL((gemm_nt_f64_kernel<BM, BN, 2, 2>), dim3(tm * tn, splits), dim3(256), 0, s,
+                     M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tm, tn, k_per_split,
+                     c_split_stride);
   LAUNCH_CHECK();
   return AFQMC_OK;
+}
+
+// Tile edge: a 128-wide tile runs at 65 TFLOP/s against 61 of a 64-wide one (8192 x 4096 x
+// 4096), but in rounds of 256 tiles (one per CU) a partly filled last round weighs more.
+// 128 where it has two rounds and still does more per round (measured at 2048 x 10000 x
+// 400, 4.9 rounds: 280 against 317 us; 2048 x 5050 x 400, 2.5 rounds: 167 against 147).
+int gemm_f64_tile(int M, int N, int splits) {
+  const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * splits;
+  const int64_t t64 = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits;
+  if (t128 < 512) return 64;
+  const double e128 = (double)t128 / (double)((t128 + 255) / 256);
+  const double e64 = (double)t64 / (double)((t64 + 255) / 256);
+  return 65.0 * e128 > 61.0 * e64 ? 128 : 64;
 }
 
 }  // namespace
@@ -223,46 +231,30 @@ int launch_gemm_nt_f64_split(hipStream_t s, int M, int N, int K, double alpha, c
   if (splits < 1) splits = 1;
   int kps = (K + splits - 1) / splits;
   kps = (kps + GEMM_BK - 1) / GEMM_BK * GEMM_BK;
-  const bool vec2 = ((lda | ldb | K) % 2 == 0) && ((uintptr_t)A % 16 == 0) &&
-                    ((uintptr_t)B % 16 == 0);
-  const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big_tiles * splits >= 512)
+  if (gemm_f64_tile(M, N, splits) == 128)
     return launch_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits, kps,
-                                  c_split_stride, vec2);
+                                  c_split_stride);
   return launch_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits, kps,
-                              c_split_stride, vec2);
+                              c_split_stride);
 }
 
 int launch_gemm_nt_f64(hipStream_t s, int M, int N, int K, double alpha, const double* A,
                        int lda, const double* B, int ldb, double beta, double* C, int ldc) {
   if (M <= 0 || N <= 0) return AFQMC_OK;
   if (K <= 0) return afqmc_set_error(AFQMC_ERR_ARG, "gemm: K=%d", K);
-  const bool vec2 = ((lda | ldb | K) % 2 == 0) && ((uintptr_t)A % 16 == 0) &&
-                    ((uintptr_t)B % 16 == 0);
-  const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big_tiles >= 512)
-    return launch_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0,
-                                  vec2);
-  return launch_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0, vec2);
+  if (gemm_f64_tile(M, N, 1) == 128)
+    return launch_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
+  return launch_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
 }
 
-int launch_gemm_f64_grouped(hipStream_t s, int bm, bool vec2, const GemmArgs* args,
-                            const int* start, int nprob, int nblocks) {
-  if (bm == 128) {
-    if (vec2)
-      hipLaunchKernelGGL((gemm_f64_grouped_kernel<128, 128, 2>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-    else
-      hipLaunchKernelGGL((gemm_f64_grouped_kernel<128, 128, 1>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-  } else {
-    if (vec2)
-      hipLaunchKernelGGL((gemm_f64_grouped_kernel<64, 64, 2>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-    else
-      hipLaunchKernelGGL((gemm_f64_grouped_kernel<64, 64, 1>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-  }
+int launch_gemm_f64_grouped(hipStream_t s, int bm, const GemmArgs* args, const int* start,
+                            int nprob, int nblocks) {
+  if (bm == 128)
+    hipLaunchKernelGGL((gemm_f64_grouped_kernel<128, 128>), dim3(nblocks), dim3(256), 0, s, args,
+                       start, nprob);
+  else
+    hipLaunchKernelGGL((gemm_f64_grouped_kernel<64, 64>), dim3(nblocks), dim3(256), 0, s, args,
+                       start, nprob);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }

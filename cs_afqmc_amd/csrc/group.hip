@@ -48,7 +48,7 @@ struct afqmc_group {
   bool f32 = false;           // FP32 mode: the float64 operands on float32 MFMA
   int fb_bm = 0, vhs_bm = 0;  // GEMM tile edge (0: heuristic)
   int cg_bm = 0;              // tile edge of the energy's float64 c_g product (0: heuristic)
-  bool f64_vec2 = true;
+  bool f32_vec2 = true;       // every FP32-mode product has an even K
   // built tables
   std::vector<Launch> meas, taylor;
   Launch fb{}, vhs{}, fields{}, weights{};
@@ -68,7 +68,6 @@ struct afqmc_group {
   // step's; en_ptrs are the energies outputs the finishing table was built for
   Launch qr{}, ovc{}, fb64{}, fin{};
   std::vector<Launch> meas_ov, meas_en, exch;
-  bool fb64_vec2 = true;
   std::vector<void*> en_ptrs;
   // block fields draws (afqmc_group_fields_normal_key), keys the table was built for
   Launch draw{};
@@ -95,7 +94,7 @@ int heuristic_bm(int64_t tiles128) { return tiles128 >= 512 ? 128 : 64; }
 
 int build(afqmc_group* g) {
   g->host_tab.clear();
-  g->f64_vec2 = true;
+  g->f32_vec2 = true;
   g->meas.clear();
   g->taylor.clear();
   std::vector<unsigned char>& tab = g->host_tab;
@@ -176,7 +175,7 @@ int build(afqmc_group* g) {
           a.K = c->kdim[s];
           a.A = c->green[s];
           a.B = c->rot_chol[s];
-          if (a.K % 2) g->f64_vec2 = false;
+          if (a.K % 2) g->f32_vec2 = false;
         }
         a.lda = a.ldb = a.K;
         a.tiles_m = (a.M + bm - 1) / bm;
@@ -255,7 +254,7 @@ int build(afqmc_group* g) {
           a.A = c->xs;
           a.B = chol_t_of(c, cs);
           a.C = vhs_of(c, cs);
-          if (a.K % 2) g->f64_vec2 = false;
+          if (a.K % 2) g->f32_vec2 = false;
         }
         a.lda = a.ldb = a.K;
         a.tiles_m = (a.M + bm - 1) / bm;
@@ -466,7 +465,6 @@ int build(afqmc_group* g) {
       for (int s = 0; s < m.c->nspin; ++s)
         t128 += (int64_t)((2 * m.c->d.n_walkers + 127) / 128) * ((m.c->d.nchol + 127) / 128);
     const int bm = g->cg_bm ? g->cg_bm : heuristic_bm(t128);
-    g->fb64_vec2 = true;
     int b = 0;
     for (const Member& m : g->mem) {
       afqmc_ctx* c = m.c;
@@ -482,7 +480,6 @@ int build(afqmc_group* g) {
         a.C = c->fb + (int64_t)s * 2 * W * G;
         a.lda = a.ldb = a.K;
         a.ldc = G;
-        if (a.K % 2) g->fb64_vec2 = false;
         a.tiles_m = (a.M + bm - 1) / bm;
         a.tiles_n = (a.N + bm - 1) / bm;
         args.push_back(a);
@@ -650,9 +647,9 @@ int run_gemm(afqmc_group* g, const Launch& L, int out_f32) {
     return launch_gemm_bf16x3_grouped(g->stream, L.k0, out_f32, targs<GemmArgs>(g, L),
                                       tstart(g, L), L.nprob, L.nblocks);
   if (g->f32)
-    return launch_gemm_f32_grouped(g->stream, L.k0, g->f64_vec2, targs<GemmArgs>(g, L),
+    return launch_gemm_f32_grouped(g->stream, L.k0, g->f32_vec2, targs<GemmArgs>(g, L),
                                    tstart(g, L), L.nprob, L.nblocks);
-  return launch_gemm_f64_grouped(g->stream, L.k0, g->f64_vec2, targs<GemmArgs>(g, L),
+  return launch_gemm_f64_grouped(g->stream, L.k0, targs<GemmArgs>(g, L),
                                  tstart(g, L), L.nprob, L.nblocks);
 }
 
@@ -867,7 +864,7 @@ extern "C" int afqmc_group_energy(afqmc_group* g, void* const* energies) {
   if (rc) return rc;
   PhaseTimer t(&g->prof, g->stream, AFQMC_PH_ENERGY);
   // c_g = force bias, contracted in float64 as the single context's energy does
-  if ((rc = launch_gemm_f64_grouped(g->stream, g->fb64.k0, g->fb64_vec2,
+  if ((rc = launch_gemm_f64_grouped(g->stream, g->fb64.k0,
                                     targs<GemmArgs>(g, g->fb64), tstart(g, g->fb64),
                                     g->fb64.nprob, g->fb64.nblocks)))
     return rc;
@@ -934,7 +931,7 @@ extern "C" int afqmc_group_tune(afqmc_group* g, double* ms_out) {
   float best[3][2];  // [fb / vhs / c_g][64 / 128]
   auto run = [&](int which) {
     if (which == 2)
-      return launch_gemm_f64_grouped(g->stream, g->fb64.k0, g->fb64_vec2,
+      return launch_gemm_f64_grouped(g->stream, g->fb64.k0,
                                      targs<GemmArgs>(g, g->fb64), tstart(g, g->fb64),
                                      g->fb64.nprob, g->fb64.nblocks);
     return run_gemm(g, which ? g->vhs : g->fb, which);
