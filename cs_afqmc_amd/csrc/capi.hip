@@ -24,8 +24,9 @@ extern "C" const char* afqmc_last_error(void) { return g_err; }
 namespace {
 
 // Every allocation ends with DEV_PAD unused bytes: the 16-byte operand loads of the
-// float64 GEMM and exchange may start on the last element of a row of odd length.
-constexpr size_t DEV_PAD = 16;
+// float64 GEMM may start on the last element of a row of odd length, and the Taylor
+// kernel reads the last row of exp_h1 to its tile's end (15 elements).
+constexpr size_t DEV_PAD = 256;
 template <typename T>
 int dalloc(afqmc_ctx* c, T** p, size_t count) {
   *p = nullptr;

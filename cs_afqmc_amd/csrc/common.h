@@ -151,6 +151,12 @@ __device__ inline void xcd_tile(int bx, int tiles_m, int tiles_n, bool m_major, 
   }
 }
 
+// Barrier over the workgroup's LDS traffic only: waits for this wave's LDS operations, not
+// for its global loads in flight (operands loaded ahead stay outstanding across it)
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ---------------------------------------------------------------- reductions
 template <int NT>
 __device__ inline double block_sum(double v, double* red) {

@@ -59,13 +59,6 @@ struct GjState {
 };
 static_assert(sizeof(GjState) <= 256 * sizeof(int), "GjState exceeds its LDS slot");
 
-// Barrier over the workgroup's LDS traffic only: waits for this wave's LDS operations,
-// not for its global loads in flight (the Green product's first operands are loaded
-// before the inversion and stay outstanding across it)
-__device__ inline void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // 1 / x for x > 0 of moderate range: hardware estimate plus two Newton steps
 __device__ inline double rcp_f64(double x) {
   double y = __builtin_amdgcn_rcp(x);

@@ -152,73 +152,103 @@ __global__ __launch_bounds__(1024) void taylor_grouped_kernel(const TaylorArgs* 
 }
 
 // ------------------------------------------------------------------------------------
-// Register-resident form (N <= 128, n <= 32).  One workgroup per (walker, spin); wave r
-// keeps rows [16 r, 16 r + 16) of A = [Vr | Vi] (N x 2Np, Np = N rounded up to 4) in
-// registers for the whole series, so V is read from HBM once.  The complex product is
-// one real product  [ur | ui] = [Vr | Vi] [[tr, ti], [-ti, tr]]  whose B operand lives
-// in LDS as 2Np rows: rows [0, Np) = [tr | ti], rows [Np, 2Np) = [-ti | tr] (columns
-// padded to CTP*16), so k-group kg reads rows 4 kg .. 4 kg + 3 of one uniform array.
-// The series is evaluated in Horner form  y <- t0 + V y / k  (k = K..1), which equals
-// t0 + sum_k V^k t0 / k! of propagation.py:67-92.
+// Register-resident form (N <= 128, n <= 32).  One workgroup per (walker, spin) of NW =
+// ceil(N / 16) waves; wave r keeps rows [16 r, 16 r + 16) of A = [Vr | Vi] (N x 2Np, Np =
+// N rounded up to 4) in registers for the whole series, so V is read from HBM once.  The
+// complex product is one real product  [ur | ui] = [Vr | Vi] [[tr, ti], [-ti, tr]]  whose
+// B operand lives in LDS as 2Np rows: rows [0, Np) = [tr | ti], rows [Np, 2Np) =
+// [-ti | tr] (columns padded to CTP*16), so k-group kg reads rows 4 kg .. 4 kg + 3 of one
+// uniform array.  The series is evaluated in Horner form  y <- t0 + V y / k  (k = K..1),
+// which equals t0 + sum_k V^k t0 / k! of propagation.py:67-92.
+//
+// Bound by float64 MFMA once a walker's loads are out of the way, and a CU holds one or
+// two walkers only (V fills the registers), so nothing may wait in turn:
+//   - every load is unconditional, from a clamped index, and masked after; as masked loads
+//     the 2Np / 4 loads of a V row each waited for HBM on their own;
+//   - the walker and the rows of E are loaded first and V last, so V arrives while the
+//     first product E w runs (the barriers wait for LDS only);
+//   - the rows of E are whole in registers before their product, instead of one L2 round
+//     trip per k group;
+//   - y / k is a multiplication by 1 / k with one correction step, not a division.
 template <int CTP>
 struct RegTile {
   static constexpr int RS = 16 * CTP + ((CTP % 2 == 0) ? 16 : 0);  // == 16 (mod 32) doubles
 };
 
-template <int NKGV, int CTP>
+// x / k for a small integer k, rk = 1 / k: the quotient corrected by its residual
+__device__ inline double div_small(double x, double k, double rk) {
+  const double q = x * rk;
+  return fma(fma(-q, k, x), rk, q);
+}
+
+template <int NW, int CTP>
 __device__ __forceinline__ void taylor_reg_body(int N, int n, int n_terms_k,
                                                 cplx* __restrict__ walkers,
                                                 const double* __restrict__ expE,
-                                                const double* __restrict__ vhs, const int w) {
+                                                const double* __restrict__ vhs, int nv,
+                                                const int w) {
+  constexpr int NKG = 4 * NW;  // k-groups of one half (of E, Vr or Vi) for N = 16 NW
   constexpr int RS = RegTile<CTP>::RS;
+  constexpr int NT = 64 * NW;
   extern __shared__ double TT[];  // [2 Np][RS]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rb = wave * 16;
   const int Np = (N + 3) & ~3;
-  const int nkg = Np >> 2;         // k-groups of one half (E products)
-  const int nkgv = 2 * nkg;        // k-groups of [Vr | Vi]
+  const int nkg = Np >> 2;         // k-groups in use: NKG - 3 <= nkg <= NKG
   const int s = lane >> 4, col = lane & 15;
   const int p = rb + col;          // A-operand row of this lane
-  const bool prow = p < N;
+  const int pc = min(p, N - 1);    // (rows p >= N are never stored)
   const int n2 = 2 * n;
   cplx* phi = walkers + (int64_t)w * N * n;
-  const double* Vr = vhs + (int64_t)w * 2 * N * N;
-  const double* Vi = Vr + (int64_t)N * N;
+  const double* Vr = vhs + (int64_t)w * 2 * nv;
+  const double* Vi = Vr + nv;
+  // V planes hold all N^2 entries row-major, or (nv = N(N+1)/2, symmetric V) the upper
+  // triangle row by row: entry (a, b), a <= b, at a N - a (a - 1) / 2 + b - a
+  const bool packed = nv != N * N;
 
-  // A = [Vr | Vi] rows in registers: k-group kg, slot s -> column q = 4 kg + s
-  double va[NKGV];
+  // walker tile: [tr | ti] and [-ti | tr]; rows q >= N zero (whatever A holds there)
+  for (int e = threadIdx.x; e < N * n; e += NT) {
+    const int q = e / n, j = e - q * n;
+    const cplx z = phi[e];
+    double* up = TT + q * RS + j;
+    double* lo = up + Np * RS;
+    up[0] = z.re;
+    up[n] = z.im;
+    lo[0] = -z.im;
+    lo[n] = z.re;
+  }
+  for (int e = threadIdx.x; e < (Np - N) * RS; e += NT)
+    TT[N * RS + e] = TT[(Np + N) * RS + e] = 0.0;
+
+  // rows of E, k-group kg: E[p][4 kg + s]; what is read past the row's end (the next row,
+  // or the padding after the matrix) is zeroed before the product
+  double ea[NKG];
+  auto load_e = [&](const double* erow) {
 #pragma unroll
-  for (int kg = 0; kg < NKGV; ++kg) {
-    const int q = 4 * kg + s;
-    double v = 0.0;
-    if (kg < nkgv && prow) {
-      if (q < Np) {
-        if (q < N) v = Vr[(int64_t)p * N + q];
-      } else if (q - Np < N) {
-        v = Vi[(int64_t)p * N + q - Np];
-      }
-    }
-    va[kg] = v;
+    for (int kg = 0; kg < NKG; ++kg) ea[kg] = erow[4 * kg];
+  };
+  load_e(expE + (pc * N + s));
+  __builtin_amdgcn_sched_barrier(0);
+  // rows of V in registers: k-group kg, slot s -> column q = 4 kg + s, of which real and
+  // imaginary part share the index.  The scheduling barriers keep the indices of a few
+  // loads in registers, not of all.
+  double vr[NKG], vi[NKG];
+#pragma unroll
+  for (int kg = 0; kg < NKG; ++kg) {
+    const int qc = min(4 * kg + s, N - 1);
+    const int a = min(pc, qc), b = max(pc, qc);
+    const int idx = packed ? a * N - (a * (a - 1)) / 2 + (b - a) : pc * N + qc;
+    vr[kg] = Vr[idx];
+    vi[kg] = Vi[idx];
+    if (kg % 2 == 1) __builtin_amdgcn_sched_barrier(0);
   }
-
-  // walker tile: [tr | ti] and [-ti | tr], zero padded
-  for (int e = threadIdx.x; e < Np * RS; e += blockDim.x) {
-    const int q = e / RS, c = e - (e / RS) * RS;
-    double up = 0.0, lo = 0.0;
-    if (q < N && c < n2) {
-      const int j = c < n ? c : c - n;
-      const cplx z = phi[(int64_t)q * n + j];
-      up = c < n ? z.re : z.im;
-      lo = c < n ? -z.im : z.re;
-    }
-    TT[e] = up;
-    TT[Np * RS + e] = lo;
-  }
-  __syncthreads();
+  __builtin_amdgcn_sched_barrier(0);
+  lds_barrier();
 
   const double* bbase = TT + s * RS + col;  // + kg * 4 RS + ct * 16
+  const double* blo = bbase + Np * RS;
 
-  // y rows -> both halves (rows >= Np never written: they belong to the lower half)
+  // y rows -> both halves (rows q >= N keep their zeros)
   auto put = [&](const double4_t* v) {
 #pragma unroll
     for (int ct = 0; ct < CTP; ++ct)
@@ -226,7 +256,7 @@ __device__ __forceinline__ void taylor_reg_body(int N, int n, int n_terms_k,
       for (int r = 0; r < 4; ++r) {
         const int row = rb + s + 4 * r;
         const int cc = ct * 16 + col;
-        if (row < Np) {
+        if (row < N) {
           TT[row * RS + cc] = v[ct][r];
           if (cc < n)
             TT[(Np + row) * RS + cc + n] = v[ct][r];
@@ -235,58 +265,62 @@ __device__ __forceinline__ void taylor_reg_body(int N, int n, int n_terms_k,
         }
       }
   };
-
-  auto e_product = [&](double4_t* acc) {
-#pragma unroll
-    for (int ct = 0; ct < CTP; ++ct) acc[ct] = double4_t{0.0, 0.0, 0.0, 0.0};
-    double a = (prow && s < N) ? expE[(int64_t)p * N + s] : 0.0;
-    for (int kg = 0; kg < nkg; ++kg) {
-      const int qn = 4 * (kg + 1) + s;
-      const double an = (kg + 1 < nkg && prow && qn < N) ? expE[(int64_t)p * N + qn] : 0.0;
-#pragma unroll
-      for (int ct = 0; ct < CTP; ++ct)
-        acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bbase[kg * 4 * RS + ct * 16], acc[ct],
-                                                       0, 0, 0);
-      a = an;
-    }
-  };
-
-  double4_t t0[CTP], u[CTP];
-  e_product(t0);
-  __syncthreads();
-  put(t0);
-  __syncthreads();
-  for (int k = n_terms_k; k >= 1; --k) {
-#pragma unroll
-    for (int ct = 0; ct < CTP; ++ct) u[ct] = double4_t{0.0, 0.0, 0.0, 0.0};
+  // acc += A y over the rows a[] of A and one half of y; B of k-group kg + 1 is read from
+  // LDS under the MFMAs of kg
+  auto product = [&](const double (&a)[NKG], const double* bb, double4_t* acc) {
     double b[CTP];
 #pragma unroll
-    for (int ct = 0; ct < CTP; ++ct) b[ct] = bbase[ct * 16];
+    for (int ct = 0; ct < CTP; ++ct) b[ct] = bb[ct * 16];
 #pragma unroll
-    for (int kg = 0; kg < NKGV; ++kg) {
-      if (kg < nkgv) {
-        // software pipeline: B of k-group kg + 1 is read from LDS under the MFMAs of kg
+    for (int kg = 0; kg < NKG; ++kg) {
+      if (kg < NKG - 3 || kg < nkg) {
         double bn[CTP];
 #pragma unroll
         for (int ct = 0; ct < CTP; ++ct)
-          bn[ct] = (kg + 1 < nkgv) ? bbase[(kg + 1) * 4 * RS + ct * 16] : 0.0;
+          bn[ct] = bb[(kg + 1 < NKG - 3 ? kg + 1 : min(kg + 1, nkg - 1)) * 4 * RS + ct * 16];
 #pragma unroll
         for (int ct = 0; ct < CTP; ++ct)
-          u[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[kg], b[ct], u[ct], 0, 0, 0);
+          acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kg], b[ct], acc[ct], 0, 0, 0);
 #pragma unroll
         for (int ct = 0; ct < CTP; ++ct) b[ct] = bn[ct];
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
-    const double rk = (double)k;
+  };
+  auto zero = [&](double4_t* acc) {
+#pragma unroll
+    for (int ct = 0; ct < CTP; ++ct) acc[ct] = double4_t{0.0, 0.0, 0.0, 0.0};
+  };
+
+  auto e_product = [&](double4_t* acc) {
+#pragma unroll
+    for (int kg = NKG - 4; kg < NKG; ++kg) ea[kg] = 4 * kg + s < N ? ea[kg] : 0.0;
+    zero(acc);
+    product(ea, bbase, acc);
+  };
+
+  double4_t t0[CTP], u[CTP];
+  e_product(t0);
+  lds_barrier();
+  put(t0);
+  lds_barrier();
+#pragma unroll 1
+  for (int k = n_terms_k; k >= 1; --k) {
+    zero(u);
+    product(vr, bbase, u);
+    product(vi, blo, u);
+    lds_barrier();
+    const double dk = (double)k, rk = 1.0 / dk;
 #pragma unroll
     for (int ct = 0; ct < CTP; ++ct)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[ct][r] = t0[ct][r] + u[ct][r] / rk;
+      for (int r = 0; r < 4; ++r) u[ct][r] = t0[ct][r] + div_small(u[ct][r], dk, rk);
     put(u);
-    __syncthreads();
+    lds_barrier();
   }
+  int eoff = pc * N + s;
+  asm volatile("" : "+v"(eoff));  // (addressed anew: nothing of E stays in registers meanwhile)
+  load_e(expE + eoff);
   e_product(u);
 #pragma unroll
   for (int ct = 0; ct < CTP; ++ct)
@@ -301,33 +335,40 @@ __device__ __forceinline__ void taylor_reg_body(int N, int n, int n_terms_k,
     }
 }
 
-template <int NKGV, int CTP>
-__global__ __launch_bounds__(512) void taylor_reg_kernel(
-    int N, int n, int n_terms_k, cplx* __restrict__ walkers, const double* __restrict__ expE,
-    const double* __restrict__ vhs) {
-  taylor_reg_body<NKGV, CTP>(N, n, n_terms_k, walkers, expE, vhs, blockIdx.x);
+// waves of a register-form workgroup (a template key) and its column tiles
+inline int reg_waves(int N) { return (N + 15) / 16; }
+inline int reg_ct(int n) { return (2 * n + 15) / 16; }
+inline size_t reg_shm(int N, int ct) {
+  return (size_t)2 * ((N + 3) & ~3) * (16 * ct + ((ct % 2 == 0) ? 16 : 0)) * sizeof(double);
 }
 
-template <int NKGV, int CTP>
-__global__ __launch_bounds__(512) void taylor_reg_grouped_kernel(
+template <int NW, int CTP>
+__global__ __launch_bounds__(64 * NW) void taylor_reg_kernel(
+    int N, int n, int n_terms_k, cplx* __restrict__ walkers, const double* __restrict__ expE,
+    const double* __restrict__ vhs, int nv) {
+  taylor_reg_body<NW, CTP>(N, n, n_terms_k, walkers, expE, vhs, nv, blockIdx.x);
+}
+
+template <int NW, int CTP>
+__global__ __launch_bounds__(64 * NW) void taylor_reg_grouped_kernel(
     const TaylorArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
   const TaylorArgs a = args[p];
-  taylor_reg_body<NKGV, CTP>(a.N, a.n, a.K, a.walkers, static_cast<const double*>(a.E),
-                             static_cast<const double*>(a.vhs), blockIdx.x - start[p]);
+  taylor_reg_body<NW, CTP>(a.N, a.n, a.K, a.walkers, static_cast<const double*>(a.E),
+                           static_cast<const double*>(a.vhs), a.nv, blockIdx.x - start[p]);
 }
 
-template <int NKGV, int CTP>
+template <int NW, int CTP>
 int launch_reg(afqmc_ctx* c, int W, int n, cplx* wk, const double* E, const double* V) {
   const int N = c->d.norb;
-  const int nwaves = (N + 15) / 16;
-  const int Np = (N + 3) & ~3;
-  const size_t shm = (size_t)2 * Np * RegTile<CTP>::RS * sizeof(double);
+  if (reg_waves(N) != NW || reg_ct(n) != CTP)
+    return afqmc_set_error(AFQMC_ERR_ARG, "taylor f64: %d waves do not fit N %d", NW, N);
+  const size_t shm = reg_shm(N, CTP);
   static int lds_limit = 0;
-  const int rc = ensure_dyn_lds((const void*)taylor_reg_kernel<NKGV, CTP>, shm, &lds_limit);
+  const int rc = ensure_dyn_lds((const void*)taylor_reg_kernel<NW, CTP>, shm, &lds_limit);
   if (rc) return rc;
-  hipLaunchKernelGGL((taylor_reg_kernel<NKGV, CTP>), dim3(W), dim3(nwaves * 64), shm, c->stream,
-                     N, n, c->d.n_exp_terms - 1, wk, E, V);
+  hipLaunchKernelGGL((taylor_reg_kernel<NW, CTP>), dim3(W), dim3(NW * 64), shm, c->stream, N, n,
+                     c->d.n_exp_terms - 1, wk, E, V, N * N);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }
@@ -986,14 +1027,13 @@ int launch_bfs(afqmc_ctx* c, int W, int n, cplx* wk, int s) {
   return AFQMC_OK;
 }
 
-template <int NKGV>
+template <int NW>
 int launch_reg_ct(afqmc_ctx* c, int W, int n, cplx* wk, const double* E, const double* V) {
-  const int ctp = (2 * n + 15) / 16;
-  switch (ctp) {
-    case 1: return launch_reg<NKGV, 1>(c, W, n, wk, E, V);
-    case 2: return launch_reg<NKGV, 2>(c, W, n, wk, E, V);
-    case 3: return launch_reg<NKGV, 3>(c, W, n, wk, E, V);
-    default: return launch_reg<NKGV, 4>(c, W, n, wk, E, V);
+  switch (reg_ct(n)) {
+    case 1: return launch_reg<NW, 1>(c, W, n, wk, E, V);
+    case 2: return launch_reg<NW, 2>(c, W, n, wk, E, V);
+    case 3: return launch_reg<NW, 3>(c, W, n, wk, E, V);
+    default: return launch_reg<NW, 4>(c, W, n, wk, E, V);
   }
 }
 
@@ -1002,9 +1042,6 @@ int launch_reg_ct(afqmc_ctx* c, int W, int n, cplx* wk, const double* E, const d
 // The kernel launch_taylor picks for spin s, as a plan for grouped launches.
 void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl) {
   const int N = c->d.norb, n = c->nocc[s];
-  const int Np = (N + 3) & ~3;
-  const int nkgv = 2 * ((N + 3) / 4);
-  const int bucket = nkgv <= 32 ? 32 : nkgv <= 48 ? 48 : nkgv <= 56 ? 56 : 64;
   const int ctp = (2 * n + 15) / 16 > 4 ? 4 : (2 * n + 15) / 16;
   pl->nthreads = ((N + 15) / 16) * 64;
   pl->blocks_per_walker = 1;
@@ -1026,10 +1063,9 @@ void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl) {
     }
   } else if (N <= 128 && c->nocc[0] <= 32 && c->nocc[1] <= 32) {
     pl->kind = TAYLOR_REG_F64;
-    pl->nkgv = bucket;
+    pl->nkgv = reg_waves(N);
     pl->ct = ctp;
-    const int rs = 16 * ctp + ((ctp % 2 == 0) ? 16 : 0);
-    pl->shm = (size_t)2 * Np * rs * sizeof(double);
+    pl->shm = reg_shm(N, ctp);
   } else {
     pl->kind = TAYLOR_STREAM_F64;
     pl->blocks_per_walker = (n + 15) / 16;
@@ -1082,13 +1118,18 @@ int launch_taylor(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
     for (int s = 0; s < c->nspin; ++s) {
       const int n = c->nocc[s];
       cplx* wk = (s == 0) ? wup : wdn;
-      // register budget: 2 ceil(N/4) k-groups of [Vr | Vi] per lane, bucketed
-      const int nkgv = 2 * ((N + 3) / 4);
-      const double* V = vhs_of(c, s);
-      const int rc = nkgv <= 32   ? launch_reg_ct<32>(c, W, n, wk, c->exp_h1[s], V)
-                     : nkgv <= 48 ? launch_reg_ct<48>(c, W, n, wk, c->exp_h1[s], V)
-                     : nkgv <= 56 ? launch_reg_ct<56>(c, W, n, wk, c->exp_h1[s], V)
-                                  : launch_reg_ct<64>(c, W, n, wk, c->exp_h1[s], V);
+      const double *E = c->exp_h1[s], *V = vhs_of(c, s);
+      int rc;
+      switch (reg_waves(N)) {
+        case 1: rc = launch_reg_ct<1>(c, W, n, wk, E, V); break;
+        case 2: rc = launch_reg_ct<2>(c, W, n, wk, E, V); break;
+        case 3: rc = launch_reg_ct<3>(c, W, n, wk, E, V); break;
+        case 4: rc = launch_reg_ct<4>(c, W, n, wk, E, V); break;
+        case 5: rc = launch_reg_ct<5>(c, W, n, wk, E, V); break;
+        case 6: rc = launch_reg_ct<6>(c, W, n, wk, E, V); break;
+        case 7: rc = launch_reg_ct<7>(c, W, n, wk, E, V); break;
+        default: rc = launch_reg_ct<8>(c, W, n, wk, E, V); break;
+      }
       if (rc) return rc;
     }
     return AFQMC_OK;
@@ -1122,16 +1163,16 @@ int launch_grouped_fn(KernelFn fn, hipStream_t st, const TaylorArgs* args, const
   return AFQMC_OK;
 }
 
-template <int NKGV>
+template <int NW>
 int reg_grouped(int ct, hipStream_t st, const TaylorArgs* args, const int* start, int nprob,
                 int nblocks, int nthreads, size_t shm) {
   static int lim[4] = {};
   const int ci = ct < 1 ? 0 : (ct > 4 ? 3 : ct - 1);
   switch (ct) {
-    case 1: return launch_grouped_fn(taylor_reg_grouped_kernel<NKGV, 1>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
-    case 2: return launch_grouped_fn(taylor_reg_grouped_kernel<NKGV, 2>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
-    case 3: return launch_grouped_fn(taylor_reg_grouped_kernel<NKGV, 3>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
-    case 4: return launch_grouped_fn(taylor_reg_grouped_kernel<NKGV, 4>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
+    case 1: return launch_grouped_fn(taylor_reg_grouped_kernel<NW, 1>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
+    case 2: return launch_grouped_fn(taylor_reg_grouped_kernel<NW, 2>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
+    case 3: return launch_grouped_fn(taylor_reg_grouped_kernel<NW, 3>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
+    case 4: return launch_grouped_fn(taylor_reg_grouped_kernel<NW, 4>, st, args, start, nprob, nblocks, nthreads, shm, &lim[ci]);
   }
   return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: column tiles %d", ct);
 }
@@ -1144,11 +1185,15 @@ int launch_taylor_grouped(hipStream_t st, int kind, int nkgv, int ct, const Tayl
                           const int* start, int nprob, int nblocks, int nthreads, size_t shm) {
   if (kind == TAYLOR_REG_F64) {
     switch (nkgv) {
-      case 32: return reg_grouped<32>(ct, st, args, start, nprob, nblocks, nthreads, shm);
-      case 48: return reg_grouped<48>(ct, st, args, start, nprob, nblocks, nthreads, shm);
-      case 56: return reg_grouped<56>(ct, st, args, start, nprob, nblocks, nthreads, shm);
-      case 64: return reg_grouped<64>(ct, st, args, start, nprob, nblocks, nthreads, shm);
-      default: return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: nkgv %d", nkgv);
+      case 1: return reg_grouped<1>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 2: return reg_grouped<2>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 3: return reg_grouped<3>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 4: return reg_grouped<4>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 5: return reg_grouped<5>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 6: return reg_grouped<6>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 7: return reg_grouped<7>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      case 8: return reg_grouped<8>(ct, st, args, start, nprob, nblocks, nthreads, shm);
+      default: return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: %d waves", nkgv);
     }
   }
   if (kind == TAYLOR_REG_BF16X3) {
