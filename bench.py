@@ -94,7 +94,7 @@ def phase_kernel(precision, phase, norb, nelec):
     reg = norb <= 128 and max(nelec) <= 32
     if phase == "taylor":
         if precision in ("fp64", "fp32"):
-            return "taylor_reg_kernel" if reg else "taylor_kernel"
+            return "taylor_reg_kernel" if reg else "taylor_stream_kernel"
         return "taylor_bf_kernel" if reg else "taylor_bfs_kernel"
     if phase in ("vhs_gemm", "fb_gemm"):
         return {"fp64": "gemm_nt_f64_kernel", "fp32": "gemm_nt_f32_kernel"}.get(

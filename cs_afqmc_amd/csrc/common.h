@@ -423,7 +423,7 @@ struct FieldsArgs {
   cplx* terms;
 };
 struct TaylorArgs {
-  int N, n, K, rows_pad;
+  int N, n, K, W;
   int nv;           // stored entries of one V plane (N*N, or N(N+1)/2 packed)
   cplx* walkers;
   const void* E;    // float64 / float32 exp_h1, or the hi plane of exp_h1 - I (bf16 kernel)
@@ -512,7 +512,8 @@ enum TaylorKind {
 };
 
 struct TaylorPlan {
-  int kind, nkgv, ct, nthreads, blocks_per_walker;
+  int kind, nkgv, ct, nthreads;
+  int nblocks;  // over the context's walker capacity
   size_t shm;
 };
 void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl);

@@ -230,16 +230,16 @@ int build(afqmc_group* g) {
     int64_t t128 = 0;
     for (const Member& m : g->mem)
       t128 += (int64_t)m.c->chol_spins * ((2 * m.c->d.n_walkers + 127) / 128) *
-              (((int64_t)m.c->d.norb * m.c->d.norb + 127) / 128);
+              (((int64_t)m.c->vhs_nv + 127) / 128);
     const int bm = g->vhs_bm ? g->vhs_bm : heuristic_bm(t128);
     int b = 0;
     for (const Member& m : g->mem) {
       afqmc_ctx* c = m.c;
-      const int W = c->d.n_walkers, N = c->d.norb;
+      const int W = c->d.n_walkers;
       for (int cs = 0; cs < c->chol_spins; ++cs) {
         GemmArgs a{};
         a.M = 2 * W;
-        a.N = g->mixed ? c->vhs_nv : N * N;
+        a.N = c->vhs_nv;
         a.alpha = 1.0f;
         a.ldc = a.N;
         if (g->mixed) {
@@ -284,8 +284,8 @@ int build(afqmc_group* g) {
         a.N = c->d.norb;
         a.n = c->nocc[s];
         a.K = c->d.n_exp_terms - 1;
-        a.rows_pad = ((a.N + 15) / 16) * 16;
-        a.nv = g->mixed ? c->vhs_nv : a.N * a.N;
+        a.W = c->d.n_walkers;
+        a.nv = c->vhs_nv;
         a.walkers = s == 0 ? m.wup : m.wdn;
         a.E = c->exp_h1[s];
         if (pl.kind == TAYLOR_REG_BF16X3 || pl.kind == TAYLOR_STREAM_BF16X3) {
@@ -294,7 +294,7 @@ int build(afqmc_group* g) {
         }
         a.vhs = g->mixed ? (const void*)vhs_f32_of(c, s) : (const void*)vhs_of(c, s);
         const auto key = std::make_tuple(pl.kind, pl.nkgv, pl.ct, pl.nthreads);
-        by_key[key].push_back({a, c->d.n_walkers * pl.blocks_per_walker});
+        by_key[key].push_back({a, pl.nblocks});
         shm[key] = std::max(shm[key], pl.shm);
       }
     }

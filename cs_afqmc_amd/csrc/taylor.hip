@@ -1,154 +1,305 @@
 // Trotterised propagator on walker tiles:  w <- E (t0 + sum_{k=1}^{K} V^k t0 / k!),
 // t0 = E w, with E = exp_h1 (real N x N) and V = VHS (complex N x N, per walker).
 // Follows propagator._apply_trotprop_det (propagation.py:67-92): carry_k = V carry_{k-1}
-// unscaled, each term divided by k!, summed, then added to t0.
-//
-// One workgroup per (walker, spin, 16-column chunk of the walker).  ceil(N/16) waves;
-// wave r owns output rows [16 r, 16 r + 16).  The 16-column chunk of the current
-// vector t lives in LDS (re / im planes, double buffered); V and E rows stream from
-// global memory as the A operand of v_mfma_f64_16x16x4f64.  Columns of a walker are
-// independent under left multiplication, so chunks never communicate.
+// unscaled, each term divided by k!, summed, then added to t0 (here in Horner form).
+// Columns of a walker are independent under left multiplication.
 #include "common.h"
 
 namespace {
 
-// LDS: T[buf][plane][q][j], q < rows_pad, j < 16
-__device__ inline double* tptr(double* T, int rows_pad, int buf, int plane) {
-  return T + (int64_t)((buf * 2 + plane) * rows_pad) * 16;
+// x / k for a small integer k, rk = 1 / k: the quotient corrected by its residual
+__device__ inline double div_small(double x, double k, double rk) {
+  const double q = x * rk;
+  return fma(fma(-q, k, x), rk, q);
 }
 
-// acc{R,I} (+)= A x T for a real A (E):  A rows [rb, rb+16), all N columns
-__device__ inline void mm_real(const double* __restrict__ A, int N, int rb, const double* tr,
-                               const double* ti, int lane, double4_t& accR, double4_t& accI) {
-  const int p = rb + (lane & 15);
-  const int s = lane >> 4;
-  const bool prow = p < N;
-  const int nkg = (N + 3) >> 2;
-  for (int kg = 0; kg < nkg; ++kg) {
-    const int q = 4 * kg + s;
-    const double a = (prow && q < N) ? A[(int64_t)p * N + q] : 0.0;
-    const double br = tr[q * 16 + (lane & 15)];
-    const double bi = ti[q * 16 + (lane & 15)];
-    accR = __builtin_amdgcn_mfma_f64_16x16x4f64(a, br, accR, 0, 0, 0);
-    accI = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bi, accI, 0, 0, 0);
-  }
-}
+// ------------------------------------------------------------------------------------
+// Streaming float64 form (N > 128 or n > 32).  One workgroup per walker of one spin and
+// chunk of 16 of its columns; wave r owns output rows [16 r, 16 r + 16).  y = [yr | yi]
+// lives in LDS, rows q of 32 doubles.  The rows of V stream from memory (L2 or HBM) once
+// per Horner term as the A operand of v_mfma_f64_16x16x4f64: four real products per k
+// group,
+//   ur = Vr yr - Vi yi,  ui = Vr yi + Vi yr.
+//
+// What it is shaped by (measured at norb 131, 29 + 26 columns, 777 walkers, both spins:
+// 1.89 ms with masked loads of one entry per k group):
+//   - a block of 16 k is four MFMAs, number 2 h + e taking k = 16 g + 8 h + 2 s + e in the
+//     lanes s = l / 16, so a lane reads two consecutive entries of its row at a time
+//     instead of one entry of each of four k groups;
+//   - the registers of a pair are refilled with the next block's entries as soon as its
+//     MFMAs are issued: loads stay in flight under the other pair's MFMAs and the other
+//     waves', without a second set of registers.  Registers decide here: two workgroups
+//     have to share a CU to cover each other's barriers, and the dispatcher counts
+//     ceil(waves / 4) waves on every SIMD for each;
+//   - no copies or avoidable index arithmetic in the loop: VALU instructions take issue
+//     slots from float64 MFMA.
+// With V kept as its upper triangle, blocks right of the diagonal read rows as before,
+// blocks left of it read the stored rows q, 16 consecutive p each, and the block on the
+// diagonal reads entry by entry.
+typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
 
-// complex V (split planes) x complex T
-__device__ inline void mm_cplx(const double* __restrict__ Vr, const double* __restrict__ Vi,
-                               int N, int rb, const double* tr, const double* ti, int lane,
-                               double4_t& accR, double4_t& accI) {
-  const int p = rb + (lane & 15);
-  const int s = lane >> 4;
-  const bool prow = p < N;
-  const int nkg = (N + 3) >> 2;
-  for (int kg = 0; kg < nkg; ++kg) {
-    const int q = 4 * kg + s;
-    const bool ok = prow && q < N;
-    const double ar = ok ? Vr[(int64_t)p * N + q] : 0.0;
-    const double ai = ok ? Vi[(int64_t)p * N + q] : 0.0;
-    const double br = tr[q * 16 + (lane & 15)];
-    const double bi = ti[q * 16 + (lane & 15)];
-    accR = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, accR, 0, 0, 0);
-    accR = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, accR, 0, 0, 0);
-    accI = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, accI, 0, 0, 0);
-    accI = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, accI, 0, 0, 0);
-  }
-}
+// the BLGP field of a float64 MFMA negates its operands; bit 0: A
+constexpr int MFMA_NEG_A = 1;
 
-// write a wave's 16x16 output tile (rows rb + lane/16 + 4r, col lane%16) into T planes
-__device__ inline void put_tile(double* tr, double* ti, int rb, int lane, const double4_t& R,
-                                const double4_t& I) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int q = rb + (lane >> 4) + 4 * r;
-    tr[q * 16 + (lane & 15)] = R[r];
-    ti[q * 16 + (lane & 15)] = I[r];
-  }
-}
+constexpr int TS_RS = 32;  // doubles per LDS row
+// Column c of row q of y sits at c ^ ts_swz(q): the B operands of a wave (rows 2 s + e,
+// 16 columns each) and its stores of D tiles (rows s + 4 r) then meet both halves of the
+// banks
+__device__ inline int ts_swz(int q) { return (((q >> 1) ^ q) & 1) << 4; }
 
-__device__ __forceinline__ void taylor_body(int N, int n, int n_terms_k,
-                                            cplx* __restrict__ walkers,
-                                            const double* __restrict__ expE,
-                                            const double* __restrict__ vhs, int rows_pad,
-                                            const int w, const int chunk) {
-  extern __shared__ double T[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <bool PACKED>
+__device__ __forceinline__ void taylor_stream_body(int N, int n, int n_terms_k,
+                                                   cplx* __restrict__ walkers,
+                                                   const double* __restrict__ expE,
+                                                   const double* __restrict__ vhs, int nv,
+                                                   const int w, const int c0) {
+  constexpr int RS = TS_RS;
+  extern __shared__ double YS[];  // [16 ceil(N / 16)][RS]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = lane >> 4, col = lane & 15;
   const int rb = wave * 16;
-  const int c0 = chunk * 16;
+  const int nb = (N + 15) >> 4;         // blocks of 16 k
+  const int pc = min(rb + col, N - 1);  // A row of this lane (rows >= N are never stored)
   cplx* phi = walkers + (int64_t)w * N * n;
-  const double* Vr = vhs + (int64_t)w * 2 * N * N;
-  const double* Vi = Vr + (int64_t)N * N;
+  const double* Vr = vhs + (int64_t)w * 2 * nv;
+  const double* Vi = Vr + nv;
+  // V planes hold all N^2 entries row-major, or (PACKED: nv = N(N+1)/2, symmetric V) the
+  // upper triangle row by row: entry (a, b), a <= b, at a N - a (a - 1) / 2 + b - a
 
-  // load the chunk (zero padded) into buffer 0
-  {
-    double* tr = tptr(T, rows_pad, 0, 0);
-    double* ti = tptr(T, rows_pad, 0, 1);
-    for (int e = threadIdx.x; e < rows_pad * 16; e += blockDim.x) {
-      const int q = e >> 4, j = e & 15;
-      cplx v = cplx{0.0, 0.0};
-      if (q < N && c0 + j < n) v = phi[(int64_t)q * n + c0 + j];
-      tr[e] = v.re;
-      ti[e] = v.im;
-    }
+  // the walker's chunk; rows q >= N and columns past n zero
+  for (int e = threadIdx.x; e < nb * 256; e += blockDim.x) {
+    const int q = e >> 4, j = e & 15;
+    const cplx z = phi[min(q, N - 1) * n + min(c0 + j, n - 1)];
+    const bool ok = q < N && c0 + j < n;
+    double* row = YS + q * RS;
+    const int sw = ts_swz(q);
+    row[j ^ sw] = ok ? z.re : 0.0;
+    row[(16 + j) ^ sw] = ok ? z.im : 0.0;
   }
   __syncthreads();
 
-  // t0 = E w
-  double4_t t0R = {0, 0, 0, 0}, t0I = {0, 0, 0, 0};
-  mm_real(expE, N, rb, tptr(T, rows_pad, 0, 0), tptr(T, rows_pad, 0, 1), lane, t0R, t0I);
-  put_tile(tptr(T, rows_pad, 1, 0), tptr(T, rows_pad, 1, 1), rb, lane, t0R, t0I);
-  __syncthreads();
-
-  double4_t sR = {0, 0, 0, 0}, sI = {0, 0, 0, 0};
-  int cur = 1;
-  double fact = 1.0;
-  for (int k = 1; k <= n_terms_k; ++k) {
-    fact *= (double)k;
-    double4_t cR = {0, 0, 0, 0}, cI = {0, 0, 0, 0};
-    mm_cplx(Vr, Vi, N, rb, tptr(T, rows_pad, cur, 0), tptr(T, rows_pad, cur, 1), lane, cR, cI);
+  auto put = [&](const double4_t& yr, const double4_t& yi) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      sR[r] += cR[r] / fact;
-      sI[r] += cI[r] / fact;
+      const int q = rb + s + 4 * r;
+      if (q < N) {
+        double* row = YS + q * RS;
+        const int sw = ts_swz(q);
+        row[col ^ sw] = yr[r];
+        row[(16 + col) ^ sw] = yi[r];
+      }
     }
-    put_tile(tptr(T, rows_pad, cur ^ 1, 0), tptr(T, rows_pad, cur ^ 1, 1), rb, lane, cR, cI);
-    __syncthreads();
-    cur ^= 1;
+  };
+  // loads at a uniform base plus a 32-bit byte offset
+  auto at = [](const double* base, uint32_t o) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + o);
+  };
+  auto load2 = [](double* a, const double* base, uint32_t o) {
+    const d2u_t x = *reinterpret_cast<const d2u_t*>(reinterpret_cast<const char*>(base) + o);
+    a[0] = x.x;
+    a[1] = x.y;
+  };
+  // entries past the row's end (of the last block) are zeroed: they meet zero rows of y
+  auto mask = [&](double (&a)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      a[u] = 16 * (nb - 1) + 8 * (u >> 1) + 2 * s + (u & 1) < N ? a[u] : 0.0;
+  };
+  // B of the MFMAs with k = row + 2 s + e: two buffers, one read from LDS while the other
+  // is in use
+  struct Yop {
+    double r, i;
+  };
+  const int sw0 = (s & 1) << 4;  // ts_swz of even rows 2 s; odd rows: the other half
+  const double* y0r = YS + 2 * s * RS + (col ^ sw0);
+  const double* y0i = YS + 2 * s * RS + (col ^ sw0 ^ 16);
+  auto loady = [&](Yop& y, int row, int e) {
+    y.r = (e ? y0i : y0r)[row * RS];
+    y.i = (e ? y0r : y0i)[row * RS];
+  };
+  // One pass over k: mma(y, u) with the operand of MFMA u of each block, refill(g, h) once
+  // pair h is free
+  auto pass = [&](auto&& mma, auto&& refill, auto&& last) {
+    Yop y0, y1;
+    loady(y0, 0, 0);
+#pragma unroll 1
+    for (int g = 0; g < nb; ++g) {
+      const int gn = g + 1 < nb ? g + 1 : 0;
+      if (g == nb - 1) last();
+      loady(y1, 16 * g + 1, 1);
+      mma(y0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      loady(y0, 16 * g + 8, 0);
+      mma(y1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      refill(gn, 0);
+      loady(y1, 16 * g + 9, 1);
+      mma(y0, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      loady(y0, 16 * gn, 0);
+      mma(y1, 3);
+      __builtin_amdgcn_sched_barrier(0);
+      refill(gn, 1);
+    }
+  };
+  const double4_t z4 = {0.0, 0.0, 0.0, 0.0};
+  double vr[4], vi[4];
+  // E y, a real operator on both halves (rows of E in vr)
+  const uint32_t erow = 8u * (uint32_t)(pc * N + 2 * s);
+  auto load_e = [&](int g, int h) { load2(vr + 2 * h, expE, erow + 128u * g + 64u * h); };
+  auto e_product = [&](double4_t& ar, double4_t& ai) {
+    ar = ai = z4;
+    load_e(0, 0);
+    load_e(0, 1);
+    pass(
+        [&](const Yop& y, int u) {
+          ar = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[u], y.r, ar, 0, 0, 0);
+          ai = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[u], y.i, ai, 0, 0, 0);
+        },
+        load_e, [&]() { mask(vr); });
+  };
+  // pair h of block g of V
+  const uint32_t vrow =
+      8u * (uint32_t)(PACKED ? pc * N - (pc * (pc - 1)) / 2 - pc + 2 * s : pc * N + 2 * s);
+  auto load_v = [&](int g, int h) {
+    if (!PACKED || g > wave) {
+      const uint32_t o = vrow + 128u * g + 64u * h;
+      load2(vr + 2 * h, Vr, o);
+      load2(vi + 2 * h, Vi, o);
+    } else if (g < wave) {  // entries (q, p), q < p: rows q and q + 1 N - q - 1 apart
+      const int q = 16 * g + 8 * h + 2 * s;
+      const uint32_t o = 8u * (uint32_t)(q * N - (q * (q + 1)) / 2 + pc);
+      const uint32_t o1 = o + 8u * (uint32_t)(N - q - 1);
+      vr[2 * h] = at(Vr, o);
+      vi[2 * h] = at(Vi, o);
+      vr[2 * h + 1] = at(Vr, o1);
+      vi[2 * h + 1] = at(Vi, o1);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int q = min(16 * g + 8 * h + 2 * s + e, N - 1);
+        const int a = min(pc, q), b = max(pc, q);
+        const uint32_t o = 8u * (uint32_t)(a * N - (a * (a - 1)) / 2 + (b - a));
+        vr[2 * h + e] = at(Vr, o);
+        vi[2 * h + e] = at(Vi, o);
+      }
+    }
+  };
+
+  double4_t t0r, t0i, ur, ui;
+  e_product(t0r, t0i);
+  load_v(0, 0);
+  load_v(0, 1);
+  lds_barrier();
+  put(t0r, t0i);
+  lds_barrier();
+#pragma unroll 1
+  for (int k = n_terms_k; k >= 1; --k) {
+    ur = ui = z4;
+    // (the pass ends with block 0 of V loaded for the next term)
+    pass(
+        [&](const Yop& y, int u) {
+          ur = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[u], y.r, ur, 0, 0, 0);
+          ui = __builtin_amdgcn_mfma_f64_16x16x4f64(vr[u], y.i, ui, 0, 0, 0);
+          ur = __builtin_amdgcn_mfma_f64_16x16x4f64(vi[u], y.i, ur, 0, 0, MFMA_NEG_A);
+          ui = __builtin_amdgcn_mfma_f64_16x16x4f64(vi[u], y.r, ui, 0, 0, 0);
+        },
+        load_v,
+        [&]() {
+          mask(vr);
+          mask(vi);
+        });
+    lds_barrier();
+    const double dk = (double)k, rk = 1.0 / dk;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      ur[r] = t0r[r] + div_small(ur[r], dk, rk);
+      ui[r] = t0i[r] + div_small(ui[r], dk, rk);
+    }
+    put(ur, ui);
+    lds_barrier();
   }
-  // R = t0 + sum_k terms
+  e_product(ur, ui);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    t0R[r] += sR[r];
-    t0I[r] += sI[r];
-  }
-  put_tile(tptr(T, rows_pad, 0, 0), tptr(T, rows_pad, 0, 1), rb, lane, t0R, t0I);
-  __syncthreads();
-  double4_t oR = {0, 0, 0, 0}, oI = {0, 0, 0, 0};
-  mm_real(expE, N, rb, tptr(T, rows_pad, 0, 0), tptr(T, rows_pad, 0, 1), lane, oR, oI);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int p = rb + (lane >> 4) + 4 * r;
-    const int j = c0 + (lane & 15);
-    if (p < N && j < n) phi[(int64_t)p * n + j] = cplx{oR[r], oI[r]};
+    const int p = rb + s + 4 * r, j = c0 + col;
+    if (p < N && j < n) phi[p * n + j] = cplx{ur[r], ui[r]};
   }
 }
 
-__global__ __launch_bounds__(1024) void taylor_kernel(
-    int N, int n, int n_terms_k, cplx* __restrict__ walkers, const double* __restrict__ expE,
-    const double* __restrict__ vhs, int rows_pad) {
-  taylor_body(N, n, n_terms_k, walkers, expE, vhs, rows_pad, blockIdx.x, blockIdx.y);
+// Blocks are dealt round-robin to the 8 XCDs (block b on XCD b % 8): block
+// b = 8 (q units + u) + r takes unit u (a column chunk of one spin) of walker 8 q + r, so
+// the units of a walker run on one XCD, one dispatch round apart, and mostly share its V
+// (the same one for both spins unless the vectors are spin resolved) through that XCD's
+// L2; and the spins of a launch fill its last round together.
+__device__ inline bool stream_block(int b, int W, int units, int* w, int* unit) {
+  const int g = b >> 3;
+  *unit = g % units;
+  *w = 8 * (g / units) + (b & 7);
+  return *w < W;
 }
 
-// grouped: local block b = walker * chunks + chunk, chunks = ceil(n / 16)
-__global__ __launch_bounds__(1024) void taylor_grouped_kernel(const TaylorArgs* __restrict__ args,
-                                                              const int* __restrict__ start,
-                                                              int nprob) {
+// column chunks of a spin with n columns
+__host__ __device__ inline int stream_chunks(int n) { return (n + 15) / 16; }
+
+// registers for two workgroups per CU up to STREAM_SMALL waves (N <= 192), else one
+constexpr int STREAM_SMALL = 12;
+constexpr int stream_threads(bool small) { return small ? 64 * STREAM_SMALL : 1024; }
+constexpr int stream_wpe(bool small) { return small ? 6 : 4; }
+
+template <bool SMALL>
+__global__ __launch_bounds__(stream_threads(SMALL), stream_wpe(SMALL)) void taylor_stream_kernel(
+    int N, int n0, int n1, int n_terms_k, int W, cplx* __restrict__ w0, cplx* __restrict__ w1,
+    const double* __restrict__ e0, const double* __restrict__ e1, const double* __restrict__ v0,
+    const double* __restrict__ v1, int nv) {
+  const int u0 = stream_chunks(n0), u1 = n1 ? stream_chunks(n1) : 0;
+  int w, u;
+  if (!stream_block(blockIdx.x, W, u0 + u1, &w, &u)) return;
+  const bool dn = u >= u0;
+  const int n = dn ? n1 : n0, c0 = 16 * (dn ? u - u0 : u);
+  cplx* wk = dn ? w1 : w0;
+  const double *E = dn ? e1 : e0, *V = dn ? v1 : v0;
+  if (nv == N * N)
+    taylor_stream_body<false>(N, n, n_terms_k, wk, E, V, nv, w, c0);
+  else
+    taylor_stream_body<true>(N, n, n_terms_k, wk, E, V, nv, w, c0);
+}
+
+template <bool SMALL>
+__global__ __launch_bounds__(stream_threads(SMALL), stream_wpe(SMALL)) void taylor_stream_grouped_kernel(
+    const TaylorArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
   const TaylorArgs a = args[p];
-  const int b = blockIdx.x - start[p], chunks = (a.n + 15) / 16;
-  taylor_body(a.N, a.n, a.K, a.walkers, static_cast<const double*>(a.E),
-              static_cast<const double*>(a.vhs), a.rows_pad, b / chunks, b % chunks);
+  int w, u;
+  if (!stream_block(blockIdx.x - start[p], a.W, stream_chunks(a.n), &w, &u)) return;
+  if (a.nv == a.N * a.N)
+    taylor_stream_body<false>(a.N, a.n, a.K, a.walkers, static_cast<const double*>(a.E),
+                              static_cast<const double*>(a.vhs), a.nv, w, 16 * u);
+  else
+    taylor_stream_body<true>(a.N, a.n, a.K, a.walkers, static_cast<const double*>(a.E),
+                             static_cast<const double*>(a.vhs), a.nv, w, 16 * u);
+}
+
+inline int stream_blocks(int W, int units) { return 8 * ((W + 7) / 8) * units; }
+inline size_t stream_shm(int N) { return (size_t)((N + 15) / 16) * 16 * TS_RS * sizeof(double); }
+
+// both spins of the context (or its one)
+template <bool SMALL>
+int launch_stream(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
+  const int N = c->d.norb, s1 = c->nspin - 1;
+  const size_t shm = stream_shm(N);
+  static int lds_limit = 0;
+  const int rc = ensure_dyn_lds((const void*)taylor_stream_kernel<SMALL>, shm, &lds_limit);
+  if (rc) return rc;
+  const int n0 = c->nocc[0], n1 = c->nspin == 2 ? c->nocc[1] : 0;
+  const int units = stream_chunks(n0) + (n1 ? stream_chunks(n1) : 0);
+  hipLaunchKernelGGL((taylor_stream_kernel<SMALL>), dim3(stream_blocks(W, units)),
+                     dim3(64 * ((N + 15) / 16)), shm, c->stream, N, n0, n1, c->d.n_exp_terms - 1,
+                     W, wup, wdn, c->exp_h1[0], c->exp_h1[s1], vhs_of(c, 0),
+                     vhs_of(c, s1), c->vhs_nv);
+  LAUNCH_CHECK();
+  return AFQMC_OK;
 }
 
 // ------------------------------------------------------------------------------------
@@ -174,12 +325,6 @@ template <int CTP>
 struct RegTile {
   static constexpr int RS = 16 * CTP + ((CTP % 2 == 0) ? 16 : 0);  // == 16 (mod 32) doubles
 };
-
-// x / k for a small integer k, rk = 1 / k: the quotient corrected by its residual
-__device__ inline double div_small(double x, double k, double rk) {
-  const double q = x * rk;
-  return fma(fma(-q, k, x), rk, q);
-}
 
 template <int NW, int CTP>
 __device__ __forceinline__ void taylor_reg_body(int N, int n, int n_terms_k,
@@ -368,7 +513,7 @@ int launch_reg(afqmc_ctx* c, int W, int n, cplx* wk, const double* E, const doub
   const int rc = ensure_dyn_lds((const void*)taylor_reg_kernel<NW, CTP>, shm, &lds_limit);
   if (rc) return rc;
   hipLaunchKernelGGL((taylor_reg_kernel<NW, CTP>), dim3(W), dim3(NW * 64), shm, c->stream, N, n,
-                     c->d.n_exp_terms - 1, wk, E, V, N * N);
+                     c->d.n_exp_terms - 1, wk, E, V, c->vhs_nv);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }
@@ -1044,7 +1189,7 @@ void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl) {
   const int N = c->d.norb, n = c->nocc[s];
   const int ctp = (2 * n + 15) / 16 > 4 ? 4 : (2 * n + 15) / 16;
   pl->nthreads = ((N + 15) / 16) * 64;
-  pl->blocks_per_walker = 1;
+  pl->nblocks = c->d.n_walkers;
   pl->nkgv = 0;
   pl->ct = 0;
   if (c->taylor_bf) {
@@ -1068,8 +1213,8 @@ void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl) {
     pl->shm = reg_shm(N, ctp);
   } else {
     pl->kind = TAYLOR_STREAM_F64;
-    pl->blocks_per_walker = (n + 15) / 16;
-    pl->shm = (size_t)((N + 15) / 16) * 16 * 16 * 4 * sizeof(double);
+    pl->nblocks = stream_blocks(c->d.n_walkers, stream_chunks(n));
+    pl->shm = stream_shm(N);
   }
 }
 
@@ -1134,21 +1279,8 @@ int launch_taylor(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
     }
     return AFQMC_OK;
   }
-  const int nwaves = (N + 15) / 16;
-  const int rows_pad = nwaves * 16;
-  const size_t shm = (size_t)rows_pad * 16 * 4 * sizeof(double);
-  static int lds_limit = 0;
-  const int lrc = ensure_dyn_lds((const void*)taylor_kernel, shm, &lds_limit);
-  if (lrc) return lrc;
-  for (int s = 0; s < c->nspin; ++s) {
-    const int n = c->nocc[s];
-    cplx* wk = (s == 0) ? wup : wdn;
-    dim3 grid(W, (n + 15) / 16);
-    hipLaunchKernelGGL(taylor_kernel, grid, dim3(nwaves * 64), shm, c->stream, N, n,
-                       c->d.n_exp_terms - 1, wk, c->exp_h1[s], vhs_of(c, s), rows_pad);
-    LAUNCH_CHECK();
-  }
-  return AFQMC_OK;
+  return (N + 15) / 16 <= STREAM_SMALL ? launch_stream<true>(c, W, wup, wdn)
+                                       : launch_stream<false>(c, W, wup, wdn);
 }
 
 namespace {
@@ -1220,7 +1352,10 @@ int launch_taylor_grouped(hipStream_t st, int kind, int nkgv, int ct, const Tayl
       default: return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: column tiles %d", ct);
     }
   }
-  static int lim64 = 0;
-  return launch_grouped_fn(taylor_grouped_kernel, st, args, start, nprob, nblocks, nthreads, shm,
-                           &lim64);
+  static int lim64[2] = {};
+  if (nthreads <= 64 * STREAM_SMALL)
+    return launch_grouped_fn(taylor_stream_grouped_kernel<true>, st, args, start, nprob, nblocks,
+                             nthreads, shm, &lim64[0]);
+  return launch_grouped_fn(taylor_stream_grouped_kernel<false>, st, args, start, nprob, nblocks,
+                           nthreads, shm, &lim64[1]);
 }
