@@ -109,6 +109,27 @@ int set_device(const afqmc_ctx* c) {
   return AFQMC_OK;
 }
 
+// Sets c->vhs_nv: N (N + 1) / 2 when the count Cholesky vectors are symmetric, else N^2.
+// The mixed mode takes an asymmetry of 1e-12 of the largest entry, below its products'
+// rounding (2^-17); the other modes one of 2^-50, the rounding that rotating integrals to
+// an orbital basis leaves.
+int symmetric_vectors(afqmc_ctx* c, const double* chol, int64_t count) {
+  const int N = c->d.norb;
+  c->vhs_nv = N * N;
+  unsigned long long st[2] = {0ull, 0ull};
+  int rc = dalloc(c, &c->sym_stat, 2);
+  if (!rc) rc = zero_async(c->sym_stat, sizeof(st), c->stream);
+  if (!rc) rc = launch_sym_check(c->stream, N, count, chol, c->sym_stat);
+  if (!rc) rc = copy_async(st, c->sym_stat, sizeof(st), c->stream);
+  if (!rc) rc = sync_stream(c->stream);
+  if (rc) return rc;
+  double asym, amax;
+  std::memcpy(&asym, &st[0], sizeof(double));
+  std::memcpy(&amax, &st[1], sizeof(double));
+  if (asym <= (c->mixed ? 1e-12 : 0x1p-50) * amax) c->vhs_nv = N * (N + 1) / 2;
+  return AFQMC_OK;
+}
+
 // fb[w][c][g] = mult * sum_s green_s[w][c][:] . rot_chol_s[g][:], as c->fb_parts split-K
 // slices of (2W, G) that the consumers add in slice order
 // arithmetic: FB_BF16 the split-bf16 planes of the mixed mode; otherwise the float64
@@ -226,9 +247,13 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
       off_h1 += (size_t)n * N;
       off_rc += (size_t)G * n * N;
     }
-    // transposed Cholesky vectors (N*N, G): K-contiguous B operand of the VHS GEMM,
-    // transposed on the device from the (G, N*N) array (read in place when the caller
-    // passes device memory, else from a temporary upload)
+    // transposed Cholesky vectors (one row per entry of V): K-contiguous B operand of the
+    // VHS GEMM, transposed on the device from the (G, N*N) array (read in place when the
+    // caller passes device memory, else from a temporary upload).  Symmetric vectors, as
+    // they are for real orbitals, keep V as its upper triangle: half the VHS product, its
+    // output and the Taylor kernels' reads.
+    c->mixed = d.precision == AFQMC_PREC_BF16X3;
+    c->f32 = d.precision == AFQMC_PREC_FP32;
     {
       const size_t per = (size_t)G * N * N;
       double* raw = nullptr;
@@ -237,9 +262,11 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
         rc = upload(c, &raw, ham->chol, c->chol_spins * per);
         src = raw;
       }
-      if (!rc) rc = dalloc(c, &c->chol_t, c->chol_spins * per);
+      if (!rc) rc = symmetric_vectors(c, src, (int64_t)c->chol_spins * G);
+      if (!rc) rc = dalloc(c, &c->chol_t, (size_t)c->chol_spins * c->vhs_nv * G);
       for (int cs = 0; cs < c->chol_spins && !rc; ++cs)
-        rc = launch_transpose_f64(c->stream, G, N * N, src + cs * per, c->chol_t + cs * per);
+        rc = launch_transpose_f64(c->stream, G, N * N, c->vhs_nv == N * N ? 0 : N, src + cs * per,
+                                  chol_t_of(c, cs));
       (void)hipStreamSynchronize(c->stream);
       if (raw) {
         (void)hipFree(raw);
@@ -250,40 +277,16 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
     TRY(upload(c, &c->mf_shifts, reinterpret_cast<const cplx*>(ham->mf_shifts), (size_t)G));
 
     // mixed mode: split-bf16 planes of the contraction operands (zero padded to 32)
-    c->mixed = d.precision == AFQMC_PREC_BF16X3;
-    c->f32 = d.precision == AFQMC_PREC_FP32;
-    c->vhs_nv = N * N;
     c->Gp = (G + 31) / 32 * 32;
     c->Np32 = (N + 31) / 32 * 32;
     c->taylor_bf = c->mixed;  // split-bf16 Taylor kernels (register or streaming form)
     if (c->mixed) {
       const size_t nn = (size_t)N * N;
-      // V kept as its upper triangle (half the VHS product, its output and the Taylor
-      // kernels' reads) when the Cholesky vectors are symmetric, as they are for real
-      // orbitals
-      {
-        unsigned long long st[2] = {0ull, 0ull};
-        TRY(dalloc(c, &c->sym_stat, 2));
-        TRY(zero_async(c->sym_stat, 2 * sizeof(unsigned long long), c->stream));
-        for (int cs = 0; cs < c->chol_spins; ++cs)  // maxima accumulate over the spins
-          TRY(launch_sym_check(c->stream, N, G, chol_t_of(c, cs), c->sym_stat));
-        TRY(copy_async(st, c->sym_stat, sizeof(st), c->stream));
-        TRY(sync_stream(c->stream));
-        double asym, amax;
-        std::memcpy(&asym, &st[0], sizeof(double));
-        std::memcpy(&amax, &st[1], sizeof(double));
-        if (asym <= 1e-12 * amax) c->vhs_nv = N * (N + 1) / 2;
-      }
       for (int h = 0; h < 2; ++h)
         TRY(dalloc(c, &c->chol_t_bf[h], (size_t)c->chol_spins * c->vhs_nv * c->Gp));
-      for (int cs = 0; cs < c->chol_spins; ++cs) {
-        if (c->vhs_nv != N * N)
-          TRY(launch_split_bf16_sym(c->stream, N, G, chol_t_of(c, cs), chol_t_bf_of(c, 0, cs),
-                                    chol_t_bf_of(c, 1, cs), c->Gp));
-        else
-          TRY(launch_split_bf16(c->stream, (int)nn, G, chol_t_of(c, cs), G,
-                                chol_t_bf_of(c, 0, cs), chol_t_bf_of(c, 1, cs), c->Gp));
-      }
+      for (int cs = 0; cs < c->chol_spins; ++cs)
+        TRY(launch_split_bf16(c->stream, c->vhs_nv, G, chol_t_of(c, cs), G, chol_t_bf_of(c, 0, cs),
+                              chol_t_bf_of(c, 1, cs), c->Gp));
       for (int s = 0; s < c->nspin; ++s) {
         const size_t rows = (size_t)G * c->nocc[s];
         for (int h = 0; h < 2; ++h) {
@@ -334,7 +337,7 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
     }
     TRY(dalloc(c, &c->fb, (size_t)c->fb_cap * W * 2 * G));
     TRY(dalloc(c, &c->xs, (size_t)W * 2 * G));
-    if (!c->taylor_bf) TRY(dalloc(c, &c->vhs, (size_t)c->chol_spins * W * 2 * N * N));
+    if (!c->taylor_bf) TRY(dalloc(c, &c->vhs, (size_t)c->chol_spins * W * 2 * c->vhs_nv));
     TRY(dalloc(c, &c->terms, (size_t)W * 2));
     TRY(dalloc(c, &c->dets, (size_t)W * 2));
     {
@@ -390,7 +393,6 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
   if ((rc = set_device(c))) return rc;
   cplx* wu = static_cast<cplx*>(walkers_up);
   cplx* wd = static_cast<cplx*>(walkers_dn);
-  const int N = c->d.norb;
   // force bias: Green of the current walkers (or the one the previous step left),
   // then the rot_chol contraction
   const bool reuse = (flags & AFQMC_STEP_REUSE_GREEN) && c->green_src == walkers_up &&
@@ -419,11 +421,11 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
                                        chol_t_bf_of(c, 1, cs), c->Gp, vhs_f32_of(c, cs),
                                        c->vhs_nv, 1, 0);
       else if (c->f32)
-        rc = launch_gemm_nt_f32(c->stream, 2 * W, N * N, c->d.nchol, 1.0, c->xs, c->d.nchol,
-                                chol_t_of(c, cs), c->d.nchol, 0.0, vhs_of(c, cs), N * N);
+        rc = launch_gemm_nt_f32(c->stream, 2 * W, c->vhs_nv, c->d.nchol, 1.0, c->xs, c->d.nchol,
+                                chol_t_of(c, cs), c->d.nchol, 0.0, vhs_of(c, cs), c->vhs_nv);
       else
-        rc = launch_gemm_nt_f64(c->stream, 2 * W, N * N, c->d.nchol, 1.0, c->xs, c->d.nchol,
-                                chol_t_of(c, cs), c->d.nchol, 0.0, vhs_of(c, cs), N * N);
+        rc = launch_gemm_nt_f64(c->stream, 2 * W, c->vhs_nv, c->d.nchol, 1.0, c->xs, c->d.nchol,
+                                chol_t_of(c, cs), c->d.nchol, 0.0, vhs_of(c, cs), c->vhs_nv);
     }
     if (rc) return rc;
   }

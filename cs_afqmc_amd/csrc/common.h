@@ -209,7 +209,7 @@ struct afqmc_ctx {
   double* trial[2];      // (N, n_sigma)
   double* rot_h1[2];     // (n_sigma, N)
   double* rot_chol[2];   // (G, n_sigma, N)
-  double* chol_t;        // (N*N, G): transposed Cholesky vectors
+  double* chol_t;        // (vhs_nv, G): transposed Cholesky vectors
   double* exp_h1[2];     // (N, N)
   cplx* mf_shifts;       // (G)
 
@@ -236,7 +236,7 @@ struct afqmc_ctx {
   int fb_cap;            // slices allocated
   int fb_parts;          // slices written by the last force-bias contraction
   double* xs;            // (W, 2, G): i sqrt(dt) * shifted fields, split
-  double* vhs;           // (W, 2, N*N)
+  double* vhs;           // chol_spins x (W, 2, vhs_nv), + padding
   cplx* terms;           // (W, 2): shift_term, fb_term
   cplx* dets;            // (W, 2): det(C_sigma^H w_sigma)
   cplx* energy_x;        // (sum_s g_tiles_s, W) exchange partial sums
@@ -257,13 +257,13 @@ struct afqmc_ctx {
 // set shared by both spins unless the vectors are spin resolved.
 inline int chol_spin(const afqmc_ctx* c, int s) { return c->chol_spins == 2 ? s : 0; }
 inline double* chol_t_of(const afqmc_ctx* c, int s) {
-  return c->chol_t + (size_t)chol_spin(c, s) * c->d.norb * c->d.norb * c->d.nchol;
+  return c->chol_t + (size_t)chol_spin(c, s) * c->vhs_nv * c->d.nchol;
 }
 inline uint16_t* chol_t_bf_of(const afqmc_ctx* c, int h, int s) {
   return c->chol_t_bf[h] + (size_t)chol_spin(c, s) * c->vhs_nv * c->Gp;
 }
 inline double* vhs_of(const afqmc_ctx* c, int s) {
-  return c->vhs + (size_t)chol_spin(c, s) * c->d.n_walkers * 2 * c->d.norb * c->d.norb;
+  return c->vhs + (size_t)chol_spin(c, s) * c->d.n_walkers * 2 * c->vhs_nv;
 }
 inline float* vhs_f32_of(const afqmc_ctx* c, int s) {
   return c->vhs_f32 + (size_t)chol_spin(c, s) * c->vhs_f32_stride;
@@ -338,8 +338,13 @@ int launch_gemm_nt_f32(hipStream_t s, int M, int N, int K, double alpha, const d
 int launch_gemm_nt_f32_split(hipStream_t s, int M, int N, int K, double alpha, const double* A,
                              int lda, const double* B, int ldb, double* C, int ldc, int splits,
                              int64_t c_split_stride);
-// dst (cols x rows) = src (rows x cols)^T, float64
-int launch_transpose_f64(hipStream_t s, int rows, int cols, const double* src, double* dst);
+// dst (cols x rows) = src (rows x cols)^T, float64; packed_n > 0: only the upper triangle
+// of each row's packed_n x packed_n matrix (dst packed_n (packed_n + 1) / 2 x rows)
+int launch_transpose_f64(hipStream_t s, int rows, int cols, int packed_n, const double* src,
+                         double* dst);
+// largest asymmetry and entry of count n x n matrices, as bit patterns into out[0], out[1]
+int launch_sym_check(hipStream_t s, int n, int64_t count, const double* L,
+                     unsigned long long* out);
 // gemm_bf16x3.hip: split-bf16 NT GEMM (K, lda, ldb multiples of 32 / 8), float / double out
 int launch_gemm_nt_bf16x3_f32(hipStream_t s, int M, int N, int K, float alpha,
                               const uint16_t* Ah, const uint16_t* Al, int64_t lda,
@@ -351,9 +356,6 @@ int launch_gemm_nt_bf16x3_f64(hipStream_t s, int M, int N, int K, float alpha,
                               int64_t ldc, int splits, int64_t c_split_stride);
 int launch_split_bf16(hipStream_t s, int rows, int cols, const double* x, int64_t ld_src,
                       uint16_t* hi, uint16_t* lo, int64_t ld_dst);
-int launch_sym_check(hipStream_t s, int N, int G, const double* chol_t, unsigned long long* out);
-int launch_split_bf16_sym(hipStream_t s, int N, int G, const double* chol_t, uint16_t* hi,
-                          uint16_t* lo, int ld_dst);
 // measure.hip: green_f64 -> c->green (float64 split layout); green_bf -> c->green_bf
 // With tail, the last spin's launch also applies the per-walker weight update (thread 0 of
 // each walker's block); the population-control shift then comes from launch_pcs.

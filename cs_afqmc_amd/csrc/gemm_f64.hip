@@ -261,8 +261,10 @@ int launch_gemm_f64_grouped(hipStream_t s, int bm, const GemmArgs* args, const i
 
 namespace {
 
-// dst (cols x rows) = src (rows x cols)^T through 32 x 32 LDS tiles
-__global__ __launch_bounds__(256) void transpose_f64_kernel(int rows, int cols,
+// dst (cols x rows) = src (rows x cols)^T through 32 x 32 LDS tiles.  With n > 0 (cols =
+// n^2) only the columns (p, k), p <= k, of a row's n x n matrix are kept: dst row
+// p n - p (p - 1) / 2 + k - p, the upper triangle row by row.
+__global__ __launch_bounds__(256) void transpose_f64_kernel(int rows, int cols, int n,
                                                            const double* __restrict__ src,
                                                            double* __restrict__ dst) {
   __shared__ double tile[32][33];
@@ -274,18 +276,77 @@ __global__ __launch_bounds__(256) void transpose_f64_kernel(int rows, int cols,
   }
   __syncthreads();
   for (int j = ty; j < 32; j += 8) {
-    const int c = c0 + j, r = r0 + tx;
-    if (r < rows && c < cols) dst[(int64_t)c * rows + r] = tile[tx][j];
+    int c = c0 + j;
+    const int r = r0 + tx;
+    if (r >= rows || c >= cols) continue;
+    if (n) {
+      const int p = c / n, k = c - p * n;
+      if (k < p) continue;
+      c = p * n - (p * (p - 1)) / 2 + k - p;
+    }
+    dst[(int64_t)c * rows + r] = tile[tx][j];
+  }
+}
+
+// Symmetry of count n x n matrices: out[0] = max |L[p][k] - L[k][p]| and out[1] = max |L|
+// as the bit patterns of non-negative doubles (ordered like the values, so atomicMax
+// applies).  A block takes one pair (I, J), I <= J, of 32 x 32 tiles of one matrix, both
+// read along rows, the second one compared through LDS.
+__global__ __launch_bounds__(256) void sym_check_kernel(int n, int nt,
+                                                        const double* __restrict__ L,
+                                                        unsigned long long* __restrict__ out) {
+  __shared__ double tile[32][33];
+  int I = 0, J = blockIdx.x;
+  while (J >= nt - I) J -= nt - I++;
+  J += I;
+  const double* m = L + (int64_t)blockIdx.y * n * n;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  double asym = 0.0, amax = 0.0;
+  for (int j = ty; j < 32; j += 8) {
+    const int r = J * 32 + j, c = I * 32 + tx;
+    const double v = (r < n && c < n) ? m[(int64_t)r * n + c] : 0.0;
+    tile[j][tx] = v;
+    amax = fmax(amax, fabs(v));
+  }
+  __syncthreads();
+  for (int j = ty; j < 32; j += 8) {
+    const int r = I * 32 + j, c = J * 32 + tx;
+    if (r < n && c < n) {
+      const double v = m[(int64_t)r * n + c];
+      amax = fmax(amax, fabs(v));
+      asym = fmax(asym, fabs(v - tile[tx][j]));
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    asym = fmax(asym, __shfl_xor(asym, off, 64));
+    amax = fmax(amax, __shfl_xor(amax, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    if (asym > 0.0) atomicMax(&out[0], (unsigned long long)__double_as_longlong(asym));
+    if (amax > 0.0) atomicMax(&out[1], (unsigned long long)__double_as_longlong(amax));
   }
 }
 
 }  // namespace
 
-int launch_transpose_f64(hipStream_t s, int rows, int cols, const double* src, double* dst) {
+int launch_transpose_f64(hipStream_t s, int rows, int cols, int packed_n, const double* src,
+                         double* dst) {
   if (rows <= 0 || cols <= 0) return AFQMC_OK;
   dim3 grid((cols + 31) / 32, (rows + 31) / 32);
   if (grid.y > 65535) return afqmc_set_error(AFQMC_ERR_SIZE, "transpose: %d rows", rows);
-  hipLaunchKernelGGL(transpose_f64_kernel, grid, dim3(256), 0, s, rows, cols, src, dst);
+  hipLaunchKernelGGL(transpose_f64_kernel, grid, dim3(256), 0, s, rows, cols, packed_n, src, dst);
   LAUNCH_CHECK();
+  return AFQMC_OK;
+}
+
+int launch_sym_check(hipStream_t s, int n, int64_t count, const double* L,
+                     unsigned long long* out) {
+  const int nt = (n + 31) / 32;
+  for (int64_t c0 = 0; c0 < count; c0 += 65535) {
+    const unsigned nc = (unsigned)(count - c0 < 65535 ? count - c0 : 65535);
+    hipLaunchKernelGGL(sym_check_kernel, dim3(nt * (nt + 1) / 2, nc), dim3(256), 0, s, n, nt,
+                       L + c0 * n * n, out);
+    LAUNCH_CHECK();
+  }
   return AFQMC_OK;
 }

@@ -91,3 +91,27 @@ def test_step_force_bias_and_energy(gpu, wt, norb, nelec, nchol, W):
     assert rel(pd["walkers"], od["walkers"]) < TOL
     assert rel(pd["overlaps"], od["overlaps"]) < TOL
     assert rel(pd["weights"], od["weights"]) < TOL
+
+
+@pytest.mark.parametrize("asym,packed", [(0.0, True), (2.0**-53, True), (1e-7, False)])
+@pytest.mark.parametrize("wt,norb,nelec,nchol,W", [("rhf", 33, (5, 5), 21, 9),
+                                                   ("uhf", 131, (5, 3), 18, 5)])
+def test_vhs_layout_follows_symmetry(gpu, wt, norb, nelec, nchol, W, asym, packed):
+    """V is kept as its upper triangle for Cholesky vectors that are symmetric up to the
+    rounding of an orbital rotation, and whole for any larger asymmetry; both layouts give
+    the oracle's step (register and streaming Taylor kernel)."""
+    print(f"symmetry {wt} N={norb} asym={asym}", flush=True)
+    hd, wd, nelec = problem(wt, norb, nelec, nchol)
+    chol = np.array(hd["chol"]).reshape(nchol, norb, norb)
+    skew = np.random.default_rng(5).uniform(-1.0, 1.0, (norb, norb))
+    chol += asym * np.max(np.abs(chol)) * np.triu(skew, 1)[None]
+    hd = dict(hd, chol=chol.reshape(nchol, norb * norb))
+    trial, prop, hdat, wave, oh = make(wt, norb, nelec, nchol, W, hd, wd)
+    entries = norb * (norb + 1) // 2 if packed else norb * norb
+    assert hdat["_afqmc_device"].vhs_entries() == entries
+    rng = np.random.default_rng(3)
+    walkers = problems.random_walkers(wt, norb, nelec, W, rng, near=wd["mo_coeff"], noise=0.1)
+    fields = rng.standard_normal((W, nchol))
+    pd, od = one_step(wt, trial, prop, hdat, wave, oh, wd, walkers, fields, gpu, norb)
+    assert rel(pd["walkers"], od["walkers"]) < TOL
+    assert rel(pd["weights"], od["weights"]) < TOL
