@@ -43,6 +43,27 @@ __host__ __device__ inline cplx cdiv(cplx a, cplx b) {
 }
 __host__ __device__ inline double cabs1(cplx a) { return fabs(a.re) + fabs(a.im); }
 
+// the value of lane l (uniform) in every lane
+__device__ inline double readlane_f64(double x, int l) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+__device__ inline cplx readlane_c(cplx x, int l) {
+  return cplx{readlane_f64(x.re, l), readlane_f64(x.im, l)};
+}
+
+// 1 / x for x > 0 of moderate range: hardware estimate plus two Newton steps
+__device__ inline double rcp_f64(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  double e = fma(-x, y, 1.0);
+  y = fma(y, e, y);
+  e = fma(-x, y, 1.0);
+  return fma(y, e, y);
+}
+
 // ---------------------------------------------------------------- bf16 split
 // x ~= hi + lo with hi = bf16(x), lo = bf16(x - hi), both rounded to nearest even
 // (gfx950's v_cvt_pk_bf16_f32 rounds to nearest even)
@@ -445,7 +466,7 @@ struct GemmArgs {
 
 // block ends: QR, overlap products, local energies
 struct QrArgs {
-  int m, n, use_lds;
+  int m, n, slots;  // slots: vectors held in LDS
   cplx* walkers;
 };
 struct OvcArgs {
@@ -490,10 +511,11 @@ int launch_exchange_grouped(hipStream_t st, int kind, const ExchArgs* args, cons
                             int nprob, int nblocks);
 int launch_energy_finish_grouped(hipStream_t st, const FinishArgs* args, const int* start,
                                  int nprob, int nblocks);
-// LDS bytes of the QR walker copy (0: factorised in place in global memory)
+// vectors the QR keeps in LDS, and their bytes
+int qr_slots(int m, int n);
 size_t qr_lds_bytes(int m, int n);
 int launch_qr_grouped(hipStream_t st, const QrArgs* args, const int* start, int nprob,
-                      int nblocks, size_t shm);
+                      int nblocks, size_t shm, int max_m, int max_n);
 int launch_overlap_combine_grouped(hipStream_t st, const OvcArgs* args, const int* start,
                                    int nprob, int nblocks);
 constexpr int OVC_NT = 256;  // threads (walkers) per overlap-combine block

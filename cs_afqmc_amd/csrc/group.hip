@@ -361,7 +361,7 @@ int build(afqmc_group* g) {
     std::vector<QrArgs> qa;
     std::vector<int> qs;
     size_t qshm = 0;
-    int b = 0;
+    int b = 0, max_m = 0, max_n = 0;
     for (const Member& m : g->mem) {
       afqmc_ctx* c = m.c;
       for (int s = 0; s < c->nspin; ++s) {
@@ -369,9 +369,11 @@ int build(afqmc_group* g) {
         QrArgs a{};
         a.m = c->d.norb;
         a.n = c->nocc[s];
-        a.use_lds = lb > 0 ? 1 : 0;
+        a.slots = qr_slots(a.m, a.n);
         a.walkers = s == 0 ? m.wup : m.wdn;
         qshm = std::max(qshm, lb);
+        max_m = std::max(max_m, a.m);
+        max_n = std::max(max_n, a.n);
         qa.push_back(a);
         qs.push_back(b);
         b += c->d.n_walkers;
@@ -379,6 +381,8 @@ int build(afqmc_group* g) {
     }
     g->qr = Launch{};
     g->qr.shm = qshm;
+    g->qr.k0 = max_m;
+    g->qr.k1 = max_n;
     g->qr.nprob = (int)qa.size();
     g->qr.nblocks = b;
     put_table(tab, g->qr, qa, qs);
@@ -827,7 +831,7 @@ extern "C" int afqmc_group_orthonormalize(afqmc_group* g) {
   if (rc) return rc;
   PhaseTimer t(&g->prof, g->stream, AFQMC_PH_QR);
   return launch_qr_grouped(g->stream, targs<QrArgs>(g, g->qr), tstart(g, g->qr), g->qr.nprob,
-                           g->qr.nblocks, g->qr.shm);
+                           g->qr.nblocks, g->qr.shm, g->qr.k0, g->qr.k1);
 }
 
 extern "C" int afqmc_group_overlap(afqmc_group* g) {

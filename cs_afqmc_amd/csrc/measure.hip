@@ -30,17 +30,6 @@ namespace {
 
 constexpr int MEAS_KC = 4;  // k-groups whose operands are loaded ahead of their MFMAs
 
-__device__ inline double readlane_f64(double x, int l) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-__device__ inline cplx readlane_c(cplx x, int l) {
-  return cplx{readlane_f64(x.re, l), readlane_f64(x.im, l)};
-}
-
 constexpr int GJ_PB = 4;  // panel width: the K of one f64 MFMA
 
 // LDS of the inversion: B (n x ld complex), then the state below (256 ints)
@@ -58,15 +47,6 @@ struct GjState {
   cplx det;
 };
 static_assert(sizeof(GjState) <= 256 * sizeof(int), "GjState exceeds its LDS slot");
-
-// 1 / x for x > 0 of moderate range: hardware estimate plus two Newton steps
-__device__ inline double rcp_f64(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-x, y, 1.0);
-  return fma(y, e, y);
-}
 
 // Panel [k0, k0 + pb) on one wave, lane = row r < n (n <= 64), rows kept in place
 // (implicit pivoting).  Pivot of column k: the largest |re| + |im| over the rows not yet

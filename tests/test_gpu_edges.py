@@ -115,3 +115,22 @@ def test_vhs_layout_follows_symmetry(gpu, wt, norb, nelec, nchol, W, asym, packe
     pd, od = one_step(wt, trial, prop, hdat, wave, oh, wd, walkers, fields, gpu, norb)
     assert rel(pd["walkers"], od["walkers"]) < TOL
     assert rel(pd["weights"], od["weights"]) < TOL
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e140, 1e-140])
+@pytest.mark.parametrize("norb,n", [(1, 1), (9, 9), (64, 16), (65, 17), (129, 33), (193, 49),
+                                    (250, 50), (256, 64)])
+def test_orthonormalize_columns_and_scales(gpu, norb, n, scale):
+    """Q of LAPACK's Householder QR, at each count of waves, columns per wave and rows per
+    lane, with all reflectors in LDS and in batches, and where the squared norms leave the
+    fast root's range.  Q of a Gaussian matrix moves by about its condition number (below
+    1e4 here) times 2^-53 per rounding: 1e-11."""
+    print(f"qr N={norb} n={n} scale={scale}", flush=True)
+    hd, wd, nelec = problem("rhf", norb, (n, n), 1)
+    trial, prop, hdat, wave, _ = make("rhf", norb, nelec, 1, 3, hd, wd)
+    rng = np.random.default_rng(17)
+    w = rng.standard_normal((3, norb, n)) + 1j * rng.standard_normal((3, norb, n))
+    got = hdat["_afqmc_device"].orthonormalize(to_dev(scale * w, gpu))
+    ref = np.array([np.linalg.qr(x)[0] for x in w])
+    assert np.max(np.linalg.cond(w)) < 1e4
+    assert rel(got, ref) < 1e-11
