@@ -322,8 +322,13 @@ __global__ __launch_bounds__(256) void sym_check_kernel(int n, int nt,
     amax = fmax(amax, __shfl_xor(amax, off, 64));
   }
   if ((threadIdx.x & 63) == 0) {
-    if (asym > 0.0) atomicMax(&out[0], (unsigned long long)__double_as_longlong(asym));
-    if (amax > 0.0) atomicMax(&out[1], (unsigned long long)__double_as_longlong(amax));
+    // (a wave below the maximum so far leaves it alone: 10^5 waves share the two words)
+    const double v[2] = {asym, amax};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const auto bits = (unsigned long long)__double_as_longlong(v[i]);
+      if (bits > __atomic_load_n(&out[i], __ATOMIC_RELAXED)) atomicMax(&out[i], bits);
+    }
   }
 }
 

@@ -206,8 +206,8 @@ __device__ __forceinline__ void gj_invert(cplx* B, int ld, int n, GjState* st, i
 // waves per walker (two for n <= 24, four beyond) and the LDS the two-wave kernel's
 // cross-wave overlap reduction needs
 constexpr int meas_waves(int t2) { return t2 <= 3 ? 2 : 4; }
-// waves per SIMD the register budget is compiled for (n > 48 needs more than 256)
-constexpr int meas_wpe(int t2) { return t2 >= 7 ? 1 : 2; }
+// waves per SIMD the register budget is compiled for
+constexpr int meas_wpe(int t2) { return t2 <= 3 ? 2 : t2 == 4 ? 4 : t2 <= 6 ? 3 : 2; }
 constexpr int meas_ti(int t2) { return t2 > 3 ? 1 : (t2 + 1) / 2; }
 constexpr size_t meas_red_bytes(int t2) {
   return t2 <= 3 ? (size_t)meas_ti(t2) * t2 * 4 * 64 * sizeof(double) : 0;
@@ -579,98 +579,237 @@ __device__ __forceinline__ void measure_narrow_body(
   for (int tp = wv; tp < tp_n; tp += NW) tile(tp);
 }
 
-// n > 24: four waves per walker.  They take alternate row tiles of O (each over the
-// whole K = N), share the blocked inversion of O, and take alternate column tiles of the
-// Green's function.
-template <int T2, int TI, bool STAGE>
+// n > 24: four waves per walker; four (n <= 32) or three (n <= 48) walkers share a CU.
+//   - Overlaps: chunks of 16 rows of the walker and of the trial pass through LDS (loaded
+//     once by all waves, two chunks ahead in registers: the walker comes from HBM), and the
+//     tiles of O are dealt to the waves one by one.
+//   - The inversion on all four waves.
+//   - Green's function: X is first laid out in LDS as the A operand, P[k][c] = [Xr | Xi]
+//     through the pivot maps (in place of O), so a k group is one read per row tile without
+//     maps or selections: rows k < n of A are P[k][r], rows n + k are P[k] with its halves
+//     exchanged and the first negated.  One 16-byte load of the walker feeds both.
+// Per walker at norb 200, n = 40 and two walkers per CU, in cycles (MFMA alone in brackets):
+// overlaps 44k (13k), inversion 82k, Green's function 55k (26k); with the operands read as
+// they came (X through both maps for each tile) it was 42k, 83k and 108k.  2048 walkers:
+// 442 -> 330 us; norb 131, n = 29, 777 walkers: 124 -> 85 us; norb 250, n = 50, 512: 310 ->
+// 170 us.
+constexpr int MW_KC = 16;  // rows per chunk of the overlap product
+// doubles per LDS row: 16 T2 columns, == 16 (mod 32), so rows k and k + 1 meet different
+// bank halves
+__host__ __device__ constexpr int mw_ps(int t2) { return 16 * t2 + (t2 % 2 ? 0 : 16); }
+__host__ __device__ constexpr int mw_ts(int t2) {  // of the trial's rows: ceil(n / 16) tiles
+  const int ti = (t2 + 1) / 2;
+  return 16 * ti + (ti % 2 ? 0 : 16);
+}
+// LDS shared in turn by the overlap's chunks (two buffers), O and P
+__host__ __device__ constexpr size_t mw_region(int t2, int n) {
+  const size_t stage = (size_t)2 * MW_KC * (mw_ps(t2) + mw_ts(t2)) * sizeof(double);
+  const size_t o = (size_t)n * gj_ld(n) * sizeof(cplx);
+  const size_t p = (size_t)((n + 3) & ~3) * mw_ps(t2) * sizeof(double);
+  const size_t m = stage > o ? (stage > p ? stage : p) : (o > p ? o : p);
+  return (m + 15) & ~(size_t)15;
+}
+constexpr size_t mw_bytes(int t2, int n) { return mw_region(t2, n) + 256 * sizeof(int); }
+
+template <int T2>
 __device__ __forceinline__ void measure_wide_body(
     int N, int n, const cplx* __restrict__ walkers, const double* __restrict__ trial,
     cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ ghi,
     uint16_t* __restrict__ glo, int ld16, const int w, const WeightsArgs& tail) {
-  constexpr int NW = 4;
+  constexpr int NW = 4, NT = 64 * NW, KC = MW_KC;
+  constexpr int PS = mw_ps(T2), TS = mw_ts(T2);
+  constexpr int TIM = (T2 + 1) / 2;             // row tiles of O at most
+  constexpr int UPW = (TIM * T2 + NW - 1) / NW;  // tiles of O per wave
+  constexpr int NE = (8 * T2 * KC + NT - 1) / NT;  // chunk elements per thread (n <= 8 T2)
   extern __shared__ double smem[];
   const int n2 = 2 * n, ld = gj_ld(n);
-  cplx* M = reinterpret_cast<cplx*>(smem);               // O, then its inverse: n x ld
-  GjState* st = reinterpret_cast<GjState*>(M + n * ld);  // the inversion's state
+  cplx* M = reinterpret_cast<cplx*>(smem);  // O, then its inverse: n x ld
+  GjState* st = reinterpret_cast<GjState*>(reinterpret_cast<char*>(smem) + mw_region(T2, n));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int s = lane >> 4, col = lane & 15;
   const cplx* phi = walkers + (int64_t)w * N * n;
-  // walker operand: staged once into LDS with 16-byte loads (all in flight together)
-  // when it fits, else read from global memory (L2)
-  const double* phid = reinterpret_cast<const double*>(phi);
-  if (STAGE) {
-    cplx* ph = reinterpret_cast<cplx*>(reinterpret_cast<int*>(st) + 256);
-    for (int e = tid; e < N * n; e += 64 * NW) ph[e] = phi[e];
-    phid = reinterpret_cast<const double*>(ph);
+
+  // ---- O = C^T w, [Or | Oi] = C^T [wr | wi] in 16 x 16 tiles, tile u of the wave:
+  // number wv + 4 u, row-major over ceil(n / 16) x T2
+  const int tiles = ((n + 15) >> 4) * T2;
+  {
+    double* sb = smem;                 // [2][KC][PS]: [wr | wi]
+    double* sa = smem + 2 * KC * PS;   // [2][KC][TS]: C
+    // two sets: a chunk's loads are issued two chunks ahead of its products
+    cplx rw0[NE], rw1[NE];
+    double rt0[NE], rt1[NE];
+    int ow[NE], ot[NE];  // LDS offsets of the thread's elements of a chunk
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int e = tid + NT * i, r = e / n, j = e - r * n;
+      ow[i] = r * PS + j;
+      ot[i] = r * TS + j;
+    }
+    // a chunk is contiguous in both arrays; past the last row: any entry, zeros of C
+    auto load = [&](cplx (&rw)[NE], double (&rt)[NE], int p0) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) {
+        const int e = min(p0 * n + tid + NT * i, N * n - 1);
+        rw[i] = phi[e];
+        rt[i] = trial[e];
+      }
+    };
+    auto store = [&](const cplx (&rw)[NE], const double (&rt)[NE], int buf, int p0) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) {
+        const int e = tid + NT * i;
+        if (e >= KC * n) continue;
+        double* b = sb + buf * KC * PS + ow[i];
+        b[0] = rw[i].re;
+        b[n] = rw[i].im;
+        sa[buf * KC * TS + ot[i]] = p0 * n + e < N * n ? rt[i] : 0.0;
+      }
+    };
+    int aoff[UPW], boff[UPW];
+    double4_t acc[UPW];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+      const int t = min(wv + NW * u, tiles - 1), ti = t / T2;
+      aoff[u] = s * TS + ti * 16 + col;  // (rows i >= n and columns c >= 2n are not stored)
+      boff[u] = s * PS + (t - ti * T2) * 16 + col;
+      acc[u] = double4_t{0.0, 0.0, 0.0, 0.0};
+    }
+    const int nch = (N + KC - 1) / KC;
+    auto product = [&](int buf) {
+#pragma unroll
+      for (int kg = 0; kg < KC / 4; ++kg)
+#pragma unroll
+        for (int u = 0; u < UPW; ++u) {
+          if (wv + NW * u >= tiles) continue;  // (uniform)
+          acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(sa[(buf * KC + 4 * kg) * TS + aoff[u]],
+                                                        sb[(buf * KC + 4 * kg) * PS + boff[u]],
+                                                        acc[u], 0, 0, 0);
+        }
+    };
+    load(rw0, rt0, 0);
+    load(rw1, rt1, KC);
+    store(rw0, rt0, 0, 0);
+    lds_barrier();
+    for (int ch = 0; ch < nch; ch += 2) {
+      load(rw0, rt0, (ch + 2) * KC);
+      product(0);
+      store(rw1, rt1, 1, (ch + 1) * KC);
+      lds_barrier();
+      if (ch + 1 >= nch) break;
+      load(rw1, rt1, (ch + 3) * KC);
+      product(1);
+      store(rw0, rt0, 0, (ch + 2) * KC);
+      lds_barrier();
+    }
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+      const int t = wv + NW * u, ti = t / T2, c = (t - ti * T2) * 16 + col;
+      if (t >= tiles || c >= n2) continue;
+      const int cj = c < n ? c : c - n, ci = c < n ? 0 : 1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = ti * 16 + s + 4 * r;
+        if (row < n) reinterpret_cast<double*>(&M[row * ld + cj])[ci] = acc[u][r];
+      }
+    }
   }
-  __syncthreads();
-  // row tiles of O, one per wave in turn
-  const int ti_total = (n + 15) >> 4;
-  for (int tb = wv; tb < ti_total; tb += NW)
-    overlap_tiles<T2, 1, 1>(N, n, tb, trial, phid, M, ld, nullptr, false, lane, 0);
 
   // ---- O^-1 and det(O): blocked in-place Gauss-Jordan on all four waves
-  gj_invert<NW, 4>(M, ld, n, st, lane, wv);
+  gj_invert<NW, TIM>(M, ld, n, st, lane, wv);
   const cplx det = st->det;
-  if (tid == 0) finish_walker(det, dets, w, spin, tail);
-  if (!(green || ghi)) return;
+  if (!(green || ghi)) {
+    if (tid == 0) finish_walker(det, dets, w, spin, tail);
+    return;
+  }
 
-  // ---- [Gr ; Gi] = [[Xr^T, -Xi^T], [Xi^T, Xr^T]] [wr^T ; wi^T], K = 2n, columns p
+  // ---- P from X (through registers: P takes the place of M), zero rows up to a k group
+  double* P = smem;
+  {
+    constexpr int NX = T2 * T2 / 4 + (T2 * T2 % 4 ? 1 : 0);  // n^2 / 256 at most
+    cplx x[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = min(tid + NT * i, n * n - 1), k = e / n, r = e - k * n;
+      x[i] = M[st->rho[k] * ld + st->rhoinv[r]];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = tid + NT * i, k = e / n, r = e - k * n;
+      if (e >= n * n) continue;
+      P[k * PS + r] = x[i].re;
+      P[k * PS + n + r] = x[i].im;
+    }
+    for (int e = tid; e < (((n + 3) & ~3) - n) * PS; e += NT) P[n * PS + e] = 0.0;
+    lds_barrier();
+  }
+
+  // (past the last barrier: only this wave waits for it)
+  if (tid == NT - 64) finish_walker(det, dets, w, spin, tail);
+
+  // ---- [Gr ; Gi] = [[Xr^T, -Xi^T], [Xi^T, Xr^T]] [wr^T ; wi^T], K = 2n, columns p; the
+  // waves take alternate column tiles
   double* gw = green ? green + (int64_t)w * n2 * N : nullptr;
   uint16_t* gh = ghi ? ghi + (int64_t)w * n2 * ld16 : nullptr;
   uint16_t* gl = ghi ? glo + (int64_t)w * n2 * ld16 : nullptr;
-  const int tp_n = (N + 15) >> 4;
-    const int nkg = (n2 + 3) >> 2;
-    // columns of X in the lane's A rows r = tr * 16 + col (pivot map, clamped index:
-    // rows r >= 2n are not stored)
-    int xcol[T2];
+  const int tp_n = (N + 15) >> 4, nkg = (n + 3) >> 2;
+  const double* P0 = P + s * PS + col;  // + 16 tr: row k < n of A
+  const double* P1[T2];                 // row n + k of A, before its sign
+  unsigned sgn[T2];
 #pragma unroll
-    for (int tr = 0; tr < T2; ++tr) {
-      const int r = tr * 16 + col;
-      xcol[tr] = st->rhoinv[min(r < n ? r : r - n, n - 1)];
-    }
-    for (int tp = wv; tp < tp_n; tp += NW) {
-      const int p = tp * 16 + col;  // B column = orbital p
-      const int pc = min(p, N - 1);   // (columns p >= N are not stored)
-      double4_t acc[T2];
+  for (int tr = 0; tr < T2; ++tr) {
+    const int r = tr * 16 + col;
+    P1[tr] = P + s * PS + (r < n ? r + n : min(r - n, n - 1));
+    sgn[tr] = r < n ? 0x80000000u : 0u;
+  }
+  auto flip = [](double v, unsigned m) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    return __longlong_as_double((long long)(u ^ ((unsigned long long)m << 32)));
+  };
+  auto load_w = [&](int tp, int kg) {
+    return phi[min(tp * 16 + col, N - 1) * n + min(4 * kg + s, n - 1)];
+  };
+  constexpr int PD = 2;  // k groups of the walker in flight
+  cplx b[PD];
 #pragma unroll
-      for (int tr = 0; tr < T2; ++tr) acc[tr] = double4_t{0.0, 0.0, 0.0, 0.0};
-      for (int kg0 = 0; kg0 < nkg; kg0 += MEAS_KC) {
-        // loads from clamped indices, unconditional; A is zero for k >= 2n
-        double a[MEAS_KC][T2], b[MEAS_KC];
+  for (int u = 0; u < PD; ++u) b[u] = load_w(wv, u);  // (clamped: valid past the last group)
+  for (int tp = wv; tp < tp_n; tp += NW) {
+    double4_t acc[T2];
 #pragma unroll
-        for (int u = 0; u < MEAS_KC; ++u) {
-          const int k = 4 * (kg0 + u) + s;
-          const int kj = min(k < n ? k : k - n, n - 1);
-          b[u] = phid[2 * ((int64_t)pc * n + kj) + (k < n ? 0 : 1)];
-          const int xr = st->rho[kj] * ld;
+    for (int tr = 0; tr < T2; ++tr) acc[tr] = double4_t{0.0, 0.0, 0.0, 0.0};
+    for (int kg0 = 0; kg0 < nkg; kg0 += PD) {
 #pragma unroll
-          for (int tr = 0; tr < T2; ++tr) {
-            const int r = tr * 16 + col;  // A row
-            const cplx x = M[xr + xcol[tr]];  // X[kj][ri]
-            // (r < n, k < n): Xr; (r < n, k >= n): -Xi; (r >= n, k < n): Xi; else Xr
-            const double v = (r < n) == (k < n) ? x.re : ((r < n) ? -x.im : x.im);
-            a[u][tr] = __builtin_unpredictable(k < n2) ? v : 0.0;
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < MEAS_KC; ++u)
+      for (int u = 0; u < PD; ++u) {
+        const int kg = kg0 + u;
+        if (kg < nkg) {  // (uniform)
+          const double* p0 = P0 + kg * 4 * PS;
 #pragma unroll
           for (int tr = 0; tr < T2; ++tr)
-            acc[tr] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][tr], b[u], acc[tr], 0, 0, 0);
-      }
+            acc[tr] = __builtin_amdgcn_mfma_f64_16x16x4f64(p0[tr * 16], b[u].re, acc[tr], 0, 0, 0);
 #pragma unroll
-      for (int tr = 0; tr < T2; ++tr)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int row = tr * 16 + s + 4 * q;
-          if (row < n2 && p < N) {
-            if (gw) gw[(int64_t)row * N + p] = acc[tr][q];
-            if (gh) split_bf16(acc[tr][q], &gh[(int64_t)row * ld16 + p], &gl[(int64_t)row * ld16 + p]);
-          }
+          for (int tr = 0; tr < T2; ++tr)
+            acc[tr] = __builtin_amdgcn_mfma_f64_16x16x4f64(flip(P1[tr][kg * 4 * PS], sgn[tr]),
+                                                           b[u].im, acc[tr], 0, 0, 0);
         }
+        // the group PD ahead, of the next tile past this one's end
+        const bool more = kg0 + PD < nkg;
+        b[u] = load_w(more ? tp : tp + NW, more ? kg + PD : u);
+      }
     }
+    const int p = tp * 16 + col;
+    if (p >= N) continue;
+#pragma unroll
+    for (int tr = 0; tr < T2; ++tr)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = tr * 16 + s + 4 * q;
+        if (row < n2) {
+          if (gw) gw[(int64_t)row * N + p] = acc[tr][q];
+          if (gh) split_bf16(acc[tr][q], &gh[(int64_t)row * ld16 + p], &gl[(int64_t)row * ld16 + p]);
+        }
+      }
+  }
 }
 
 template <int T2, int TI, int STAGE>
@@ -682,8 +821,8 @@ __global__ __launch_bounds__(64 * meas_waves(T2), meas_wpe(T2)) void measure_ker
     measure_narrow_body<T2, STAGE>(N, n, walkers, trial, dets, spin, green, ghi, glo, ld16,
                                    blockIdx.x, tail);
   else
-    measure_wide_body<T2, TI, STAGE != 0>(N, n, walkers, trial, dets, spin, green, ghi, glo,
-                                          ld16, blockIdx.x, tail);
+    measure_wide_body<T2>(N, n, walkers, trial, dets, spin, green, ghi, glo, ld16, blockIdx.x,
+                          tail);
 }
 
 template <int T2, int TI, int STAGE>
@@ -697,9 +836,8 @@ __global__ __launch_bounds__(64 * meas_waves(T2), meas_wpe(T2)) void measure_gro
     measure_narrow_body<T2, STAGE>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin, a.green,
                                    a.ghi, a.glo, a.ld16, blockIdx.x - start[p], none);
   else
-    measure_wide_body<T2, TI, STAGE != 0>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin,
-                                          a.green, a.ghi, a.glo, a.ld16, blockIdx.x - start[p],
-                                          none);
+    measure_wide_body<T2>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin, a.green, a.ghi, a.glo,
+                          a.ld16, blockIdx.x - start[p], none);
 }
 
 template <int T2, int STAGE>
@@ -719,9 +857,10 @@ int launch_measure_grouped_s(hipStream_t st, const MeasureArgs* args, const int*
 template <int T2>
 int launch_measure_grouped_t(hipStream_t st, int stage, const MeasureArgs* args,
                              const int* start, int nprob, int nblocks, size_t shm) {
-  if constexpr (T2 <= 3)
+  if constexpr (T2 <= 3) {
     if (stage == 2) return launch_measure_grouped_s<T2, 2>(st, args, start, nprob, nblocks, shm);
-  if (stage != 0) return launch_measure_grouped_s<T2, 1>(st, args, start, nprob, nblocks, shm);
+    if (stage == 1) return launch_measure_grouped_s<T2, 1>(st, args, start, nprob, nblocks, shm);
+  }
   return launch_measure_grouped_s<T2, 0>(st, args, start, nprob, nblocks, shm);
 }
 
@@ -746,9 +885,10 @@ int launch_measure_t(afqmc_ctx* c, int W, int n, const cplx* wk, int s, bool g64
   int t2, stage;
   size_t shm;
   measure_plan(c, s, &t2, &stage, &shm);
-  if constexpr (T2 <= 3)
+  if constexpr (T2 <= 3) {
     if (stage == 2) return launch_measure_s<T2, 2>(c, W, n, wk, s, g64, gbf, tail, shm);
-  if (stage != 0) return launch_measure_s<T2, 1>(c, W, n, wk, s, g64, gbf, tail, shm);
+    if (stage == 1) return launch_measure_s<T2, 1>(c, W, n, wk, s, g64, gbf, tail, shm);
+  }
   return launch_measure_s<T2, 0>(c, W, n, wk, s, g64, gbf, tail, shm);
 }
 
@@ -815,7 +955,6 @@ void measure_plan(const afqmc_ctx* c, int s, int* t2, int* stage, size_t* shm) {
     }
     return;
   }
-  const size_t base = gj_bytes(n);
-  *stage = base + walker <= 24 * 1024 ? 1 : 0;  // small walkers only: staging costs occupancy
-  *shm = *stage ? base + walker : base;
+  *stage = 0;
+  *shm = mw_bytes(*t2, n);
 }

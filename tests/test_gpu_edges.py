@@ -23,6 +23,8 @@ CASES = [
     ("rhf", 33, (5, 5), 131, 70),
     ("uhf", 65, (9, 8), 71, 33),
     ("rhf", 115, (9, 9), 37, 260),  # 128-wide GEMM tiles, partly filled
+    ("uhf", 49, (33, 25), 9, 4),    # four-wave measurement, edges of its tile counts
+    ("uhf", 66, (64, 49), 7, 3),
 ]
 
 
