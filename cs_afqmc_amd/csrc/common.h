@@ -494,15 +494,6 @@ struct FinishArgs {
   double h0;
   cplx* energies;
 };
-// exchange kernel variants (launch_exchange_grouped)
-enum ExchKind {
-  EXCH_BF16X3_WN2 = 0,
-  EXCH_BF16X3_WN4 = 1,
-  EXCH_F64_V1 = 2,
-  EXCH_F64_V2 = 3,
-  EXCH_F32_V1 = 4,
-  EXCH_F32_V2 = 5
-};
 // the exchange launch of context c, spin s, over W walkers (xpart: c's partial sums of
 // that spin), and the finishing launch's arguments; used by the single and grouped forms
 void exchange_plan(const afqmc_ctx* c, int s, int W, ExchArgs* a, int* kind, int* nblocks);

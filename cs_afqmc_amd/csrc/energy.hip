@@ -54,159 +54,164 @@ inline int exchange_chunk(int g_tiles, int64_t tile_bytes) {
 
 // ---------------------------------------------------------------- fused exchange
 
-// Exchange sums of the (g, w) blocks of an F tile held in LDS (row stride ldf):
-// F row gl*n + i, column wl*2n + c*n + j.  x_w = sum_g sum_ij f(i,j) f(j,i) is taken over
-// the pairs i <= j (weight 2 off the diagonal): each lane owns pairs and runs down the
-// tile's g.  With at least as many walkers as waves each wave takes walkers wl = v, v+NWV,
-// ...; with fewer, the waves split each walker's g range and their partial sums (parts,
-// one entry per wave in LDS) are added in wave order.  Results go to xpart[w].
-template <typename T, int NT = ENER_NT>
-__device__ inline void exchange_tile(const T* __restrict__ Fs, int ldf, int n, int g_used,
-                                     int w_used, int w0, cplx* __restrict__ xpart,
-                                     cplx* parts) {
-  constexpr int NWV = NT / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Exchange sums of a workgroup's F tile: F row gl*n + i, column wl*2n + c*n + j, and
+// x_w = sum_g sum_ij f(i,j) f(j,i), taken over the pairs i <= j (weight 2 off the
+// diagonal).  The tile goes through LDS in passes of as many whole g as fit EX_FR rows
+// (write(r0, rows) stores rows r0 .. r0 + rows - 1 to Fs), so the operand buffers' LDS
+// serves it and two or three workgroups share a CU: one reduces while the others multiply.
+// Within a pass every thread takes (g, pair) items and runs over the walkers with their
+// four loads all in flight; its sums stay in registers over the passes, EX_MAXW walkers at
+// a time (tiles of more walkers, n <= 7, add up per pass instead).  Sums over threads: wave
+// tree, then the waves in order.
+constexpr int EX_NT = 256, EX_FR = 64, EX_MAXW = 8;
+// partial sums of 4 waves x up to 64 walkers
+constexpr int EX_PARTS_BYTES = 4 * 64 * 16;
+
+template <typename T, typename WriteF>
+__device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_used, int w_used,
+                                                int w0, cplx* __restrict__ xpart, cplx* parts,
+                                                WriteF write) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int npairs = n * (n + 1) / 2;
-  const int gstride = n * ldf;
-  const int wpw = w_used >= NWV ? 1 : NWV / w_used;  // waves per walker
-  const int items = w_used * wpw;
-  const int gc = (g_used + wpw - 1) / wpw;
-  for (int it = wave; it < items; it += NWV) {
-    const int wl = it / wpw, part = it - wl * wpw;
-    const int gb = part * gc, ge = min(g_used, gb + gc);
-    const T* base = Fs + wl * 2 * n + gb * gstride;
-    double xr = 0.0, xi = 0.0;
-    for (int t = lane; t < npairs; t += 64) {
-      // pair t = a (a + 1) / 2 + b, b <= a: (i, j) = (b, a)
-      int a = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
-      if (a * (a + 1) / 2 > t) --a;
-      if ((a + 1) * (a + 2) / 2 <= t) ++a;
-      const int i = t - a * (a + 1) / 2, j = a;
-      const double wgt = i == j ? 1.0 : 2.0;
-      const T* pa = base + i * ldf + j;  // f(i, j): re pa[0], im pa[n]
-      const T* pb = base + j * ldf + i;  // f(j, i)
-      double sr = 0.0, si = 0.0;
-      for (int gl = gb; gl < ge; ++gl) {
-        const double ar = (double)pa[0], ai = (double)pa[n];
-        const double br = (double)pb[0], bi = (double)pb[n];
-        sr += ar * br - ai * bi;
-        si += ar * bi + ai * br;
-        pa += gstride;
-        pb += gstride;
+  const int gpp = EX_FR / n;  // g per pass
+  const bool persist = w_used <= EX_MAXW;
+  double xr[EX_MAXW], xi[EX_MAXW];
+#pragma unroll
+  for (int k = 0; k < EX_MAXW; ++k) xr[k] = xi[k] = 0.0;
+  for (int g0 = 0; g0 < g_used; g0 += gpp) {
+    const int gn = min(gpp, g_used - g0);
+    __syncthreads();  // the operands, or the last pass, are no longer read
+    write(g0 * n, gn * n);
+    __syncthreads();
+    const bool last = g0 + gpp >= g_used;
+    for (int wb = 0; wb < w_used; wb += EX_MAXW) {
+      if (!persist) {
+#pragma unroll
+        for (int k = 0; k < EX_MAXW; ++k) xr[k] = xi[k] = 0.0;
       }
-      xr += wgt * sr;
-      xi += wgt * si;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      xr += __shfl_down(xr, off, 64);
-      xi += __shfl_down(xi, off, 64);
-    }
-    if (lane == 0) {
-      if (wpw == 1)
-        xpart[w0 + wl] = cplx{xr, xi};
-      else
-        parts[it] = cplx{xr, xi};
+      for (int it = t; it < gn * npairs; it += EX_NT) {
+        const int gl = it / npairs, q = it - gl * npairs;
+        // pair q = a (a + 1) / 2 + b, b <= a: (i, j) = (b, a)
+        int a = (int)((sqrtf(8.0f * (float)q + 1.0f) - 1.0f) * 0.5f);
+        if (a * (a + 1) / 2 > q) --a;
+        if ((a + 1) * (a + 2) / 2 <= q) ++a;
+        const int i = q - a * (a + 1) / 2, j = a;
+        const T wgt = i == j ? (T)1 : (T)2;
+        const T* pa = Fs + (gl * n + i) * ldf + wb * 2 * n + j;  // f(i, j): re pa[0], im pa[n]
+        const T* pb = Fs + (gl * n + j) * ldf + wb * 2 * n + i;  // f(j, i)
+#pragma unroll
+        for (int k = 0; k < EX_MAXW; ++k)
+          if (wb + k < w_used) {
+            const double ar = (double)(wgt * pa[k * 2 * n]), ai = (double)(wgt * pa[k * 2 * n + n]);
+            const double br = (double)pb[k * 2 * n], bi = (double)pb[k * 2 * n + n];
+            xr[k] += ar * br - ai * bi;
+            xi[k] += ar * bi + ai * br;
+          }
+      }
+      if (!persist || last) {
+#pragma unroll
+        for (int k = 0; k < EX_MAXW; ++k)
+          if (wb + k < w_used) {
+            double vr = xr[k], vi = xi[k];
+            for (int off = 32; off > 0; off >>= 1) {
+              vr += __shfl_down(vr, off, 64);
+              vi += __shfl_down(vi, off, 64);
+            }
+            if (lane == 0) {
+              cplx* p = parts + wave * 64 + wb + k;
+              *p = g0 == 0 || persist ? cplx{vr, vi} : cplx{p->re + vr, p->im + vi};
+            }
+          }
+      }
     }
   }
-  if (wpw > 1) {  // (uniform in the workgroup)
-    __syncthreads();
-    if (threadIdx.x < w_used) {
-      double xr = 0.0, xi = 0.0;
-      for (int q = 0; q < wpw; ++q) {
-        xr += parts[threadIdx.x * wpw + q].re;
-        xi += parts[threadIdx.x * wpw + q].im;
-      }
-      xpart[w0 + threadIdx.x] = cplx{xr, xi};
-    }
+  __syncthreads();
+  if (t < w_used) {
+    cplx x = parts[t];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) x = cadd(x, parts[v * 64 + t]);
+    xpart[w0 + t] = x;
   }
 }
 
-// float64 MFMA tile 64 x 128 (4 waves as 2 x 2, each 32 x 64), BK = 16, operands k-major
-// in LDS, double buffered.  With F32 (the FP32 precision mode) the same tile runs on
+// float64 MFMA tile BM x 16 TN (four waves, BM / 4 rows each), BK = 16, operands row-major
+// in LDS as 16-byte chunks, double buffered, loaded 16 bytes at a time without conditions
+// (rows past the operands read the last row, their products belong to no (g, w) block; k
+// past N is zeroed as the registers go to LDS).  A lane's chunk feeds two float64 MFMAs or
+// four float32 ones.  With F32 (the FP32 precision mode) the same tile runs on
 // v_mfma_f32_16x16x4f32: operands rounded to float32 as they are staged, float32
 // accumulation and F tile (its D rows are 4 (l / 16) + r instead of l / 16 + 4 r); the
 // exchange sums still accumulate in float64.
-constexpr int EF_BM = 64, EF_BN = 128, EF_BK = 16, EF_PAD = 16;
-// Element (k, m) of a k-major operand tile sits at column m ^ ef_swz<F32, VEC>(k): the
-// MFMA operand reads see the same banks as without it, and the staging stores (lanes
-// along k) meet distinct banks instead of 8 (float64) or 4 (float32) k rows on one
-template <bool F32, int VEC>
-__device__ inline int ef_swz(int k) {
-  if constexpr (F32) return ((k >> 2) & 3) << (VEC == 2 ? 3 : 2);
-  return ((k >> 1) & 7) << (VEC == 2 ? 2 : 1);
-}
-constexpr int EF_LDF = 129;  // F tile row stride (odd: transposed reads spread over banks)
-constexpr int EF_OPS_BYTES = 2 * EF_BK * (EF_BM + EF_PAD) * 8 + 2 * EF_BK * (EF_BN + EF_PAD) * 8;
-constexpr int EF_F_BYTES = EF_BM * EF_LDF * 8;
-constexpr int EF_F_PARTS = EF_F_BYTES + (ENER_NT / 64) * 16;
-constexpr int EF_LDS = EF_OPS_BYTES > EF_F_PARTS ? EF_OPS_BYTES : EF_F_PARTS;
+constexpr int EF_BK = 16;
+typedef double ef_d2u_t __attribute__((ext_vector_type(2), aligned(8)));
+typedef double ef_d2_t __attribute__((ext_vector_type(2)));
+typedef float ef_f2_t __attribute__((ext_vector_type(2)));
+typedef float ef_f4_t __attribute__((ext_vector_type(4)));
 
-template <int VEC, bool F32>
-__device__ __forceinline__ void exchange_f64_body(
-    int G, int n, int N, int W, int gpt, int wpt, int g_tiles, int gc,
-    const double* __restrict__ A, const double* __restrict__ B, cplx* __restrict__ xpart,
-    const int bx) {
+template <bool F32, int BM, int TN>
+struct EfTile {
   typedef typename std::conditional<F32, float, double>::type T;
-  typedef typename std::conditional<F32, float4_t, double4_t>::type AccT;
-  constexpr int BM = EF_BM, BN = EF_BN, BK = EF_BK;
-  constexpr int TM = BM / 2 / 16, TN = BN / 2 / 16;
-  constexpr int KT = BK / VEC, RSTEP = ENER_NT / KT, A_LD = BM / RSTEP, B_LD = BN / RSTEP;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[EF_LDS];
-  typedef T AsT[BK][BM + EF_PAD];
-  typedef T BsT[BK][BN + EF_PAD];
-  AsT* As = reinterpret_cast<AsT*>(lds);
-  BsT* Bs = reinterpret_cast<BsT*>(lds + 2 * sizeof(AsT));
-  T* Fs = reinterpret_cast<T*>(lds);
+  static constexpr int BN = 16 * TN, BNP = (BN + 31) / 32 * 32;  // staged B rows
+  static constexpr int LDF = BN + 1;  // odd: transposed reads spread over the banks
+  static constexpr int OPS = 2 * (BM + BNP) * EF_BK * (int)sizeof(T);
+  static constexpr int F = (EX_FR * LDF * (int)sizeof(T) + 15) / 16 * 16;
+  static constexpr int BODY = OPS > F ? OPS : F;
+  static constexpr int LDS = BODY + EX_PARTS_BYTES;
+};
 
+template <bool F32, int BM, int TN>
+__device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int bx) {
+  typedef EfTile<F32, BM, TN> Tile;
+  typedef typename Tile::T T;
+  typedef typename std::conditional<F32, float4_t, double4_t>::type AccT;
+  typedef typename std::conditional<F32, ef_f4_t, ef_d2_t>::type ChunkT;  // 16 bytes
+  constexpr int TM = BM / 64, BK = EF_BK;
+  constexpr int RCH = F32 ? 4 : 8;  // chunks per row
+  constexpr int A_LD = BM / 32, B_LD = Tile::BNP / 32;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[Tile::LDS];
+  constexpr int BUF = (BM + Tile::BNP) * RCH;
+  ChunkT* ops = reinterpret_cast<ChunkT*>(lds);
+
+  const int n = x.n, N = x.K;
   int gt, wt;
-  exchange_tile_of(bx, g_tiles, (W + wpt - 1) / wpt, gc, &gt, &wt);
-  const int g0 = gt * gpt, w0 = wt * wpt;
-  const int M = G * n, NB = 2 * W * n;
+  exchange_tile_of(bx, x.g_tiles, (x.W + x.wpt - 1) / x.wpt, x.gc, &gt, &wt);
+  const int g0 = gt * x.gpt, w0 = wt * x.wpt;
   const int m0 = g0 * n, n0 = w0 * 2 * n;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int lk = (t % KT) * VEC, lr = t / KT;
-
-  T ra[A_LD][VEC], rb[B_LD][VEC];
+  const int lch = t & 7, lr = t >> 3;
+  const double* Ab = static_cast<const double*>(x.A) + (int64_t)m0 * N;
+  const double* Bb = static_cast<const double*>(x.B) + (int64_t)n0 * N;
+  int aoff[A_LD], boff[B_LD];
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) aoff[i] = min(lr + i * 32, x.G * n - 1 - m0) * N;
+#pragma unroll
+  for (int i = 0; i < B_LD; ++i) boff[i] = min(lr + i * 32, 2 * x.W * n - 1 - n0) * N;
+  ef_d2_t ra[A_LD], rb[B_LD];
+  // chunks past N read elements N - 1 and N (the operands' allocations end with at least
+  // one element of padding)
   auto load_tile = [&](int k0) {
-    const int k = k0 + lk;
-    const bool kok = k < N;  // VEC == 2 needs N even (checked at launch)
+    const int k = min(k0 + 2 * lch, N - 1);
 #pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      const int r = m0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < M && kok) v = *reinterpret_cast<const double2*>(A + (int64_t)r * N + k);
-        ra[i][0] = (T)v.x;
-        ra[i][VEC - 1] = (T)v.y;
-      } else {
-        ra[i][0] = (r < M && kok) ? (T)A[(int64_t)r * N + k] : (T)0;
-      }
-    }
+    for (int i = 0; i < A_LD; ++i) ra[i] = *reinterpret_cast<const ef_d2u_t*>(Ab + (aoff[i] + k));
 #pragma unroll
-    for (int i = 0; i < B_LD; ++i) {
-      const int r = n0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < NB && kok) v = *reinterpret_cast<const double2*>(B + (int64_t)r * N + k);
-        rb[i][0] = (T)v.x;
-        rb[i][VEC - 1] = (T)v.y;
-      } else {
-        rb[i][0] = (r < NB && kok) ? (T)B[(int64_t)r * N + k] : (T)0;
-      }
-    }
+    for (int i = 0; i < B_LD; ++i) rb[i] = *reinterpret_cast<const ef_d2u_t*>(Bb + (boff[i] + k));
   };
-  auto store_tile = [&](int buf) {
+  auto store_tile = [&](int buf, int k0) {
+    const bool ok0 = k0 + 2 * lch < N, ok1 = k0 + 2 * lch + 1 < N;
+    auto put = [&](int row, ef_d2_t v) {  // (32-row steps leave the swizzle unchanged)
+      if constexpr (F32) {
+        const int c = (lch >> 1) ^ ((lr >> 1) & 3);
+        reinterpret_cast<ef_f2_t*>(ops + buf * BUF + row * RCH)[c * 2 + (lch & 1)] =
+            ef_f2_t{ok0 ? (float)v.x : 0.f, ok1 ? (float)v.y : 0.f};
+      } else {
+        ops[buf * BUF + row * RCH + (lch ^ ((lr >> 1) & 7))] =
+            ef_d2_t{ok0 ? v.x : 0.0, ok1 ? v.y : 0.0};
+      }
+    };
 #pragma unroll
-    for (int i = 0; i < A_LD; ++i)
+    for (int i = 0; i < A_LD; ++i) put(lr + i * 32, ra[i]);
 #pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        As[buf][lk + v][(lr + i * RSTEP) ^ ef_swz<F32, VEC>(lk + v)] = ra[i][v];
-#pragma unroll
-    for (int i = 0; i < B_LD; ++i)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        Bs[buf][lk + v][(lr + i * RSTEP) ^ ef_swz<F32, VEC>(lk + v)] = rb[i][v];
+    for (int i = 0; i < B_LD; ++i) put(BM + lr + i * 32, rb[i]);
   };
 
   AccT acc[TM][TN];
@@ -215,160 +220,116 @@ __device__ __forceinline__ void exchange_f64_body(
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = AccT{0, 0, 0, 0};
 
-  const int nk = (N + BK - 1) / BK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  const int am = wm * (BM / 2) + (lane & 15);
-  const int bn = wn * (BN / 2) + (lane & 15);
+  const int am = wave * (BM / 4) + (lane & 15), bn = BM + (lane & 15);
   const int kq = lane >> 4;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) load_tile((kt + 1) * BK);
+  // one LDS chunk per lane and operand row: 8 (float64) or 16 (float32) k
+  auto compute = [&](int cur, int ks) {
+    const int co = F32 ? kq ^ ((lane >> 1) & 3) : (ks * 4 + kq) ^ ((lane >> 1) & 7);
+    ChunkT af[TM], bf[TN];
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      T af[TM], bf[TN];
-      const int sw = ef_swz<F32, VEC>(ks * 4 + kq);
+    for (int i = 0; i < TM; ++i) af[i] = ops[cur * BUF + (am + i * 16) * RCH + co];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = As[cur][ks * 4 + kq][(am + i * 16) ^ sw];
+    for (int j = 0; j < TN; ++j) bf[j] = ops[cur * BUF + (bn + j * 16) * RCH + co];
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = Bs[cur][ks * 4 + kq][(bn + j * 16) ^ sw];
+    for (int e = 0; e < (F32 ? 4 : 2); ++e)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           if constexpr (F32)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][e], bf[j][e], acc[i][j], 0, 0, 0);
           else
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][e], bf[j][e], acc[i][j], 0, 0, 0);
         }
-    }
-    if (kt + 1 < nk) store_tile(cur ^ 1);
+  };
+  const int nk = (N + BK - 1) / BK;
+  load_tile(0);
+  store_tile(0, 0);
+  __syncthreads();
+  for (int kt = 0; kt + 1 < nk; ++kt) {
+    const int cur = kt & 1;
+    load_tile((kt + 1) * BK);
+    compute(cur, 0);
+    if (!F32) compute(cur, 1);
+    store_tile(cur ^ 1, (kt + 1) * BK);
     __syncthreads();
   }
-  // F tile -> LDS (the operand buffers are dead after the last barrier)
+  compute((nk - 1) & 1, 0);
+  if (!F32 && N - (nk - 1) * BK > 8) compute((nk - 1) & 1, 1);
+
+  T* Fs = reinterpret_cast<T*>(lds);
+  auto write = [&](int r0, int rows) {
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = wn * (BN / 2) + j * 16 + (lane & 15);
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wm * (BM / 2) + i * 16 + (F32 ? 4 * (lane >> 4) + r : (lane >> 4) + 4 * r);
-        Fs[row * EF_LDF + col] = acc[i][j][r];
+        const int row = wave * (BM / 4) + i * 16 + (F32 ? 4 * kq + r : kq + 4 * r) - r0;
+        if ((unsigned)row < (unsigned)rows) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            Fs[row * Tile::LDF + j * 16 + (lane & 15)] = acc[i][j][r];
+        }
       }
-    }
-  __syncthreads();
-  const int g_used = (G - g0 < gpt) ? G - g0 : gpt;
-  const int w_used = (W - w0 < wpt) ? W - w0 : wpt;
-  exchange_tile<T>(Fs, EF_LDF, n, g_used, w_used, w0, xpart + (int64_t)gt * W,
-                   reinterpret_cast<cplx*>(lds + EF_F_BYTES));
+  };
+  exchange_reduce<T>(Fs, Tile::LDF, n, min(x.gpt, x.G - g0), min(x.wpt, x.W - w0), w0,
+                     x.xpart + (int64_t)gt * x.W, reinterpret_cast<cplx*>(lds + Tile::BODY),
+                     write);
 }
 
-template <int VEC, bool F32>
-__global__ __launch_bounds__(ENER_NT) void exchange_f64_kernel(
-    int G, int n, int N, int W, int gpt, int wpt, int g_tiles, int gc,
-    const double* __restrict__ A, const double* __restrict__ B, cplx* __restrict__ xpart) {
-  exchange_f64_body<VEC, F32>(G, n, N, W, gpt, wpt, g_tiles, gc, A, B, xpart, blockIdx.x);
-}
-
-template <int VEC, bool F32>
-__global__ __launch_bounds__(ENER_NT) void exchange_f64_grouped_kernel(
-    const ExchArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
-  const int p = group_of(start, nprob, blockIdx.x);
-  const ExchArgs a = args[p];
-  exchange_f64_body<VEC, F32>(a.G, a.n, a.K, a.W, a.gpt, a.wpt, a.g_tiles, a.gc,
-                              static_cast<const double*>(a.A), static_cast<const double*>(a.B),
-                              a.xpart, blockIdx.x - start[p]);
-}
-
-// split-bf16 tile 128 x 64 WN on v_mfma_f32_16x16x32_bf16 (2 x WN waves, each 64 x 64),
-// BK = 32; operand planes have K = Np32 (zero padded), so there is no k tail.  WN = 2
-// (128 columns, 4 waves) or, where it holds more whole walkers (2n columns each) per
-// tile, WN = 4 (256 columns, 8 waves): the Cholesky tile is then read once per more
-// walkers.
-// operand rows of 32 bf16 (64 B) with the chunk order c ^ ((r >> 1) & 3), as in the
-// split-bf16 GEMM, under which the 16-row operand reads meet no LDS bank conflicts
-constexpr int EB_BM = 128, EB_BK = 32, EB_LDSW = EB_BK;
-__device__ inline int eb_chunk(int r, int c) { return (c ^ ((r >> 1) & 3)) << 3; }
-template <int WN>
+// split-bf16 tile 128 x 32 TN on v_mfma_f32_16x16x32_bf16 (2 x 2 waves, each 64 x 16 TN),
+// BK = 32; operand planes have K = Np32 (zero padded), so there is no k tail.  The operands
+// go from memory straight to LDS (16 bytes a lane, 16 rows an instruction), single
+// buffered: two or three workgroups share a CU, and one loads or reduces while the others
+// multiply.  Operand rows of 32 bf16 (64 B) have the chunk order c ^ ((r >> 1) & 3), as in
+// the split-bf16 GEMM, under which the 16-row operand reads meet no LDS bank conflicts; the
+// order is made by the address each lane loads from.
+constexpr int EB_BM = 128, EB_BK = 32;
+template <int TN>
 struct EbTile {
-  static constexpr int NT = 128 * WN, BN = 64 * WN, LDF = BN + 1;
-  static constexpr int OPS = 2 * 2 * EB_BM * EB_LDSW * 2 + 2 * 2 * BN * EB_LDSW * 2;
-  static constexpr int F = EB_BM * LDF * 4;
-  static constexpr int F_PARTS = F + (NT / 64) * 16;
-  static constexpr int LDS = OPS > F_PARTS ? OPS : F_PARTS;
+  static constexpr int BN = 32 * TN, LDF = BN + 1;
+  static constexpr int OPS = 2 * (EB_BM + BN) * EB_BK * 2;
+  static constexpr int F = (EX_FR * LDF * 4 + 15) / 16 * 16;
+  static constexpr int BODY = OPS > F ? OPS : F;
+  static constexpr int LDS = BODY + EX_PARTS_BYTES;
+  static constexpr int WGS = TN <= 5 ? 3 : 2;  // workgroups per CU
+  static_assert(WGS * LDS <= 160 * 1024, "workgroups per CU");
 };
 
-template <int WN>
-__device__ __forceinline__ void exchange_bf16x3_body(
-    int G, int n, int K, int W, int gpt, int wpt, int g_tiles, int gc,
-    const uint16_t* __restrict__ Ah,
-    const uint16_t* __restrict__ Al, const uint16_t* __restrict__ Bh,
-    const uint16_t* __restrict__ Bl, cplx* __restrict__ xpart, const int bx) {
-  typedef EbTile<WN> Tile;
-  constexpr int NT = Tile::NT, BM = EB_BM, BN = Tile::BN, LDSW = EB_LDSW;
-  constexpr int TM = BM / 2 / 16, TN = BN / WN / 16;
-  constexpr int A_LD = BM * 4 / NT, B_LD = BN * 4 / NT;
-  static_assert(A_LD >= 1 && B_LD >= 1, "tile loads");
+template <int TN>
+__device__ __forceinline__ void exchange_bf16x3_body(const ExchArgs& x, const int bx) {
+  typedef EbTile<TN> Tile;
+  constexpr int BM = EB_BM, BN = Tile::BN, TM = 4, BK = EB_BK;
+  constexpr int LD = 4 + TN;  // loads per wave and k step: (8 + 2 TN) row groups, 2 planes
   __shared__ __attribute__((aligned(16))) unsigned char lds[Tile::LDS];
-  typedef uint16_t PlaneA[2][BM * LDSW];  // [hi/lo]
-  typedef uint16_t PlaneB[2][BN * LDSW];
-  PlaneA* sA = reinterpret_cast<PlaneA*>(lds);
-  PlaneB* sB = reinterpret_cast<PlaneB*>(lds + 2 * sizeof(PlaneA));
-  float* Fs = reinterpret_cast<float*>(lds);
 
+  const int n = x.n, K = x.K;
   int gt, wt;
-  exchange_tile_of(bx, g_tiles, (W + wpt - 1) / wpt, gc, &gt, &wt);
-  const int g0 = gt * gpt, w0 = wt * wpt;
-  const int M = G * n, NB = 2 * W * n;
+  exchange_tile_of(bx, x.g_tiles, (x.W + x.wpt - 1) / x.wpt, x.gc, &gt, &wt);
+  const int g0 = gt * x.gpt, w0 = wt * x.wpt;
   const int m0 = g0 * n, n0 = w0 * 2 * n;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave & 1, wn = wave >> 1;  // wn < WN
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
 
-  u32x4_t ra[2][A_LD], rb[2][B_LD];
-  auto load_tile = [&](int k0) {
+  // LDS: A hi, A lo (128 rows each), B hi, B lo (BN rows each), 1 KB per 16-row group.
+  // Group q of the wave's s-th load is wave + 4 s; rows past the operands read the last row
+  // (their products belong to no (g, w) block).
+  const uint16_t* src[LD];
+  int off[LD];
+  const int c0 = lane & 3, rl = lane >> 2;
+  const int ch = (c0 ^ ((rl >> 1) & 3)) * 8;
 #pragma unroll
-    for (int j = 0; j < A_LD; ++j) {
-      const int q = t + NT * j, row = q >> 2, ch = q & 3;
-      const int r = m0 + row;
-      u32x4_t vh = {0, 0, 0, 0}, vl = {0, 0, 0, 0};
-      if (r < M) {
-        vh = *reinterpret_cast<const u32x4_t*>(Ah + (int64_t)r * K + k0 + ch * 8);
-        vl = *reinterpret_cast<const u32x4_t*>(Al + (int64_t)r * K + k0 + ch * 8);
-      }
-      ra[0][j] = vh;
-      ra[1][j] = vl;
+  for (int s = 0; s < LD; ++s) {
+    const int q = wave + 4 * s;
+    if (s < 4) {
+      src[s] = static_cast<const uint16_t*>(s < 2 ? x.A : x.Al) + (int64_t)m0 * K;
+      off[s] = min((q & 7) * 16 + rl, x.G * n - 1 - m0) * K + ch;
+    } else {
+      const int qb = q - 16, lo = qb >= 2 * TN ? 1 : 0;
+      src[s] = static_cast<const uint16_t*>(lo ? x.Bl : x.B) + (int64_t)n0 * K;
+      off[s] = min((qb - lo * 2 * TN) * 16 + rl, 2 * x.W * n - 1 - n0) * K + ch;
     }
-#pragma unroll
-    for (int j = 0; j < B_LD; ++j) {
-      const int q = t + NT * j, row = q >> 2, ch = q & 3;
-      const int r = n0 + row;
-      u32x4_t vh = {0, 0, 0, 0}, vl = {0, 0, 0, 0};
-      if (r < NB) {
-        vh = *reinterpret_cast<const u32x4_t*>(Bh + (int64_t)r * K + k0 + ch * 8);
-        vl = *reinterpret_cast<const u32x4_t*>(Bl + (int64_t)r * K + k0 + ch * 8);
-      }
-      rb[0][j] = vh;
-      rb[1][j] = vl;
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < A_LD; ++j) {
-      const int q = t + NT * j, row = q >> 2, ch = q & 3;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        *reinterpret_cast<u32x4_t*>(&sA[buf][h][row * LDSW + eb_chunk(row, ch)]) = ra[h][j];
-    }
-#pragma unroll
-    for (int j = 0; j < B_LD; ++j) {
-      const int q = t + NT * j, row = q >> 2, ch = q & 3;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        *reinterpret_cast<u32x4_t*>(&sB[buf][h][row * LDSW + eb_chunk(row, ch)]) = rb[h][j];
-    }
-  };
+  }
 
   float4_t acc[TM][TN];
 #pragma unroll
@@ -376,77 +337,81 @@ __device__ __forceinline__ void exchange_bf16x3_body(
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int nk = K / EB_BK;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  const int arow = wm * (BM / 2) + (lane & 15);
-  const int brow = wn * (BN / WN) + (lane & 15);
-  // k chunk lane >> 4 of rows whose bits 2-3 are those of lane (row = 16 t + lane % 16)
-  const int koff = eb_chunk(lane & 15, lane >> 4);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) load_tile((kt + 1) * EB_BK);
-    bf16x8_t ah[TM], al[TM], bh[TN], bl[TN];
+  const int koff = ((lane >> 4) ^ ((lane >> 1) & 3)) * 16;
+  const unsigned char* pa = lds + (wm * 64 + (lane & 15)) * 64 + koff;
+  const unsigned char* pb = lds + 2 * BM * 64 + (wn * 16 * TN + (lane & 15)) * 64 + koff;
+  for (int k0 = 0; k0 < K; k0 += BK) {
+    if (k0) __syncthreads();  // the last step's operands are no longer read
+#pragma unroll
+    for (int s = 0; s < LD; ++s)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(src[s] + (off[s] + k0)),
+          (__attribute__((address_space(3))) void*)(lds + (wave + 4 * s) * 1024), 16, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    bf16x8_t ah[TM], al[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int o = (arow + i * 16) * LDSW + koff;
-      ah[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&sA[cur][0][o]));
-      al[i] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&sA[cur][1][o]));
+      ah[i] = *reinterpret_cast<const bf16x8_t*>(pa + i * 1024);
+      al[i] = *reinterpret_cast<const bf16x8_t*>(pa + BM * 64 + i * 1024);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int o = (brow + j * 16) * LDSW + koff;
-      bh[j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&sB[cur][0][o]));
-      bl[j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&sB[cur][1][o]));
+      const bf16x8_t bh = *reinterpret_cast<const bf16x8_t*>(pb + j * 1024);
+      const bf16x8_t bl = *reinterpret_cast<const bf16x8_t*>(pb + BN * 64 + j * 1024);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl, acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh, acc[i][j], 0, 0, 0);
     }
+  }
+
+  float* Fs = reinterpret_cast<float*>(lds);
+  auto write = [&](int r0, int rows) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-      }
-    if (kt + 1 < nk) store_tile(cur ^ 1);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = wn * (BN / WN) + j * 16 + (lane & 15);
-#pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wm * (BM / 2) + i * 16 + 4 * (lane >> 4) + r;
-        Fs[row * Tile::LDF + col] = acc[i][j][r];
+        const int row = wm * 64 + i * 16 + 4 * (lane >> 4) + r - r0;
+        if ((unsigned)row < (unsigned)rows) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            Fs[row * Tile::LDF + wn * 16 * TN + j * 16 + (lane & 15)] = acc[i][j][r];
+        }
       }
-    }
-  __syncthreads();
-  const int g_used = (G - g0 < gpt) ? G - g0 : gpt;
-  const int w_used = (W - w0 < wpt) ? W - w0 : wpt;
-  exchange_tile<float, NT>(Fs, Tile::LDF, n, g_used, w_used, w0, xpart + (int64_t)gt * W,
-                           reinterpret_cast<cplx*>(lds + Tile::F));
+  };
+  exchange_reduce<float>(Fs, Tile::LDF, n, min(x.gpt, x.G - g0), min(x.wpt, x.W - w0), w0,
+                         x.xpart + (int64_t)gt * x.W,
+                         reinterpret_cast<cplx*>(lds + Tile::BODY), write);
 }
 
-template <int WN>
-__global__ __launch_bounds__(128 * WN) void exchange_bf16x3_kernel(
-    int G, int n, int K, int W, int gpt, int wpt, int g_tiles, int gc,
-    const uint16_t* __restrict__ Ah, const uint16_t* __restrict__ Al,
-    const uint16_t* __restrict__ Bh, const uint16_t* __restrict__ Bl, cplx* __restrict__ xpart) {
-  exchange_bf16x3_body<WN>(G, n, K, W, gpt, wpt, g_tiles, gc, Ah, Al, Bh, Bl, xpart,
-                           blockIdx.x);
+template <bool F32, int BM, int TN>
+__global__ __launch_bounds__(EX_NT, 2) void exchange_f64_kernel(ExchArgs a) {
+  exchange_f64_body<F32, BM, TN>(a, blockIdx.x);
 }
 
-template <int WN>
-__global__ __launch_bounds__(128 * WN) void exchange_bf16x3_grouped_kernel(
+template <bool F32, int BM, int TN>
+__global__ __launch_bounds__(EX_NT, 2) void exchange_f64_grouped_kernel(
     const ExchArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
-  const ExchArgs a = args[p];
-  exchange_bf16x3_body<WN>(a.G, a.n, a.K, a.W, a.gpt, a.wpt, a.g_tiles, a.gc,
-                           static_cast<const uint16_t*>(a.A), static_cast<const uint16_t*>(a.Al),
-                           static_cast<const uint16_t*>(a.B), static_cast<const uint16_t*>(a.Bl),
-                           a.xpart, blockIdx.x - start[p]);
+  exchange_f64_body<F32, BM, TN>(args[p], blockIdx.x - start[p]);
+}
+
+template <int TN>
+__global__ __launch_bounds__(EX_NT, EbTile<TN>::WGS) void exchange_bf16x3_kernel(ExchArgs a) {
+  exchange_bf16x3_body<TN>(a, blockIdx.x);
+}
+
+template <int TN>
+__global__ __launch_bounds__(EX_NT, EbTile<TN>::WGS) void exchange_bf16x3_grouped_kernel(
+    const ExchArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
+  const int p = group_of(start, nprob, blockIdx.x);
+  exchange_bf16x3_body<TN>(args[p], blockIdx.x - start[p]);
 }
 
 // E_w = sum_g (c_g^2 - x_g) / 2 + sum_s m_s sum G_s rot_h1_s + h0 with c_g the summed
@@ -525,53 +490,120 @@ __global__ __launch_bounds__(ENER_NT) void energy_finish_grouped_kernel(
 
 }  // namespace
 
-// Waves across the split-bf16 exchange tile for n occupied orbitals: 4 (256 columns)
-// where that tile holds at least 1.2 times the walker columns per Cholesky row of the
-// 128-column one, else 2.
-int exchange_wn(int n) {
-  const int c2 = (128 / (2 * n)) * 2, c4 = (256 / (2 * n)) * 2;
-  return 5 * c4 >= 12 * c2 ? 4 : 2;
+namespace {
+
+// Exchange tile of a context and spin: rows bm holding gpt whole g, 16-column tiles tn (per
+// workgroup; the split-bf16 one has two waves across, so tn is even there) holding wpt whole
+// walkers.  Rows: 128, but 64 for n < 8 and where 128 would leave CUs idle (float64 / FP32).
+// Columns: the width of the best filled columns, the wider one at equal fill.
+enum { EXCH_BF16 = 0, EXCH_F64 = 1, EXCH_F32 = 2 };
+struct ExchTile {
+  int family, bm, tn, gpt, wpt;
+};
+ExchTile exchange_tile_for(const afqmc_ctx* c, int s) {
+  const int n = c->nocc[s], W = c->d.n_walkers, G = c->d.nchol;
+  ExchTile x;
+  x.family = c->mixed ? EXCH_BF16 : (c->f32 ? EXCH_F32 : EXCH_F64);
+  const int step = c->mixed ? 2 : 1;
+  if (n < 16) {
+    x.tn = 8;
+  } else {
+    x.tn = 8 * step;
+    for (int tn = 8 * step; tn >= (c->mixed ? 4 : 5) * step; tn -= step)
+      if ((16 * tn / (2 * n)) * x.tn > (16 * x.tn / (2 * n)) * tn) x.tn = tn;
+  }
+  x.bm = 128;
+  if (!c->mixed) {
+    const int gp = 128 / n, wp = 16 * x.tn / (2 * n);
+    const int64_t blocks = (int64_t)((G + gp - 1) / gp) * ((W + wp - 1) / wp);
+    if (n < 8 || blocks < 512) {
+      x.bm = 64;
+      x.tn = 8;
+    }
+  }
+  x.gpt = x.bm / n;
+  x.wpt = 16 * x.tn / (2 * n);
+  return x;
 }
 
+template <bool GROUPED, typename Single, typename Grouped>
+void launch_exchange_kernel(hipStream_t st, Single one, Grouped many, const ExchArgs& a,
+                            const ExchArgs* args, const int* start, int nprob, int nblocks) {
+  if constexpr (GROUPED)
+    hipLaunchKernelGGL(many, dim3(nblocks), dim3(EX_NT), 0, st, args, start, nprob);
+  else
+    hipLaunchKernelGGL(one, dim3(nblocks), dim3(EX_NT), 0, st, a);
+}
+
+inline int exchange_kind(const ExchTile& x) { return (x.family * 256 + x.bm) * 32 + x.tn; }
+
+template <bool GROUPED>
+int launch_exchange(hipStream_t st, int kind, const ExchArgs& a, const ExchArgs* args,
+                    const int* start, int nprob, int nblocks) {
+#define EXCH_CASE(family, bm, tn, one, many)                                                  \
+  case (family * 256 + bm) * 32 + tn:                                                         \
+    launch_exchange_kernel<GROUPED>(st, one, many, a, args, start, nprob, nblocks);           \
+    break;
+#define EXCH_BF(t) \
+  EXCH_CASE(EXCH_BF16, 128, 2 * t, exchange_bf16x3_kernel<t>, exchange_bf16x3_grouped_kernel<t>)
+#define EXCH_F(family, f32, bm, t)                                     \
+  EXCH_CASE(family, bm, t, (exchange_f64_kernel<f32, bm, t>), \
+            (exchange_f64_grouped_kernel<f32, bm, t>))
+  switch (kind) {
+    EXCH_BF(4) EXCH_BF(5) EXCH_BF(6) EXCH_BF(7) EXCH_BF(8)
+    EXCH_F(EXCH_F64, false, 128, 5) EXCH_F(EXCH_F64, false, 128, 6)
+    EXCH_F(EXCH_F64, false, 128, 7) EXCH_F(EXCH_F64, false, 128, 8)
+    EXCH_F(EXCH_F64, false, 64, 8)
+    EXCH_F(EXCH_F32, true, 128, 5) EXCH_F(EXCH_F32, true, 128, 6)
+    EXCH_F(EXCH_F32, true, 128, 7) EXCH_F(EXCH_F32, true, 128, 8)
+    EXCH_F(EXCH_F32, true, 64, 8)
+    default:
+      return afqmc_set_error(AFQMC_ERR_STATE, "exchange: no kernel for tile %d", kind);
+  }
+#undef EXCH_F
+#undef EXCH_BF
+#undef EXCH_CASE
+  LAUNCH_CHECK();
+  return AFQMC_OK;
+}
+
+}  // namespace
+
 int energy_g_tiles(const afqmc_ctx* c, int s) {
-  const int n = c->nocc[s];
-  if (n < 1) return 0;
-  const int gpt = (c->mixed ? EB_BM : EF_BM) / n;
+  if (c->nocc[s] < 1) return 0;
+  const int gpt = exchange_tile_for(c, s).gpt;
   return (c->d.nchol + gpt - 1) / gpt;
 }
 
 void exchange_plan(const afqmc_ctx* c, int s, int W, ExchArgs* a, int* kind, int* nblocks) {
+  static_assert(AFQMC_MAX_NOCC <= EX_FR && 2 * AFQMC_MAX_NOCC <= 128,
+                "a (g, w) block must fit one tile and one pass");
   const int N = c->d.norb, G = c->d.nchol, n = c->nocc[s];
   cplx* xp = c->energy_x;
   for (int t = 0; t < s; ++t) xp += (int64_t)energy_g_tiles(c, t) * W;
+  const ExchTile x = exchange_tile_for(c, s);
   *a = ExchArgs{};
   a->G = G;
   a->n = n;
   a->W = W;
   a->xpart = xp;
+  a->gpt = x.gpt;
+  a->wpt = x.wpt;
+  a->g_tiles = (G + x.gpt - 1) / x.gpt;
   if (c->mixed) {
-    const int wn = exchange_wn(n);
     a->K = c->Np32;
-    a->gpt = EB_BM / n;
-    a->wpt = 64 * wn / (2 * n);
-    a->g_tiles = (G + a->gpt - 1) / a->gpt;
     a->gc = exchange_chunk(a->g_tiles, (int64_t)a->gpt * n * c->Np32 * 4);
     a->A = c->rot_chol_bf[s][0];
     a->Al = c->rot_chol_bf[s][1];
     a->B = c->green_bf[s][0];
     a->Bl = c->green_bf[s][1];
-    *kind = wn == 4 ? EXCH_BF16X3_WN4 : EXCH_BF16X3_WN2;
   } else {
-    const bool vec2 = (N % 2 == 0);
     a->K = N;
-    a->gpt = EF_BM / n;
-    a->wpt = EF_BN / (2 * n);
-    a->g_tiles = (G + a->gpt - 1) / a->gpt;
     a->gc = exchange_chunk(a->g_tiles, (int64_t)a->gpt * n * N * 8);
     a->A = c->rot_chol[s];
     a->B = c->green[s];
-    *kind = c->f32 ? (vec2 ? EXCH_F32_V2 : EXCH_F32_V1) : (vec2 ? EXCH_F64_V2 : EXCH_F64_V1);
   }
+  *kind = exchange_kind(x);
   *nblocks = a->g_tiles * ((W + a->wpt - 1) / a->wpt);
 }
 
@@ -600,34 +632,7 @@ void energy_finish_args(const afqmc_ctx* c, int W, cplx* energies, FinishArgs* a
 
 int launch_exchange_grouped(hipStream_t st, int kind, const ExchArgs* args, const int* start,
                             int nprob, int nblocks) {
-  switch (kind) {
-    case EXCH_BF16X3_WN2:
-      hipLaunchKernelGGL(exchange_bf16x3_grouped_kernel<2>, dim3(nblocks), dim3(EbTile<2>::NT),
-                         0, st, args, start, nprob);
-      break;
-    case EXCH_BF16X3_WN4:
-      hipLaunchKernelGGL(exchange_bf16x3_grouped_kernel<4>, dim3(nblocks), dim3(EbTile<4>::NT),
-                         0, st, args, start, nprob);
-      break;
-    case EXCH_F64_V1:
-      hipLaunchKernelGGL((exchange_f64_grouped_kernel<1, false>), dim3(nblocks), dim3(ENER_NT),
-                         0, st, args, start, nprob);
-      break;
-    case EXCH_F64_V2:
-      hipLaunchKernelGGL((exchange_f64_grouped_kernel<2, false>), dim3(nblocks), dim3(ENER_NT),
-                         0, st, args, start, nprob);
-      break;
-    case EXCH_F32_V1:
-      hipLaunchKernelGGL((exchange_f64_grouped_kernel<1, true>), dim3(nblocks), dim3(ENER_NT),
-                         0, st, args, start, nprob);
-      break;
-    default:
-      hipLaunchKernelGGL((exchange_f64_grouped_kernel<2, true>), dim3(nblocks), dim3(ENER_NT),
-                         0, st, args, start, nprob);
-      break;
-  }
-  LAUNCH_CHECK();
-  return AFQMC_OK;
+  return launch_exchange<true>(st, kind, ExchArgs{}, args, start, nprob, nblocks);
 }
 
 int launch_energy_finish_grouped(hipStream_t st, const FinishArgs* args, const int* start,
@@ -641,52 +646,12 @@ int launch_energy_finish_grouped(hipStream_t st, const FinishArgs* args, const i
 // Needs the float64 Green's function of every spin in c->green (and, in the mixed mode,
 // its split-bf16 planes) and the float64 force bias in c->fb (c->fb_parts slices).
 int launch_energy(afqmc_ctx* c, int W, cplx* energies) {
-  static_assert(AFQMC_MAX_NOCC <= EF_BM && 2 * AFQMC_MAX_NOCC <= EF_BN,
-                "a (g, w) block must fit one tile");
-  static_assert(AFQMC_MAX_NOCC <= EB_BM && 2 * AFQMC_MAX_NOCC <= EbTile<2>::BN,
-                "a (g, w) block must fit one tile");
   for (int s = 0; s < c->nspin; ++s) {
     ExchArgs a;
     int kind, nb;
     exchange_plan(c, s, W, &a, &kind, &nb);
-    const dim3 grid(nb);
-    switch (kind) {
-      case EXCH_BF16X3_WN4:
-      case EXCH_BF16X3_WN2: {
-        const uint16_t* Ah = static_cast<const uint16_t*>(a.A);
-        const uint16_t* Al = static_cast<const uint16_t*>(a.Al);
-        const uint16_t* Bh = static_cast<const uint16_t*>(a.B);
-        const uint16_t* Bl = static_cast<const uint16_t*>(a.Bl);
-        if (kind == EXCH_BF16X3_WN4)
-          hipLaunchKernelGGL(exchange_bf16x3_kernel<4>, grid, dim3(EbTile<4>::NT), 0, c->stream,
-                             a.G, a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, Ah, Al, Bh, Bl,
-                             a.xpart);
-        else
-          hipLaunchKernelGGL(exchange_bf16x3_kernel<2>, grid, dim3(EbTile<2>::NT), 0, c->stream,
-                             a.G, a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, Ah, Al, Bh, Bl,
-                             a.xpart);
-        break;
-      }
-      default: {
-        const double* A = static_cast<const double*>(a.A);
-        const double* B = static_cast<const double*>(a.B);
-        const dim3 block(ENER_NT);
-        if (kind == EXCH_F32_V2)
-          hipLaunchKernelGGL((exchange_f64_kernel<2, true>), grid, block, 0, c->stream, a.G,
-                             a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, A, B, a.xpart);
-        else if (kind == EXCH_F32_V1)
-          hipLaunchKernelGGL((exchange_f64_kernel<1, true>), grid, block, 0, c->stream, a.G,
-                             a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, A, B, a.xpart);
-        else if (kind == EXCH_F64_V2)
-          hipLaunchKernelGGL((exchange_f64_kernel<2, false>), grid, block, 0, c->stream, a.G,
-                             a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, A, B, a.xpart);
-        else
-          hipLaunchKernelGGL((exchange_f64_kernel<1, false>), grid, block, 0, c->stream, a.G,
-                             a.n, a.K, W, a.gpt, a.wpt, a.g_tiles, a.gc, A, B, a.xpart);
-        break;
-      }
-    }
-    LAUNCH_CHECK();
+    int rc = launch_exchange<false>(c->stream, kind, a, nullptr, nullptr, 0, nb);
+    if (rc) return rc;
   }
   FinishArgs f;
   energy_finish_args(c, W, energies, &f);

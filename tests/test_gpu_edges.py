@@ -136,3 +136,22 @@ def test_orthonormalize_columns_and_scales(gpu, norb, n, scale):
     ref = np.array([np.linalg.qr(x)[0] for x in w])
     assert np.max(np.linalg.cond(w)) < 1e4
     assert rel(got, ref) < 1e-11
+
+
+# float32 carries 24 bits.  Split-bf16 drops lo * lo and rounds each lo, at most 3 * 2^-18 of
+# a product, twice that for tr f f: 2.3e-5 of sums of magnitudes up to four times the energy
+@pytest.mark.parametrize("precision,tol", [("fp64", TOL), ("fp32", 2e-5), ("bf16x3", 1e-4)])
+@pytest.mark.parametrize("norb,nelec,nchol,W", [
+    (3, (1, 1), 5, 200), (5, (2, 1), 9, 70), (18, (16, 8), 240, 77), (25, (22, 13), 61, 170),
+    (27, (24, 20), 61, 163), (33, (29, 17), 83, 130), (43, (40, 33), 31, 50),
+    (66, (64, 50), 19, 60)])
+def test_energy_at_each_exchange_tile(gpu, norb, nelec, nchol, W, precision, tol):
+    """Local energies at every row and column count of the exchange tile, with partly filled
+    last tiles in both directions, one and several passes and walker groups."""
+    print(f"exchange N={norb} nelec={nelec} G={nchol} W={W} {precision}", flush=True)
+    hd, wd, nelec = problem("uhf", norb, nelec, nchol)
+    trial, prop, hdat, wave, oh = make("uhf", norb, nelec, nchol, W, hd, wd, precision)
+    walkers = problems.random_walkers("uhf", norb, nelec, W, np.random.default_rng(3),
+                                      near=wd["mo_coeff"], noise=0.1)
+    got = trial.calc_energy(to_dev(walkers, gpu), hdat, wave)
+    assert rel(got, o.calc_energy("uhf", walkers, oh, wd)) < tol
