@@ -77,13 +77,11 @@ void free_ctx(afqmc_ctx* c) {
   if (!c) return;
   void* ptrs[] = {c->trial[0], c->trial[1], c->rot_h1[0], c->rot_h1[1], c->rot_chol[0],
                   c->rot_chol[1], c->chol_t, c->exp_h1[0], c->exp_h1[1], c->mf_shifts,
-                  c->emi_bf[0][0], c->emi_bf[0][1], c->emi_bf[1][0], c->emi_bf[1][1], c->chol_t_bf[0],
-                  c->chol_t_bf[1], c->rot_chol_bf[0][0], c->rot_chol_bf[0][1],
-                  c->rot_chol_bf[1][0], c->rot_chol_bf[1][1], c->green[0], c->green[1], c->fb,
+                  c->emi_bf[0][0], c->emi_bf[0][1], c->emi_bf[1][0], c->emi_bf[1][1], c->chol_t_bf,
+                  c->rot_chol_bf[0], c->rot_chol_bf[1], c->green[0], c->green[1], c->fb,
                   c->xs, c->vhs, c->terms, c->dets, c->energy_x, c->energy_acc, c->walk_tmp,
-                  c->sr_cum, c->sr_idx, c->xs_bf[0], c->xs_bf[1], c->green_bf[0][0],
-                  c->green_bf[0][1], c->green_bf[1][0], c->green_bf[1][1], c->vhs_f32,
-                  c->sym_stat};
+                  c->sr_cum, c->sr_idx, c->xs_bf, c->green_bf[0], c->green_bf[1],
+                  c->vhs_f32, c->sym_stat};
   prof_free(&c->prof);
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -154,9 +152,8 @@ int force_bias_gemm(afqmc_ctx* c, int W, int mode) {
       if (sp == 1 && big < 512 && kd >= 4096) sp = (int)std::min<int64_t>(4, (511 + big) / big);
       if (part + sp > c->fb_cap)
         return afqmc_set_error(AFQMC_ERR_STATE, "force-bias split slices exceed workspace");
-      rc = launch_gemm_nt_bf16x3_f64(c->stream, 2 * W, G, kd, (float)c->mult, c->green_bf[s][0],
-                                     c->green_bf[s][1], kd, c->rot_chol_bf[s][0],
-                                     c->rot_chol_bf[s][1], kd, c->fb + part * slice, G, sp, slice);
+      rc = launch_gemm_nt_bf16x3_f64(c->stream, 2 * W, G, kd, (float)c->mult, c->green_bf[s],
+                                     c->rot_chol_bf[s], c->fb + part * slice, G, sp, slice);
     } else {
       const int kd = c->kdim[s];
       sp = gemm_f64_splits(2 * W, G, kd);
@@ -282,26 +279,22 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
     c->taylor_bf = c->mixed;  // split-bf16 Taylor kernels (register or streaming form)
     if (c->mixed) {
       const size_t nn = (size_t)N * N;
-      for (int h = 0; h < 2; ++h)
-        TRY(dalloc(c, &c->chol_t_bf[h], (size_t)c->chol_spins * c->vhs_nv * c->Gp));
+      TRY(dalloc(c, &c->chol_t_bf, 2 * (size_t)c->chol_spins * c->vhs_nv * c->Gp));
       for (int cs = 0; cs < c->chol_spins; ++cs)
-        TRY(launch_split_bf16(c->stream, c->vhs_nv, G, chol_t_of(c, cs), G, chol_t_bf_of(c, 0, cs),
-                              chol_t_bf_of(c, 1, cs), c->Gp));
+        TRY(launch_split_bf16(c->stream, c->vhs_nv, G, chol_t_of(c, cs), G, chol_t_bf_of(c, cs),
+                              nullptr, c->Gp));
       for (int s = 0; s < c->nspin; ++s) {
         const size_t rows = (size_t)G * c->nocc[s];
-        for (int h = 0; h < 2; ++h) {
-          TRY(dalloc(c, &c->rot_chol_bf[s][h], rows * c->Np32));
-          TRY(dalloc(c, &c->green_bf[s][h], (size_t)W * 2 * c->nocc[s] * c->Np32));
-          TRY(zero_async(c->green_bf[s][h],
-                         (size_t)W * 2 * c->nocc[s] * c->Np32 * sizeof(uint16_t), c->stream));
-        }
-        TRY(launch_split_bf16(c->stream, (int)rows, N, c->rot_chol[s], N, c->rot_chol_bf[s][0],
-                              c->rot_chol_bf[s][1], c->Np32));
+        const size_t green = 2 * (size_t)W * 2 * c->nocc[s] * c->Np32;
+        TRY(dalloc(c, &c->rot_chol_bf[s], 2 * rows * c->Np32));
+        TRY(dalloc(c, &c->green_bf[s], green));
+        TRY(zero_async(c->green_bf[s], green * sizeof(uint16_t), c->stream));
+        TRY(launch_split_bf16(c->stream, (int)rows, N, c->rot_chol[s], N, c->rot_chol_bf[s],
+                              nullptr, c->Np32));
       }
-      for (int h = 0; h < 2; ++h) {
-        TRY(dalloc(c, &c->xs_bf[h], (size_t)W * 2 * c->Gp));
-        TRY(zero_async(c->xs_bf[h], (size_t)W * 2 * c->Gp * sizeof(uint16_t), c->stream));
-      }
+      const size_t xs = 2 * (size_t)W * 2 * c->Gp;
+      TRY(dalloc(c, &c->xs_bf, xs));
+      TRY(zero_async(c->xs_bf, xs * sizeof(uint16_t), c->stream));
       if (c->taylor_bf) {
         // 8 floats of tail padding: the streaming split-bf16 Taylor kernel reads V rows in
         // 8-float chunks, and the chunk that straddles the end of the last row is masked;
@@ -416,10 +409,8 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
     PhaseTimer t(c, AFQMC_PH_VHS_GEMM);
     for (int cs = 0; cs < c->chol_spins && !rc; ++cs) {
       if (c->mixed)
-        rc = launch_gemm_nt_bf16x3_f32(c->stream, 2 * W, c->vhs_nv, c->Gp, 1.0f, c->xs_bf[0],
-                                       c->xs_bf[1], c->Gp, chol_t_bf_of(c, 0, cs),
-                                       chol_t_bf_of(c, 1, cs), c->Gp, vhs_f32_of(c, cs),
-                                       c->vhs_nv, 1, 0);
+        rc = launch_gemm_nt_bf16x3_f32(c->stream, 2 * W, c->vhs_nv, c->Gp, 1.0f, c->xs_bf,
+                                       chol_t_bf_of(c, cs), vhs_f32_of(c, cs), c->vhs_nv, 1, 0);
       else if (c->f32)
         rc = launch_gemm_nt_f32(c->stream, 2 * W, c->vhs_nv, c->d.nchol, 1.0, c->xs, c->d.nchol,
                                 chol_t_of(c, cs), c->d.nchol, 0.0, vhs_of(c, cs), c->vhs_nv);

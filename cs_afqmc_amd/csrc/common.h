@@ -96,6 +96,17 @@ __device__ inline void split_bf16(double x, uint16_t* hi, uint16_t* lo) {
   *lo = (uint16_t)(hl >> 16);
 }
 
+// Split-bf16 GEMM operands: rows whose length is a multiple of 32, each block of 32 elements
+// stored as its 32 hi values, then its 32 lo values: one 128-byte line.  (As two planes, an
+// operand tile took 64 bytes of each line it touched, and the L2 request rate bounded the
+// tiles.)  bf_pos(e): where element e (rows end to end) has its hi; its lo is BF_LO further.
+constexpr int BF_LO = 32;
+__host__ __device__ inline int64_t bf_pos(int64_t e) { return e + (e & ~(int64_t)31); }
+__device__ inline void store_split_bf16(uint16_t* p, int64_t e, double x) {
+  uint16_t* q = p + bf_pos(e);
+  split_bf16(x, q, q + BF_LO);
+}
+
 // ---------------------------------------------------------------- walker weights
 struct WeightsArgs {
   int W, nspin;
@@ -242,10 +253,10 @@ struct afqmc_ctx {
   int Np32;                  // norb rounded up to 32
   int vhs_nv;                // stored entries of one V plane: N*N, or N(N+1)/2 when V is
                              // kept as its upper triangle (symmetric Cholesky vectors)
-  uint16_t* chol_t_bf[2];    // hi / lo planes of chol_t, (vhs_nv, Gp)
-  uint16_t* rot_chol_bf[2][2];  // [spin][hi/lo], (G, n_sigma, Np32)
-  uint16_t* xs_bf[2];        // [hi/lo] (2W, Gp): i sqrt(dt) x~
-  uint16_t* green_bf[2][2];  // [spin][hi/lo] (W, 2, n_sigma, Np32)
+  uint16_t* chol_t_bf;       // split-bf16 operand: chol_t, (vhs_nv, Gp)
+  uint16_t* rot_chol_bf[2];  // [spin] split-bf16 operand, (G, n_sigma, Np32)
+  uint16_t* xs_bf;           // split-bf16 operand, (2W, Gp): i sqrt(dt) x~
+  uint16_t* green_bf[2];     // [spin] split-bf16 operand, (W, 2, n_sigma, Np32)
   float* vhs_f32;            // chol_spins x [(W, 2, vhs_nv) + 8 floats of padding]
   int64_t vhs_f32_stride;    // floats between the spins' V blocks
   unsigned long long* sym_stat;  // (2) Cholesky symmetry check at creation
@@ -280,8 +291,8 @@ inline int chol_spin(const afqmc_ctx* c, int s) { return c->chol_spins == 2 ? s 
 inline double* chol_t_of(const afqmc_ctx* c, int s) {
   return c->chol_t + (size_t)chol_spin(c, s) * c->vhs_nv * c->d.nchol;
 }
-inline uint16_t* chol_t_bf_of(const afqmc_ctx* c, int h, int s) {
-  return c->chol_t_bf[h] + (size_t)chol_spin(c, s) * c->vhs_nv * c->Gp;
+inline uint16_t* chol_t_bf_of(const afqmc_ctx* c, int s) {
+  return c->chol_t_bf + 2 * (size_t)chol_spin(c, s) * c->vhs_nv * c->Gp;
 }
 inline double* vhs_of(const afqmc_ctx* c, int s) {
   return c->vhs + (size_t)chol_spin(c, s) * c->d.n_walkers * 2 * c->vhs_nv;
@@ -366,15 +377,14 @@ int launch_transpose_f64(hipStream_t s, int rows, int cols, int packed_n, const 
 // largest asymmetry and entry of count n x n matrices, as bit patterns into out[0], out[1]
 int launch_sym_check(hipStream_t s, int n, int64_t count, const double* L,
                      unsigned long long* out);
-// gemm_bf16x3.hip: split-bf16 NT GEMM (K, lda, ldb multiples of 32 / 8), float / double out
-int launch_gemm_nt_bf16x3_f32(hipStream_t s, int M, int N, int K, float alpha,
-                              const uint16_t* Ah, const uint16_t* Al, int64_t lda,
-                              const uint16_t* Bh, const uint16_t* Bl, int64_t ldb, float* C,
-                              int64_t ldc, int splits, int64_t c_split_stride);
-int launch_gemm_nt_bf16x3_f64(hipStream_t s, int M, int N, int K, float alpha,
-                              const uint16_t* Ah, const uint16_t* Al, int64_t lda,
-                              const uint16_t* Bh, const uint16_t* Bl, int64_t ldb, double* C,
-                              int64_t ldc, int splits, int64_t c_split_stride);
+// gemm_bf16x3.hip: split-bf16 NT GEMM (rows of K, a multiple of 32), float / double out
+int launch_gemm_nt_bf16x3_f32(hipStream_t s, int M, int N, int K, float alpha, const uint16_t* A,
+                              const uint16_t* B, float* C, int64_t ldc, int splits,
+                              int64_t c_split_stride);
+int launch_gemm_nt_bf16x3_f64(hipStream_t s, int M, int N, int K, float alpha, const uint16_t* A,
+                              const uint16_t* B, double* C, int64_t ldc, int splits,
+                              int64_t c_split_stride);
+// x as a split-bf16 operand at hi (lo null), or as two planes
 int launch_split_bf16(hipStream_t s, int rows, int cols, const double* x, int64_t ld_src,
                       uint16_t* hi, uint16_t* lo, int64_t ld_dst);
 // measure.hip: green_f64 -> c->green (float64 split layout); green_bf -> c->green_bf
@@ -430,8 +440,7 @@ struct MeasureArgs {
   const double* trial;
   cplx* dets;
   double* green;
-  uint16_t* ghi;
-  uint16_t* glo;
+  uint16_t* gbf;
 };
 struct FieldsArgs {
   int G, nparts, Gp, W;
@@ -441,8 +450,7 @@ struct FieldsArgs {
   const cplx* mf;
   const double* fields;  // step s reads fields + s * W * G
   double* xs;
-  uint16_t* xs_hi;
-  uint16_t* xs_lo;
+  uint16_t* xs_bf;
   cplx* terms;
 };
 struct TaylorArgs {
@@ -457,10 +465,8 @@ struct GemmArgs {
   int M, N, K, tiles_m, tiles_n;
   float alpha;
   int64_t lda, ldb, ldc;
-  const void* A;   // float64, or the bf16 hi plane
-  const void* Al;  // bf16 lo plane (split-bf16 only)
+  const void* A;  // float64 or split-bf16
   const void* B;
-  const void* Bl;
   void* C;
 };
 
@@ -476,10 +482,8 @@ struct OvcArgs {
 };
 struct ExchArgs {
   int G, n, K, W, gpt, wpt, g_tiles, gc;
-  const void* A;   // float64, or the bf16 hi plane (half-rotated Cholesky vectors)
-  const void* Al;  // bf16 lo plane (split-bf16 only)
-  const void* B;   // float64 Green's function, or its bf16 hi plane
-  const void* Bl;
+  const void* A;  // half-rotated Cholesky vectors, float64 or split-bf16
+  const void* B;  // Green's function, float64 or split-bf16
   cplx* xpart;
 };
 struct FinishArgs {

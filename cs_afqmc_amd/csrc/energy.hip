@@ -54,25 +54,45 @@ inline int exchange_chunk(int g_tiles, int64_t tile_bytes) {
 
 // ---------------------------------------------------------------- fused exchange
 
-// Exchange sums of a workgroup's F tile: F row gl*n + i, column wl*2n + c*n + j, and
-// x_w = sum_g sum_ij f(i,j) f(j,i), taken over the pairs i <= j (weight 2 off the
-// diagonal).  The tile goes through LDS in passes of as many whole g as fit EX_FR rows
-// (write(r0, rows) stores rows r0 .. r0 + rows - 1 to Fs), so the operand buffers' LDS
-// serves it and two or three workgroups share a CU: one reduces while the others multiply.
-// Within a pass every thread takes (g, pair) items and runs over the walkers with their
-// four loads all in flight; its sums stay in registers over the passes, EX_MAXW walkers at
-// a time (tiles of more walkers, n <= 7, add up per pass instead).  Sums over threads: wave
-// tree, then the waves in order.
-constexpr int EX_NT = 256, EX_FR = 64, EX_MAXW = 8;
-// partial sums of 4 waves x up to 64 walkers
-constexpr int EX_PARTS_BYTES = 4 * 64 * 16;
+// Exchange sums of a workgroup's F tile: F row gl*n + i, column wl*2n + 2j + c (the re and
+// im of an entry side by side: the operand rows are staged in that order), and x_w =
+// sum_g sum_ij f(i,j) f(j,i), taken over the pairs i <= j (weight 2 off the diagonal).  The
+// tile goes through LDS in passes of as many whole g as fit EX_FR rows (write(r0, rows)
+// stores rows r0 .. r0 + rows - 1 to Fs), so the operand buffers' LDS serves it and two or
+// three workgroups share a CU: one reduces while the others multiply.  A wave's vector
+// instructions and MFMAs take turns on its SIMD, so the instruction count of this part is
+// what it costs: every thread takes (g, pair) items, with the pair from a table, and runs
+// over the walkers; its sums stay in registers over the passes, EX_MAXW walkers at a time
+// (tiles of more walkers, n <= 7, add up per pass instead).  Sums over threads: wave tree,
+// then the waves in order.
+constexpr int EX_NT = 256, EX_FR = 64, EX_MAXW = 8, EX_WMAX = 64;
+
+// (i, j), i <= j, of pair q = j (j + 1) / 2 + i
+struct PairTable {
+  uint16_t ij[AFQMC_MAX_NOCC * (AFQMC_MAX_NOCC + 1) / 2];
+  constexpr PairTable() : ij() {
+    int q = 0;
+    for (int j = 0; j < AFQMC_MAX_NOCC; ++j)
+      for (int i = 0; i <= j; ++i) ij[q++] = (uint16_t)(i | j << 8);
+  }
+};
+__device__ const PairTable exchange_pairs{};
+
+// operand row of F column col: column w*2n + 2j + c holds walker row w*2n + c*n + j
+__device__ inline int exchange_col_row(int col, int n) {
+  const int w = (int)(((float)col + 0.5f) * (1.0f / (float)(2 * n)));
+  const int e = col - w * 2 * n;
+  return w * 2 * n + (e & 1) * n + (e >> 1);
+}
 
 template <typename T, typename WriteF>
 __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_used, int w_used,
                                                 int w0, cplx* __restrict__ xpart, cplx* parts,
                                                 WriteF write) {
+  typedef T T2 __attribute__((ext_vector_type(2)));
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int npairs = n * (n + 1) / 2;
+  const float inv_pairs = 1.0f / (float)npairs;
   const int gpp = EX_FR / n;  // g per pass
   const bool persist = w_used <= EX_MAXW;
   double xr[EX_MAXW], xi[EX_MAXW];
@@ -90,22 +110,22 @@ __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_use
         for (int k = 0; k < EX_MAXW; ++k) xr[k] = xi[k] = 0.0;
       }
       for (int it = t; it < gn * npairs; it += EX_NT) {
-        const int gl = it / npairs, q = it - gl * npairs;
-        // pair q = a (a + 1) / 2 + b, b <= a: (i, j) = (b, a)
-        int a = (int)((sqrtf(8.0f * (float)q + 1.0f) - 1.0f) * 0.5f);
-        if (a * (a + 1) / 2 > q) --a;
-        if ((a + 1) * (a + 2) / 2 <= q) ++a;
-        const int i = q - a * (a + 1) / 2, j = a;
+        // (exact: the product is off by less than half of 1 / npairs)
+        const int gl = (int)(((float)it + 0.5f) * inv_pairs);
+        const int ij = exchange_pairs.ij[it - gl * npairs];
+        const int i = ij & 255, j = ij >> 8;
         const T wgt = i == j ? (T)1 : (T)2;
-        const T* pa = Fs + (gl * n + i) * ldf + wb * 2 * n + j;  // f(i, j): re pa[0], im pa[n]
-        const T* pb = Fs + (gl * n + j) * ldf + wb * 2 * n + i;  // f(j, i)
+        const T* pa = Fs + (gl * n + i) * ldf + wb * 2 * n + 2 * j;  // f(i, j)
+        const T* pb = Fs + (gl * n + j) * ldf + wb * 2 * n + 2 * i;  // f(j, i)
 #pragma unroll
         for (int k = 0; k < EX_MAXW; ++k)
           if (wb + k < w_used) {
-            const double ar = (double)(wgt * pa[k * 2 * n]), ai = (double)(wgt * pa[k * 2 * n + n]);
-            const double br = (double)pb[k * 2 * n], bi = (double)pb[k * 2 * n + n];
-            xr[k] += ar * br - ai * bi;
-            xi[k] += ar * bi + ai * br;
+            const T2 fa = *reinterpret_cast<const T2*>(pa + k * 2 * n);
+            const T2 fb = *reinterpret_cast<const T2*>(pb + k * 2 * n);
+            const double ar = (double)(wgt * fa.x), ai = (double)(wgt * fa.y);
+            const double br = (double)fb.x, bi = (double)fb.y;
+            xr[k] = fma(-ai, bi, fma(ar, br, xr[k]));
+            xi[k] = fma(ai, br, fma(ar, bi, xi[k]));
           }
       }
       if (!persist || last) {
@@ -118,7 +138,7 @@ __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_use
               vi += __shfl_down(vi, off, 64);
             }
             if (lane == 0) {
-              cplx* p = parts + wave * 64 + wb + k;
+              cplx* p = parts + wave * EX_WMAX + wb + k;
               *p = g0 == 0 || persist ? cplx{vr, vi} : cplx{p->re + vr, p->im + vi};
             }
           }
@@ -129,7 +149,7 @@ __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_use
   if (t < w_used) {
     cplx x = parts[t];
 #pragma unroll
-    for (int v = 1; v < 4; ++v) x = cadd(x, parts[v * 64 + t]);
+    for (int v = 1; v < 4; ++v) x = cadd(x, parts[v * EX_WMAX + t]);
     xpart[w0 + t] = x;
   }
 }
@@ -152,11 +172,12 @@ template <bool F32, int BM, int TN>
 struct EfTile {
   typedef typename std::conditional<F32, float, double>::type T;
   static constexpr int BN = 16 * TN, BNP = (BN + 31) / 32 * 32;  // staged B rows
-  static constexpr int LDF = BN + 1;  // odd: transposed reads spread over the banks
+  // an odd number of entries: reads down a column spread over the banks
+  static constexpr int LDF = BN + 2;
   static constexpr int OPS = 2 * (BM + BNP) * EF_BK * (int)sizeof(T);
   static constexpr int F = (EX_FR * LDF * (int)sizeof(T) + 15) / 16 * 16;
   static constexpr int BODY = OPS > F ? OPS : F;
-  static constexpr int LDS = BODY + EX_PARTS_BYTES;
+  static constexpr int LDS = BODY + 4 * EX_WMAX * (int)sizeof(cplx);
 };
 
 template <bool F32, int BM, int TN>
@@ -177,7 +198,8 @@ __device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int b
   exchange_tile_of(bx, x.g_tiles, (x.W + x.wpt - 1) / x.wpt, x.gc, &gt, &wt);
   const int g0 = gt * x.gpt, w0 = wt * x.wpt;
   const int m0 = g0 * n, n0 = w0 * 2 * n;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lch = t & 7, lr = t >> 3;
   const double* Ab = static_cast<const double*>(x.A) + (int64_t)m0 * N;
   const double* Bb = static_cast<const double*>(x.B) + (int64_t)n0 * N;
@@ -185,7 +207,8 @@ __device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int b
 #pragma unroll
   for (int i = 0; i < A_LD; ++i) aoff[i] = min(lr + i * 32, x.G * n - 1 - m0) * N;
 #pragma unroll
-  for (int i = 0; i < B_LD; ++i) boff[i] = min(lr + i * 32, 2 * x.W * n - 1 - n0) * N;
+  for (int i = 0; i < B_LD; ++i)
+    boff[i] = min(exchange_col_row(lr + i * 32, n), 2 * x.W * n - 1 - n0) * N;
   ef_d2_t ra[A_LD], rb[B_LD];
   // chunks past N read elements N - 1 and N (the operands' allocations end with at least
   // one element of padding)
@@ -260,16 +283,20 @@ __device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int b
   T* Fs = reinterpret_cast<T*>(lds);
   auto write = [&](int r0, int rows) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
+      const int rb = wave * (BM / 4) + i * 16 - r0;  // the same in the wave
+      if (rb + 16 <= 0 || rb >= rows) continue;
+      const int row = rb + (F32 ? 4 * kq : kq);
+      T* p = Fs + row * Tile::LDF + (lane & 15);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wave * (BM / 4) + i * 16 + (F32 ? 4 * kq + r : kq + 4 * r) - r0;
-        if ((unsigned)row < (unsigned)rows) {
+        constexpr int RS = F32 ? 1 : 4;
+        if ((unsigned)(row + RS * r) < (unsigned)rows) {
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-            Fs[row * Tile::LDF + j * 16 + (lane & 15)] = acc[i][j][r];
+          for (int j = 0; j < TN; ++j) p[RS * r * Tile::LDF + j * 16] = acc[i][j][r];
         }
       }
+    }
   };
   exchange_reduce<T>(Fs, Tile::LDF, n, min(x.gpt, x.G - g0), min(x.wpt, x.W - w0), w0,
                      x.xpart + (int64_t)gt * x.W, reinterpret_cast<cplx*>(lds + Tile::BODY),
@@ -278,19 +305,22 @@ __device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int b
 
 // split-bf16 tile 128 x 32 TN on v_mfma_f32_16x16x32_bf16 (2 x 2 waves, each 64 x 16 TN),
 // BK = 32; operand planes have K = Np32 (zero padded), so there is no k tail.  The operands
-// go from memory straight to LDS (16 bytes a lane, 16 rows an instruction), single
+// go from memory straight to LDS (16 bytes a lane, 8 rows an instruction), single
 // buffered: two or three workgroups share a CU, and one loads or reduces while the others
-// multiply.  Operand rows of 32 bf16 (64 B) have the chunk order c ^ ((r >> 1) & 3), as in
-// the split-bf16 GEMM, under which the 16-row operand reads meet no LDS bank conflicts; the
-// order is made by the address each lane loads from.
+// multiply.  LDS rows (32 hi, then 32 lo values) have the chunk order c ^ ((r >> 1) & 7), as
+// in the split-bf16 GEMM, under which the 16-row operand reads meet no LDS bank conflicts;
+// the order is made by the address each lane loads from.
 constexpr int EB_BM = 128, EB_BK = 32;
 template <int TN>
 struct EbTile {
-  static constexpr int BN = 32 * TN, LDF = BN + 1;
+  static constexpr int BN = 32 * TN;
+  // an odd number of entries, and rows 4 apart 24 banks apart: neither the reads down a
+  // column nor the stores of accumulators meet on a bank
+  static constexpr int LDF = BN + 6;
   static constexpr int OPS = 2 * (EB_BM + BN) * EB_BK * 2;
   static constexpr int F = (EX_FR * LDF * 4 + 15) / 16 * 16;
   static constexpr int BODY = OPS > F ? OPS : F;
-  static constexpr int LDS = BODY + EX_PARTS_BYTES;
+  static constexpr int LDS = BODY + 4 * EX_WMAX * (int)sizeof(cplx);
   static constexpr int WGS = TN <= 5 ? 3 : 2;  // workgroups per CU
   static_assert(WGS * LDS <= 160 * 1024, "workgroups per CU");
 };
@@ -298,8 +328,8 @@ struct EbTile {
 template <int TN>
 __device__ __forceinline__ void exchange_bf16x3_body(const ExchArgs& x, const int bx) {
   typedef EbTile<TN> Tile;
-  constexpr int BM = EB_BM, BN = Tile::BN, TM = 4, BK = EB_BK;
-  constexpr int LD = 4 + TN;  // loads per wave and k step: (8 + 2 TN) row groups, 2 planes
+  constexpr int BM = EB_BM, TM = 4, BK = EB_BK;
+  constexpr int LD = 4 + TN;  // loads per wave and k step: 16 + 4 TN row groups
   __shared__ __attribute__((aligned(16))) unsigned char lds[Tile::LDS];
 
   const int n = x.n, K = x.K;
@@ -311,24 +341,19 @@ __device__ __forceinline__ void exchange_bf16x3_body(const ExchArgs& x, const in
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wm = wave & 1, wn = wave >> 1;
 
-  // LDS: A hi, A lo (128 rows each), B hi, B lo (BN rows each), 1 KB per 16-row group.
-  // Group q of the wave's s-th load is wave + 4 s; rows past the operands read the last row
-  // (their products belong to no (g, w) block).
-  const uint16_t* src[LD];
-  int off[LD];
-  const int c0 = lane & 3, rl = lane >> 2;
-  const int ch = (c0 ^ ((rl >> 1) & 3)) * 8;
+  // LDS: the 128 rows of A, then the BN rows of B, 1 KB per group of 8 rows.  The wave's s-th
+  // load is group wave + 4 s; rows past the operands read the last row (their products
+  // belong to no (g, w) block).
+  const unsigned char* Ab = static_cast<const unsigned char*>(x.A) + 4 * (int64_t)m0 * K;
+  const unsigned char* Bb = static_cast<const unsigned char*>(x.B) + 4 * (int64_t)n0 * K;
+  uint32_t off[LD];
+  const int rl = lane >> 3;
 #pragma unroll
   for (int s = 0; s < LD; ++s) {
-    const int q = wave + 4 * s;
-    if (s < 4) {
-      src[s] = static_cast<const uint16_t*>(s < 2 ? x.A : x.Al) + (int64_t)m0 * K;
-      off[s] = min((q & 7) * 16 + rl, x.G * n - 1 - m0) * K + ch;
-    } else {
-      const int qb = q - 16, lo = qb >= 2 * TN ? 1 : 0;
-      src[s] = static_cast<const uint16_t*>(lo ? x.Bl : x.B) + (int64_t)n0 * K;
-      off[s] = min((qb - lo * 2 * TN) * 16 + rl, 2 * x.W * n - 1 - n0) * K + ch;
-    }
+    const int r = (wave + 4 * s) * 8 + rl;
+    const int row = s < 4 ? min(r, x.G * n - 1 - m0)
+                          : min(exchange_col_row(r - BM, n), 2 * x.W * n - 1 - n0);
+    off[s] = 4 * row * K + 16 * ((lane & 7) ^ ((r >> 1) & 7));
   }
 
   float4_t acc[TM][TN];
@@ -337,28 +362,29 @@ __device__ __forceinline__ void exchange_bf16x3_body(const ExchArgs& x, const in
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int koff = ((lane >> 4) ^ ((lane >> 1) & 3)) * 16;
-  const unsigned char* pa = lds + (wm * 64 + (lane & 15)) * 64 + koff;
-  const unsigned char* pb = lds + 2 * BM * 64 + (wn * 16 * TN + (lane & 15)) * 64 + koff;
+  // k chunk lane >> 4 of the hi values; of the lo values: chunk ^ 4
+  const int koff = ((lane >> 4) ^ ((lane >> 1) & 7)) * 16;
+  const unsigned char* pa = lds + (wm * 64 + (lane & 15)) * 128;
+  const unsigned char* pb = lds + (BM + wn * 16 * TN + (lane & 15)) * 128;
   for (int k0 = 0; k0 < K; k0 += BK) {
     if (k0) __syncthreads();  // the last step's operands are no longer read
 #pragma unroll
     for (int s = 0; s < LD; ++s)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src[s] + (off[s] + k0)),
+          (const __attribute__((address_space(1))) void*)((s < 4 ? Ab : Bb) + 4 * k0 + off[s]),
           (__attribute__((address_space(3))) void*)(lds + (wave + 4 * s) * 1024), 16, 0, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     bf16x8_t ah[TM], al[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      ah[i] = *reinterpret_cast<const bf16x8_t*>(pa + i * 1024);
-      al[i] = *reinterpret_cast<const bf16x8_t*>(pa + BM * 64 + i * 1024);
+      ah[i] = *reinterpret_cast<const bf16x8_t*>(pa + i * 2048 + koff);
+      al[i] = *reinterpret_cast<const bf16x8_t*>(pa + i * 2048 + (koff ^ 64));
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const bf16x8_t bh = *reinterpret_cast<const bf16x8_t*>(pb + j * 1024);
-      const bf16x8_t bl = *reinterpret_cast<const bf16x8_t*>(pb + BN * 64 + j * 1024);
+      const bf16x8_t bh = *reinterpret_cast<const bf16x8_t*>(pb + j * 2048 + koff);
+      const bf16x8_t bl = *reinterpret_cast<const bf16x8_t*>(pb + j * 2048 + (koff ^ 64));
 #pragma unroll
       for (int i = 0; i < TM; ++i)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[i][j], 0, 0, 0);
@@ -374,16 +400,19 @@ __device__ __forceinline__ void exchange_bf16x3_body(const ExchArgs& x, const in
   float* Fs = reinterpret_cast<float*>(lds);
   auto write = [&](int r0, int rows) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
+      const int rb = wm * 64 + i * 16 - r0;  // the same in the wave
+      if (rb + 16 <= 0 || rb >= rows) continue;
+      const int row = rb + 4 * (lane >> 4);
+      float* p = Fs + row * Tile::LDF + wn * 16 * TN + (lane & 15);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = wm * 64 + i * 16 + 4 * (lane >> 4) + r - r0;
-        if ((unsigned)row < (unsigned)rows) {
+        if ((unsigned)(row + r) < (unsigned)rows) {
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-            Fs[row * Tile::LDF + wn * 16 * TN + j * 16 + (lane & 15)] = acc[i][j][r];
+          for (int j = 0; j < TN; ++j) p[r * Tile::LDF + j * 16] = acc[i][j][r];
         }
       }
+    }
   };
   exchange_reduce<float>(Fs, Tile::LDF, n, min(x.gpt, x.G - g0), min(x.wpt, x.W - w0), w0,
                          x.xpart + (int64_t)gt * x.W,
@@ -508,9 +537,10 @@ ExchTile exchange_tile_for(const afqmc_ctx* c, int s) {
   if (n < 16) {
     x.tn = 8;
   } else {
+    const int fixed = c->mixed ? 0 : 2;
     x.tn = 8 * step;
     for (int tn = 8 * step; tn >= (c->mixed ? 4 : 5) * step; tn -= step)
-      if ((16 * tn / (2 * n)) * x.tn > (16 * x.tn / (2 * n)) * tn) x.tn = tn;
+      if ((16 * tn / (2 * n)) * (x.tn + fixed) > (16 * x.tn / (2 * n)) * (tn + fixed)) x.tn = tn;
   }
   x.bm = 128;
   if (!c->mixed) {
@@ -593,10 +623,8 @@ void exchange_plan(const afqmc_ctx* c, int s, int W, ExchArgs* a, int* kind, int
   if (c->mixed) {
     a->K = c->Np32;
     a->gc = exchange_chunk(a->g_tiles, (int64_t)a->gpt * n * c->Np32 * 4);
-    a->A = c->rot_chol_bf[s][0];
-    a->Al = c->rot_chol_bf[s][1];
-    a->B = c->green_bf[s][0];
-    a->Bl = c->green_bf[s][1];
+    a->A = c->rot_chol_bf[s];
+    a->B = c->green_bf[s];
   } else {
     a->K = N;
     a->gc = exchange_chunk(a->g_tiles, (int64_t)a->gpt * n * N * 8);

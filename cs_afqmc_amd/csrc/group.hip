@@ -118,8 +118,7 @@ int build(afqmc_group* g) {
         a.trial = c->trial[s];
         a.dets = c->dets;
         a.green = g->mixed ? nullptr : c->green[s];
-        a.ghi = g->mixed ? c->green_bf[s][0] : nullptr;
-        a.glo = g->mixed ? c->green_bf[s][1] : nullptr;
+        a.gbf = g->mixed ? c->green_bf[s] : nullptr;
         const auto key = std::make_pair(t2, stage);
         by_key[key].push_back({a, c->d.n_walkers});
         shm[key] = std::max(shm[key], sh);
@@ -167,10 +166,8 @@ int build(afqmc_group* g) {
         a.C = c->fb + (int64_t)s * 2 * W * G;
         if (g->mixed) {
           a.K = c->nocc[s] * c->Np32;
-          a.A = c->green_bf[s][0];
-          a.Al = c->green_bf[s][1];
-          a.B = c->rot_chol_bf[s][0];
-          a.Bl = c->rot_chol_bf[s][1];
+          a.A = c->green_bf[s];
+          a.B = c->rot_chol_bf[s];
         } else {
           a.K = c->kdim[s];
           a.A = c->green[s];
@@ -210,8 +207,7 @@ int build(afqmc_group* g) {
       a.mf = c->mf_shifts;
       a.fields = m.fields;
       a.xs = c->xs;
-      a.xs_hi = g->mixed ? c->xs_bf[0] : nullptr;
-      a.xs_lo = g->mixed ? c->xs_bf[1] : nullptr;
+      a.xs_bf = g->mixed ? c->xs_bf : nullptr;
       a.terms = c->terms;
       args.push_back(a);
       start.push_back(b);
@@ -244,10 +240,8 @@ int build(afqmc_group* g) {
         a.ldc = a.N;
         if (g->mixed) {
           a.K = c->Gp;
-          a.A = c->xs_bf[0];
-          a.Al = c->xs_bf[1];
-          a.B = chol_t_bf_of(c, 0, cs);
-          a.Bl = chol_t_bf_of(c, 1, cs);
+          a.A = c->xs_bf;
+          a.B = chol_t_bf_of(c, cs);
           a.C = vhs_f32_of(c, cs);
         } else {
           a.K = c->d.nchol;
@@ -410,8 +404,7 @@ int build(afqmc_group* g) {
           a.trial = c->trial[s];
           a.dets = c->dets;
           a.green = which == 1 ? c->green[s] : nullptr;
-          a.ghi = (which == 1 && c->mixed) ? c->green_bf[s][0] : nullptr;
-          a.glo = (which == 1 && c->mixed) ? c->green_bf[s][1] : nullptr;
+          a.gbf = (which == 1 && c->mixed) ? c->green_bf[s] : nullptr;
           const auto key = std::make_pair(t2, stage);
           by_key[key].push_back({a, c->d.n_walkers});
           shm[key] = std::max(shm[key], sh);

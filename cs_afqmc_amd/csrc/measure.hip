@@ -368,8 +368,7 @@ __device__ __forceinline__ void green_bf_load_b(const double* __restrict__ phid,
 template <int T2, int NW>
 __device__ __forceinline__ void green_bf_tiles(int N, int n, const double* __restrict__ phid,
                                                const cplx* M, int ld, const GjState* st,
-                                               uint16_t* __restrict__ gh,
-                                               uint16_t* __restrict__ gl, int ld16, int lane,
+                                               uint16_t* __restrict__ gbf, int ld16, int lane,
                                                int wv, double (&bpre)[GreenBf<T2>::KB][8]) {
   constexpr int KB = GreenBf<T2>::KB;
   const int n2 = 2 * n;
@@ -434,8 +433,9 @@ __device__ __forceinline__ void green_bf_tiles(int N, int n, const double* __res
         if (r < n2) {
           const float v = acc[tr][j];
           const uint16_t h = f32_to_bf16_rne(v);
-          gh[(int64_t)r * ld16 + p] = h;
-          gl[(int64_t)r * ld16 + p] = f32_to_bf16_rne(v - __uint_as_float((uint32_t)h << 16));
+          uint16_t* q = gbf + bf_pos((int64_t)r * ld16 + p);
+          q[0] = h;
+          q[BF_LO] = f32_to_bf16_rne(v - __uint_as_float((uint32_t)h << 16));
         }
       }
   }
@@ -453,8 +453,8 @@ __device__ __forceinline__ void green_bf_tiles(int N, int n, const double* __res
 template <int T2, int STAGE>
 __device__ __forceinline__ void measure_narrow_body(
     int N, int n, const cplx* __restrict__ walkers, const double* __restrict__ trial,
-    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ ghi,
-    uint16_t* __restrict__ glo, int ld16, const int w, const WeightsArgs& tail) {
+    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ gbf,
+    int ld16, const int w, const WeightsArgs& tail) {
   constexpr int NW = 2, TI = meas_ti(T2);
   constexpr int NKG = 4 * T2;  // k groups of 2n <= 16 T2
   extern __shared__ double smem[];
@@ -490,7 +490,7 @@ __device__ __forceinline__ void measure_narrow_body(
   // ---- O^-1 and det(O) (blocked in-place Gauss-Jordan, both waves); then
   // [Gr ; Gi] = [[Xr^T, -Xi^T], [Xi^T, Xr^T]] [wr^T ; wi^T], K = 2n, columns p in tiles
   // of 16, tiles split between the waves.
-  const bool want_green = green || ghi;
+  const bool want_green = green || gbf;
   const int tp_n = (N + 15) >> 4;
   // B[k][p] = re / im of w[p][k mod n]: 32-bit offsets within a walker row (tile
   // invariant), one row base per tile, clamped loads masked after
@@ -510,13 +510,12 @@ __device__ __forceinline__ void measure_narrow_body(
   double b[NKG];
   double bbf[GreenBf<T2>::KB][8];
   if (green && wv < tp_n) load_b(b, wv);
-  if (!green && ghi && wv < tp_n) green_bf_load_b<T2>(phid, N, n, wv, lane, bbf);
+  if (!green && gbf && wv < tp_n) green_bf_load_b<T2>(phid, N, n, wv, lane, bbf);
   gj_invert<NW, 2>(M, ld, n, st, lane, wv);
   if (threadIdx.x == 0) finish_walker(st->det, dets, w, spin, tail);
   if (!want_green) return;
   if (!green) {  // split-bf16 planes only (mixed mode's step)
-    green_bf_tiles<T2, NW>(N, n, phid, M, ld, st, ghi + (int64_t)w * n2 * ld16,
-                           glo + (int64_t)w * n2 * ld16, ld16, lane, wv, bbf);
+    green_bf_tiles<T2, NW>(N, n, phid, M, ld, st, gbf + 2 * (int64_t)w * n2 * ld16, ld16, lane, wv, bbf);
     return;
   }
 
@@ -546,8 +545,7 @@ __device__ __forceinline__ void measure_narrow_body(
       a[kg][tr] = k < n2 ? v : 0.0;  // (rows r >= 2n are not stored)
     }
   double* gw = green ? green + (int64_t)w * n2 * N : nullptr;
-  uint16_t* gh = ghi ? ghi + (int64_t)w * n2 * ld16 : nullptr;
-  uint16_t* gl = ghi ? glo + (int64_t)w * n2 * ld16 : nullptr;
+  uint16_t* gb = gbf ? gbf + 2 * (int64_t)w * n2 * ld16 : nullptr;
   // tile tp; the walker operand of tile tp + NW loads into b once the MFMAs have read it
   auto tile = [&](int tp) {
     double4_t acc[T2];
@@ -563,8 +561,7 @@ __device__ __forceinline__ void measure_narrow_body(
     const int p = tp * 16 + col;
     if (p >= N) return;
     double* gwp = gw ? gw + (int64_t)s * N + p : nullptr;
-    uint16_t* ghp = gh ? gh + (int64_t)s * ld16 + p : nullptr;
-    uint16_t* glp = gh ? gl + (int64_t)s * ld16 + p : nullptr;
+    uint16_t* gbp = gb ? gb + bf_pos((int64_t)s * ld16 + p) : nullptr;
 #pragma unroll
     for (int tr = 0; tr < T2; ++tr)
 #pragma unroll
@@ -572,7 +569,10 @@ __device__ __forceinline__ void measure_narrow_body(
         const int r0 = tr * 16 + 4 * q;
         if (r0 + s < n2) {
           if (gwp) gwp[(int64_t)r0 * N] = acc[tr][q];
-          if (ghp) split_bf16(acc[tr][q], &ghp[(int64_t)r0 * ld16], &glp[(int64_t)r0 * ld16]);
+          if (gbp) {
+            uint16_t* e = gbp + 2 * (int64_t)r0 * ld16;
+            split_bf16(acc[tr][q], e, e + BF_LO);
+          }
         }
       }
   };
@@ -614,8 +614,8 @@ constexpr size_t mw_bytes(int t2, int n) { return mw_region(t2, n) + 256 * sizeo
 template <int T2>
 __device__ __forceinline__ void measure_wide_body(
     int N, int n, const cplx* __restrict__ walkers, const double* __restrict__ trial,
-    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ ghi,
-    uint16_t* __restrict__ glo, int ld16, const int w, const WeightsArgs& tail) {
+    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ gbf,
+    int ld16, const int w, const WeightsArgs& tail) {
   constexpr int NW = 4, NT = 64 * NW, KC = MW_KC;
   constexpr int PS = mw_ps(T2), TS = mw_ts(T2);
   constexpr int TIM = (T2 + 1) / 2;             // row tiles of O at most
@@ -718,7 +718,7 @@ __device__ __forceinline__ void measure_wide_body(
   // ---- O^-1 and det(O): blocked in-place Gauss-Jordan on all four waves
   gj_invert<NW, TIM>(M, ld, n, st, lane, wv);
   const cplx det = st->det;
-  if (!(green || ghi)) {
+  if (!(green || gbf)) {
     if (tid == 0) finish_walker(det, dets, w, spin, tail);
     return;
   }
@@ -751,8 +751,7 @@ __device__ __forceinline__ void measure_wide_body(
   // ---- [Gr ; Gi] = [[Xr^T, -Xi^T], [Xi^T, Xr^T]] [wr^T ; wi^T], K = 2n, columns p; the
   // waves take alternate column tiles
   double* gw = green ? green + (int64_t)w * n2 * N : nullptr;
-  uint16_t* gh = ghi ? ghi + (int64_t)w * n2 * ld16 : nullptr;
-  uint16_t* gl = ghi ? glo + (int64_t)w * n2 * ld16 : nullptr;
+  uint16_t* gb = gbf ? gbf + 2 * (int64_t)w * n2 * ld16 : nullptr;
   const int tp_n = (N + 15) >> 4, nkg = (n + 3) >> 2;
   const double* P0 = P + s * PS + col;  // + 16 tr: row k < n of A
   const double* P1[T2];                 // row n + k of A, before its sign
@@ -806,7 +805,7 @@ __device__ __forceinline__ void measure_wide_body(
         const int row = tr * 16 + s + 4 * q;
         if (row < n2) {
           if (gw) gw[(int64_t)row * N + p] = acc[tr][q];
-          if (gh) split_bf16(acc[tr][q], &gh[(int64_t)row * ld16 + p], &gl[(int64_t)row * ld16 + p]);
+          if (gb) store_split_bf16(gb, (int64_t)row * ld16 + p, acc[tr][q]);
         }
       }
   }
@@ -815,13 +814,13 @@ __device__ __forceinline__ void measure_wide_body(
 template <int T2, int TI, int STAGE>
 __global__ __launch_bounds__(64 * meas_waves(T2), meas_wpe(T2)) void measure_kernel(
     int N, int n, const cplx* __restrict__ walkers, const double* __restrict__ trial,
-    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ ghi,
-    uint16_t* __restrict__ glo, int ld16, WeightsArgs tail) {
+    cplx* __restrict__ dets, int spin, double* __restrict__ green, uint16_t* __restrict__ gbf,
+    int ld16, WeightsArgs tail) {
   if constexpr (T2 <= 3)
-    measure_narrow_body<T2, STAGE>(N, n, walkers, trial, dets, spin, green, ghi, glo, ld16,
+    measure_narrow_body<T2, STAGE>(N, n, walkers, trial, dets, spin, green, gbf, ld16,
                                    blockIdx.x, tail);
   else
-    measure_wide_body<T2>(N, n, walkers, trial, dets, spin, green, ghi, glo, ld16, blockIdx.x,
+    measure_wide_body<T2>(N, n, walkers, trial, dets, spin, green, gbf, ld16, blockIdx.x,
                           tail);
 }
 
@@ -834,9 +833,9 @@ __global__ __launch_bounds__(64 * meas_waves(T2), meas_wpe(T2)) void measure_gro
   const WeightsArgs none{};
   if constexpr (T2 <= 3)
     measure_narrow_body<T2, STAGE>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin, a.green,
-                                   a.ghi, a.glo, a.ld16, blockIdx.x - start[p], none);
+                                   a.gbf, a.ld16, blockIdx.x - start[p], none);
   else
-    measure_wide_body<T2>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin, a.green, a.ghi, a.glo,
+    measure_wide_body<T2>(a.N, a.n, a.walkers, a.trial, a.dets, a.spin, a.green, a.gbf,
                           a.ld16, blockIdx.x - start[p], none);
 }
 
@@ -873,8 +872,8 @@ int launch_measure_s(afqmc_ctx* c, int W, int n, const cplx* wk, int s, bool g64
   if (rc) return rc;
   hipLaunchKernelGGL((measure_kernel<T2, TI, STAGE>), dim3(W), dim3(64 * meas_waves(T2)), shm,
                      c->stream, c->d.norb, n, wk, c->trial[s], c->dets, s,
-                     g64 ? c->green[s] : nullptr, gbf ? c->green_bf[s][0] : nullptr,
-                     gbf ? c->green_bf[s][1] : nullptr, c->Np32, tail);
+                     g64 ? c->green[s] : nullptr, gbf ? c->green_bf[s] : nullptr,
+                     c->Np32, tail);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }

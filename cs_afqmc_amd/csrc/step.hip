@@ -65,7 +65,7 @@ template <int NT>
 __device__ __forceinline__ void fields_body(
     int G, double sqdt, const double* __restrict__ fb, int nparts, int64_t part_stride,
     const cplx* __restrict__ mf, const double* __restrict__ fields, double* __restrict__ xs,
-    uint16_t* __restrict__ xs_hi, uint16_t* __restrict__ xs_lo, int Gp,
+    uint16_t* __restrict__ xs_bf, int Gp,
     cplx* __restrict__ terms, cplx* __restrict__ fb_out, const int w) {
   constexpr int VT = FIELDS_NT;  // threads whose summation order is kept
   constexpr int R = VT / NT;     // virtual threads per thread
@@ -93,11 +93,11 @@ __device__ __forceinline__ void fields_body(
       // fields * field_shifts - field_shifts * field_shifts / 2
       const cplx fs2 = cmul(fs, fs);
       ft[r] = cadd(ft[r], cplx{xv * fs.re - fs2.re / 2.0, xv * fs.im - fs2.im / 2.0});
-      // VHS operand: 1j * sqrt(dt) * shifted_fields (float64, or split-bf16 planes)
-      if (xs_hi) {
+      // VHS operand: 1j * sqrt(dt) * shifted_fields (float64 or split-bf16)
+      if (xs_bf) {
         const int64_t o = (int64_t)w * 2 * Gp + g;
-        split_bf16(-sqdt * xt.im, &xs_hi[o], &xs_lo[o]);
-        split_bf16(sqdt * xt.re, &xs_hi[o + Gp], &xs_lo[o + Gp]);
+        store_split_bf16(xs_bf, o, -sqdt * xt.im);
+        store_split_bf16(xs_bf, o + Gp, sqdt * xt.re);
       } else {
         xr[g] = -sqdt * xt.im;
         xi[g] = sqdt * xt.re;
@@ -143,9 +143,9 @@ template <int NT>
 __global__ __launch_bounds__(NT) void fields_kernel(
     int G, double sqdt, const double* __restrict__ fb, int nparts, int64_t part_stride,
     const cplx* __restrict__ mf, const double* __restrict__ fields, double* __restrict__ xs,
-    uint16_t* __restrict__ xs_hi, uint16_t* __restrict__ xs_lo, int Gp,
+    uint16_t* __restrict__ xs_bf, int Gp,
     cplx* __restrict__ terms, cplx* __restrict__ fb_out) {
-  fields_body<NT>(G, sqdt, fb, nparts, part_stride, mf, fields, xs, xs_hi, xs_lo, Gp, terms,
+  fields_body<NT>(G, sqdt, fb, nparts, part_stride, mf, fields, xs, xs_bf, Gp, terms,
                   fb_out, blockIdx.x);
 }
 
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(NT) void fields_grouped_kernel(
   const int p = group_of(start, nprob, blockIdx.x);
   const FieldsArgs a = args[p];
   fields_body<NT>(a.G, a.sqdt, a.fb, a.nparts, a.part_stride, a.mf,
-                  a.fields + (int64_t)step * a.W * a.G, a.xs, a.xs_hi, a.xs_lo, a.Gp, a.terms,
+                  a.fields + (int64_t)step * a.W * a.G, a.xs, a.xs_bf, a.Gp, a.terms,
                   nullptr, blockIdx.x - start[p]);
 }
 
@@ -312,8 +312,7 @@ int launch_fields(afqmc_ctx* c, int W, const double* fields, cplx* fb_out) {
   const auto kern = fields_nt(W) == 64 ? fields_kernel<64> : fields_kernel<FIELDS_NT>;
   hipLaunchKernelGGL(kern, dim3(W), dim3(fields_nt(W)), 0, c->stream, c->d.nchol,
                      sqrt(c->d.dt), c->fb, c->fb_parts, (int64_t)2 * W * c->d.nchol, c->mf_shifts,
-                     fields, c->xs, c->mixed ? c->xs_bf[0] : nullptr,
-                     c->mixed ? c->xs_bf[1] : nullptr, c->Gp, c->terms, fb_out);
+                     fields, c->xs, c->mixed ? c->xs_bf : nullptr, c->Gp, c->terms, fb_out);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }
