@@ -13,6 +13,7 @@ AFQMC_RHF = 1
 AFQMC_UHF = 2
 AFQMC_UHF_SPIN_CHOL = 3
 AFQMC_STEP_REUSE_GREEN = 1
+AFQMC_STEP_NO_GREEN = 2
 AFQMC_SR_GLOBAL_ORDER = 1
 BLOCK_STATS_LEN = 4  # AFQMC_BLOCK_STATS_LEN: block energy, weight, zero weights, clamped
 PRECISIONS = {"fp64": 0, "fp32": 1, "bf16x3": 2}

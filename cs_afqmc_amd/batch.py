@@ -135,7 +135,8 @@ class Fragment:
         pd = self.prop_data
         for s in range(self.n_prop_steps):
             self.dev.propagate(pd["walkers"], pd["weights"], pd["overlaps"], self.fields[s],
-                               self.scalars, reuse_green=s > 0)
+                               self.scalars, reuse_green=s > 0,
+                               keep_green=s + 1 < self.n_prop_steps)
 
     def _block_single(self):
         self.begin_block()

@@ -96,7 +96,8 @@ class CorrelatedPair:
             for sy in self.s:
                 for s in range(self.n_prop_steps):
                     sy.dev.propagate(sy.pd["walkers"], sy.pd["weights"], sy.pd["overlaps"],
-                                     self.fields[s], sy.scalars, reuse_green=s > 0)
+                                     self.fields[s], sy.scalars, reuse_green=s > 0,
+                                     keep_green=s + 1 < self.n_prop_steps)
         ens = [_field_block_end(sy) for sy in self.s]
         a, b = self.s
         a.dev.cs_outliers(a.pd["weights"], b.pd["weights"], self.z_thresh)

@@ -426,11 +426,12 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
   }
   {
     // new overlaps and each walker's weight update; the Green's function of the new
-    // walkers is kept for the next step
+    // walkers is kept for the next step unless no step will reuse it
+    const bool keep = !(flags & AFQMC_STEP_NO_GREEN);
     PhaseTimer t(c, AFQMC_PH_OVERLAP);
     const WeightsArgs tail = weights_args(c, W, weights, static_cast<cplx*>(overlaps), scalars);
-    if ((rc = launch_measure(c, W, wu, wd, !c->mixed, c->mixed, &tail))) return rc;
-    c->green_src = walkers_up;
+    if ((rc = launch_measure(c, W, wu, wd, keep && !c->mixed, keep && c->mixed, &tail))) return rc;
+    if (keep) c->green_src = walkers_up;
     c->green_w = W;
   }
   // population-control shift from the summed weights

@@ -165,7 +165,6 @@ __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_use
 constexpr int EF_BK = 16;
 typedef double ef_d2u_t __attribute__((ext_vector_type(2), aligned(8)));
 typedef double ef_d2_t __attribute__((ext_vector_type(2)));
-typedef float ef_f2_t __attribute__((ext_vector_type(2)));
 typedef float ef_f4_t __attribute__((ext_vector_type(4)));
 
 template <bool F32, int BM, int TN>
@@ -223,9 +222,11 @@ __device__ __forceinline__ void exchange_f64_body(const ExchArgs& x, const int b
     const bool ok0 = k0 + 2 * lch < N, ok1 = k0 + 2 * lch + 1 < N;
     auto put = [&](int row, ef_d2_t v) {  // (32-row steps leave the swizzle unchanged)
       if constexpr (F32) {
-        const int c = (lch >> 1) ^ ((lr >> 1) & 3);
-        reinterpret_cast<ef_f2_t*>(ops + buf * BUF + row * RCH)[c * 2 + (lch & 1)] =
-            ef_f2_t{ok0 ? (float)v.x : 0.f, ok1 ? (float)v.y : 0.f};
+        // element e of chunk c is k = 4 e + c: each MFMA sums four consecutive k
+        float* p = reinterpret_cast<float*>(ops + buf * BUF + row * RCH);
+        const int c = (2 * lch) & 3, sw = (lr >> 1) & 3;
+        p[(c ^ sw) * 4 + (lch >> 1)] = ok0 ? (float)v.x : 0.f;
+        p[((c + 1) ^ sw) * 4 + (lch >> 1)] = ok1 ? (float)v.y : 0.f;
       } else {
         ops[buf * BUF + row * RCH + (lch ^ ((lr >> 1) & 7))] =
             ef_d2_t{ok0 ? v.x : 0.0, ok1 ? v.y : 0.0};

@@ -132,10 +132,11 @@ __device__ __forceinline__ void gj_panel(cplx* B, int ld, int n, int k0, int pb,
 //   x <- T x[R_K] + (x with the rows R_K cleared),  T = the panel's columns,
 // four real MFMAs per 16 x 16 tile.  On return B holds S with
 //   O^-1[i][j] = S[rho[i]][rhoinv[j]],
-// and st->det = det(O).  Ends with a barrier.
+// and st->det = det(O).  Ends with a barrier.  With det_only, column blocks that no later
+// panel reads are left as they are (the same pivots, hence the same det; no inverse).
 template <int NW, int TT>
-__device__ __forceinline__ void gj_invert(cplx* B, int ld, int n, GjState* st, int lane,
-                                          int wv) {
+__device__ __forceinline__ void gj_invert(cplx* B, int ld, int n, GjState* st, int lane, int wv,
+                                          bool det_only) {
   const int tid = threadIdx.x;
   if (tid < 64) st->vrow[tid] = tid;
   if (tid == 0) {
@@ -151,7 +152,7 @@ __device__ __forceinline__ void gj_invert(cplx* B, int ld, int n, GjState* st, i
     const int pb = min(GJ_PB, n - k0);
     if (wv == (k0 >> 4)) gj_panel(B, ld, n, k0, pb, panel, st, lane);
     lds_barrier();
-    if (!mine) continue;
+    if (!mine || (det_only && 16 * (wv + 1) <= k0 + pb)) continue;
     // loads clamped into the matrix and masked after, so they issue back to back
     const unsigned long long pm = st->pmask[panel & 1];
     const bool kok = kk < pb, cok = cb < n;
@@ -511,7 +512,7 @@ __device__ __forceinline__ void measure_narrow_body(
   double bbf[GreenBf<T2>::KB][8];
   if (green && wv < tp_n) load_b(b, wv);
   if (!green && gbf && wv < tp_n) green_bf_load_b<T2>(phid, N, n, wv, lane, bbf);
-  gj_invert<NW, 2>(M, ld, n, st, lane, wv);
+  gj_invert<NW, 2>(M, ld, n, st, lane, wv, !want_green);
   if (threadIdx.x == 0) finish_walker(st->det, dets, w, spin, tail);
   if (!want_green) return;
   if (!green) {  // split-bf16 planes only (mixed mode's step)
@@ -716,7 +717,7 @@ __device__ __forceinline__ void measure_wide_body(
   }
 
   // ---- O^-1 and det(O): blocked in-place Gauss-Jordan on all four waves
-  gj_invert<NW, TIM>(M, ld, n, st, lane, wv);
+  gj_invert<NW, TIM>(M, ld, n, st, lane, wv, !(green || gbf));
   const cplx det = st->det;
   if (!(green || gbf)) {
     if (tid == 0) finish_walker(det, dets, w, spin, tail);

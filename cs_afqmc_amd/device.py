@@ -213,9 +213,10 @@ class DeviceStep:
 
     # ------------------------------------------------------------------ entry points
     def propagate(self, walkers, weights, overlaps, fields, scalars, force_bias_out=None,
-                  reuse_green=False):
+                  reuse_green=False, keep_green=True):
         """reuse_green: the walkers are those the previous propagate on this context
-        returned (no QR / SR / edits since), so its Green's function is reused."""
+        returned (no QR / SR / edits since), so its Green's function is reused.
+        keep_green: the next propagate may reuse this one's Green's function."""
         up, dn, W = self._walkers(walkers)
         self._vec(weights, W, torch.float64, "weights")
         self._vec(overlaps, W, torch.complex128, "overlaps")
@@ -229,7 +230,8 @@ class DeviceStep:
         _lib.check(self._lib.afqmc_propagate(
             self._h, W, _dptr(up), _dptr(dn), _dptr(weights), _dptr(overlaps), _dptr(fields),
             _dptr(scalars), _dptr(force_bias_out),
-            _lib.AFQMC_STEP_REUSE_GREEN if reuse_green else 0))
+            (_lib.AFQMC_STEP_REUSE_GREEN if reuse_green else 0)
+            | (0 if keep_green else _lib.AFQMC_STEP_NO_GREEN)))
 
     def overlap(self, walkers, out=None):
         up, dn, W = self._walkers(walkers)

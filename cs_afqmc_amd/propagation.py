@@ -144,8 +144,9 @@ class propagator_restricted:
             _scalar_tensor(prop_data["e_estimate"], dev.device),
             _scalar_tensor(prop_data["pop_control_ene_shift"], dev.device),
         ]).contiguous()
+        # the walkers may be edited before the next step, which starts from them alone
         dev.propagate(walkers, prop_data["weights"], prop_data["overlaps"], fields, scalars,
-                      force_bias_out)
+                      force_bias_out, keep_green=False)
         prop_data["pop_control_ene_shift"] = scalars[1]
         return prop_data
 

@@ -57,7 +57,7 @@ class _BlockState:
         dev.fields_normal_key(self.key, self.fields)
         for s in range(self.n_prop_steps):
             dev.propagate(self.walkers, self.weights, self.overlaps, self.fields[s], self.scalars,
-                          reuse_green=s > 0)
+                          reuse_green=s > 0, keep_green=s + 1 < self.n_prop_steps)
         dev.orthonormalize(self.walkers)
         dev.overlap(self.walkers, out=self.overlaps)
         en = dev.energy(self.walkers, out=self.energies)

@@ -121,9 +121,12 @@ AFQMC_API const char* afqmc_last_error(void);
  *   flags          AFQMC_STEP_REUSE_GREEN: the walkers are exactly those the previous
  *                  afqmc_propagate on this context returned, so the Green's function
  *                  it left in the workspace is reused for the force bias (the library
- *                  also requires the same walker pointer and count, else recomputes)
+ *                  also requires the same walker pointer and count, else recomputes);
+ *                  AFQMC_STEP_NO_GREEN: no later step will reuse the new walkers' Green's
+ *                  function, so only their overlaps are computed (a later
+ *                  AFQMC_STEP_REUSE_GREEN recomputes it)
  * n_walkers may be smaller than the context's workspace size. */
-enum { AFQMC_STEP_REUSE_GREEN = 1 };
+enum { AFQMC_STEP_REUSE_GREEN = 1, AFQMC_STEP_NO_GREEN = 2 };
 AFQMC_API int afqmc_propagate(afqmc_ctx* ctx, int32_t n_walkers, void* walkers_up,
                     void* walkers_dn, double* weights, void* overlaps,
                     const double* fields, double* scalars, void* force_bias_out,
