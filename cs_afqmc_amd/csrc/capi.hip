@@ -81,7 +81,7 @@ void free_ctx(afqmc_ctx* c) {
                   c->rot_chol_bf[0], c->rot_chol_bf[1], c->green[0], c->green[1], c->fb,
                   c->xs, c->vhs, c->terms, c->dets, c->energy_x, c->energy_acc, c->walk_tmp,
                   c->sr_cum, c->sr_idx, c->xs_bf, c->green_bf[0], c->green_bf[1],
-                  c->vhs_f32, c->sym_stat};
+                  c->vhs_f32, c->sym_stat, c->step_arrived};
   prof_free(&c->prof);
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -340,6 +340,8 @@ extern "C" int afqmc_ctx_create(afqmc_ctx** out, const afqmc_dims* dims,
       TRY(dalloc(c, &c->energy_x, tiles * W));
     }
     TRY(dalloc(c, &c->walk_tmp, (size_t)W * N * (c->nocc[0] > c->nocc[1] ? c->nocc[0] : c->nocc[1])));
+    TRY(dalloc(c, &c->step_arrived, 1));
+    TRY(zero_async(c->step_arrived, sizeof(int), c->stream));
     TRY(dalloc(c, &c->sr_cum, (size_t)W));
     TRY(dalloc(c, &c->sr_idx, (size_t)W));
     TRY(sync_stream(c->stream));
@@ -390,7 +392,15 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
   // then the rot_chol contraction
   const bool reuse = (flags & AFQMC_STEP_REUSE_GREEN) && c->green_src == walkers_up &&
                      c->green_w == W;
+  const bool keep = !(flags & AFQMC_STEP_NO_GREEN);
+  const WeightsArgs tail = weights_args(c, W, weights, static_cast<cplx*>(overlaps), scalars);
   c->green_src = nullptr;
+  if (!c->prof.on && !force_bias_out && small_step_fits(c, W)) {
+    if ((rc = launch_small_step(c, W, wu, wd, fields, tail, reuse, keep))) return rc;
+    if (keep) c->green_src = walkers_up;
+    c->green_w = W;
+    return AFQMC_OK;
+  }
   if (!reuse) {
     PhaseTimer t(c, AFQMC_PH_GREEN);
     if ((rc = launch_measure(c, W, wu, wd, !c->mixed, c->mixed))) return rc;
@@ -427,9 +437,7 @@ extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* 
   {
     // new overlaps and each walker's weight update; the Green's function of the new
     // walkers is kept for the next step unless no step will reuse it
-    const bool keep = !(flags & AFQMC_STEP_NO_GREEN);
     PhaseTimer t(c, AFQMC_PH_OVERLAP);
-    const WeightsArgs tail = weights_args(c, W, weights, static_cast<cplx*>(overlaps), scalars);
     if ((rc = launch_measure(c, W, wu, wd, keep && !c->mixed, keep && c->mixed, &tail))) return rc;
     if (keep) c->green_src = walkers_up;
     c->green_w = W;

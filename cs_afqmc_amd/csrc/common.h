@@ -271,6 +271,7 @@ struct afqmc_ctx {
   double* vhs;           // chol_spins x (W, 2, vhs_nv), + padding
   cplx* terms;           // (W, 2): shift_term, fb_term
   cplx* dets;            // (W, 2): det(C_sigma^H w_sigma)
+  int* step_arrived;     // workgroups of a small_step launch that are done
   cplx* energy_x;        // (sum_s g_tiles_s, W) exchange partial sums
   cplx* energy_acc;      // (W): partial energies
   cplx* walk_tmp;        // gather target for SR (W * N * n_max)
@@ -392,6 +393,10 @@ int launch_split_bf16(hipStream_t s, int rows, int cols, const double* x, int64_
 // each walker's block); the population-control shift then comes from launch_pcs.
 int launch_measure(afqmc_ctx* c, int W, const cplx* wup, const cplx* wdn, bool green_f64,
                    bool green_bf = false, const WeightsArgs* tail = nullptr);
+// measure.hip: a whole float64 step in one launch, and whether that is the better way
+bool small_step_fits(const afqmc_ctx* c, int W);
+int launch_small_step(afqmc_ctx* c, int W, cplx* wup, cplx* wdn, const double* fields,
+                      const WeightsArgs& tail, bool reuse, bool keep);
 // taylor.hip
 int launch_taylor(afqmc_ctx* c, int W, cplx* wup, cplx* wdn);
 // step.hip

@@ -958,3 +958,465 @@ void measure_plan(const afqmc_ctx* c, int s, int* t2, int* stage, size_t* shm) {
   *stage = 0;
   *shm = mw_bytes(*t2, n);
 }
+
+// ------------------------------------------------------------------------------------
+// A whole float64 step of small problems, one workgroup per walker: Green's function (unless
+// the last step left it), force bias and fields, V, Taylor, the new overlaps and the weight
+// update, and in the workgroup that finishes last the population-control shift.
+//
+// What it is for: an H10 chain's step (norb 10, n = 5, 27 vectors, 200 walkers) is seven
+// launches of 3.5 to 9 us, each a chain of dependent loads on a mostly idle chip, plus the
+// gaps between them.  Everything but the shift is per walker, and a walker's intermediates
+// fit LDS; the price is that every walker reads the Cholesky vectors itself (small_step_fits
+// has the line).  The chain is what bounds it, so four lanes share every sum (their partial
+// sums meet in the quad), what is read from memory is asked for ahead of its use, and O
+// (n <= 8) is inverted in the registers of one wave while the others wait or multiply.
+namespace {
+
+struct SmallStep {
+  int W, N, G, nspin, chol_spins, terms_k, nv, mult, reuse, keep;
+  int n[2];
+  double dt, sqdt;
+  const double* trial[2];
+  const double* rot[2];
+  const double* chol_t;
+  const double* E[2];
+  const cplx* mf;
+  cplx* walkers[2];
+  double* green[2];
+  const double* fields;
+  WeightsArgs tail;
+  int* arrived;  // workgroups done, 0 between launches
+};
+
+constexpr int SMALL_NT = 256, SMALL_MAX_N = 32, SMALL_MAX_OCC = 8;
+constexpr int SMALL_R = SMALL_MAX_N * SMALL_MAX_OCC * 4 / SMALL_NT;  // sums per quad
+
+// lane ^ 1 and lane ^ 2 of a quad
+template <int CTRL>
+__device__ inline double quad_dpp(double x) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)u, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ inline double quad_sum(double x) {
+  x += quad_dpp<0xB1>(x);         // quad_perm [1, 0, 3, 2]
+  return x + quad_dpp<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+}
+
+// det(O) and, with full, X = O^-1 of the n x n matrix at O (rows of SMALL_MAX_OCC, LDS), by
+// one wave: lane j holds column j of O, lane 8 + j column j of the unit matrix; Gauss-Jordan
+// with row exchanges, pivots by largest |re| + |im|.
+__device__ __forceinline__ cplx small_invert(const cplx* O, cplx* X, int n, bool full, int lane) {
+  constexpr int M = SMALL_MAX_OCC;
+  cplx c[M];
+#pragma unroll
+  for (int r = 0; r < M; ++r) {
+    const cplx o = O[r * M + (lane & 7)];
+    c[r] = lane < M ? o : cplx{lane - M == r ? 1.0 : 0.0, 0.0};
+  }
+  cplx det = {1.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    if (k >= n) continue;
+    cplx p[M];  // column k, the same in all lanes
+#pragma unroll
+    for (int r = 0; r < M; ++r)
+      if (r >= k || full) p[r] = readlane_c(c[r], k);
+    int pr = k;
+    double best = fabs(p[k].re) + fabs(p[k].im);
+#pragma unroll
+    for (int r = k + 1; r < M; ++r) {
+      const double a = fabs(p[r].re) + fabs(p[r].im);
+      if (r < n && a > best) {
+        best = a;
+        pr = r;
+      }
+    }
+    pr = __builtin_amdgcn_readfirstlane(pr);
+#pragma unroll
+    for (int r = k + 1; r < M; ++r)
+      if (r == pr) {
+        const cplx a = c[k], b = p[k];
+        c[k] = c[r];
+        c[r] = a;
+        p[k] = p[r];
+        p[r] = b;
+      }
+    det = cmul(det, p[k]);
+    if (pr != k) det = cplx{-det.re, -det.im};
+    const double d2 = rcp_f64(p[k].re * p[k].re + p[k].im * p[k].im);
+    c[k] = cmul(c[k], cplx{p[k].re * d2, -p[k].im * d2});
+#pragma unroll
+    for (int r = 0; r < M; ++r)
+      if (r != k && r < n && (r > k || full)) c[r] = csub(c[r], cmul(p[r], c[k]));
+  }
+  if (full && lane >= M && lane < M + n) {
+#pragma unroll
+    for (int r = 0; r < M; ++r)
+      if (r < n) X[r * M + lane - M] = c[r];
+  }
+  return det;
+}
+
+// walker_weight_update on two lanes: the importance function on even, the phase on odd ones
+__device__ __forceinline__ void small_weight(const WeightsArgs& a, double pcs, int w, cplx onew,
+                                             cplx st, cplx ft, cplx oold, double wold, int lane) {
+  const bool phase = lane & 1;
+  const cplx e = phase ? cplx{-a.sqdt * st.re, -a.sqdt * st.im}
+                       : cplx{-a.sqdt * st.re + ft.re + a.dt * (pcs + a.h0_prop),
+                              -a.sqdt * st.im + ft.im};
+  const cplx z = cdiv(cmul(cexp_(e), onew), oold);
+  const double f = phase ? cos(atan2(z.im, z.re)) : hypot(z.re, z.im);
+  const double g = quad_dpp<0xB1>(f);
+  if (lane == 0) {
+    double ipl = f * g;
+    if (isnan(ipl)) ipl = 0.0;
+    if (ipl < 1.0e-3) ipl = 0.0;
+    if (ipl > 100.0) ipl = 0.0;
+    double wt = ipl * wold;
+    if (wt > 100.0) wt = 0.0;
+    // (written through: the last workgroup reads it, possibly on another XCD)
+    __hip_atomic_store(a.weights + w, wt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    a.overlaps[w] = onew;
+  }
+}
+
+// doubles of LDS: Green's functions, x, V, walker, E and trial of a spin, O and X
+__host__ __device__ inline int small_doubles(int N, int n0, int n1, int G) {
+  const int n = n0 > n1 ? n0 : n1;
+  return 2 * N * (n0 + n1) + 2 * G + 2 * N * N + 2 * N * n + N * N + N * n +
+         4 * SMALL_MAX_OCC * SMALL_MAX_OCC;
+}
+
+__global__ __launch_bounds__(SMALL_NT, 2) void small_step_kernel(SmallStep a) {
+  constexpr int M = SMALL_MAX_OCC;
+  extern __shared__ double smem[];
+  __shared__ double red[4 * (SMALL_NT / 64)];
+  __shared__ cplx dets[2];
+  __shared__ int last;
+  const int t = threadIdx.x, lane = t & 63, w = blockIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), q4 = t & 3;
+  const int N = a.N, G = a.G, nm = max(a.n[0], a.n[1]);
+
+  // the walker's Green's functions [re / im][i][p]
+  auto gl = [&](int s) { return smem + (s ? 2 * N * a.n[0] : 0); };
+  cplx* V = reinterpret_cast<cplx*>(gl(1) + 2 * N * a.n[1]);
+  cplx* y = V + N * N;
+  cplx* O = y + N * nm;
+  cplx* X = O + M * M;
+  double* E = reinterpret_cast<double*>(X + M * M);
+  double* C = E + N * N;
+  double* xr = C + N * nm;
+  double* xi = xr + G;
+
+  auto stage_walker = [&](int s) {
+    const int c = N * a.n[s];
+    const cplx* phi = a.walkers[s] + (int64_t)w * c;
+    for (int o = t; o < c; o += SMALL_NT) y[o] = phi[o];
+  };
+  auto stage_trial = [&](int s) {
+    const int c = N * a.n[s];
+    for (int o = t; o < c; o += SMALL_NT) C[o] = a.trial[s][o];
+  };
+  // O = C^T y, four lanes per entry (n^2 <= 64 entries)
+  auto overlap = [&](int n) {
+    const int e = t >> 2, i = e / n, j = e - i * n;
+    cplx z = {0.0, 0.0};
+    if (i < n)
+      for (int p = q4; p < N; p += 4) {
+        const double v = C[p * n + i];
+        const cplx b = y[p * n + j];
+        z.re = fma(v, b.re, z.re);
+        z.im = fma(v, b.im, z.im);
+      }
+    z.re = quad_sum(z.re);
+    z.im = quad_sum(z.im);
+    if (i < n && q4 == 0) O[i * M + j] = z;
+  };
+  // entry o = i N + p of the Green's function, (y X)[p][i]
+  auto green = [&](int o, int n) {
+    const int i = o / N, p = o - i * N;
+    cplx z = {0.0, 0.0};
+    for (int j = 0; j < n; ++j) z = cadd(z, cmul(y[p * n + j], X[j * M + i]));
+    return z;
+  };
+
+  // ---- Green's functions of the walker
+  for (int s = 0; s < a.nspin; ++s) {
+    const int n = a.n[s], c = N * n;
+    if (a.reuse) {
+      for (int e = t; e < 2 * c; e += SMALL_NT) gl(s)[e] = a.green[s][(int64_t)w * 2 * c + e];
+    } else {
+      if (s) __syncthreads();
+      stage_walker(s);
+      stage_trial(s);
+      __syncthreads();
+      overlap(n);
+      __syncthreads();
+      if (wave == 0) small_invert(O, X, n, true, lane);
+      __syncthreads();
+      for (int o = t; o < c; o += SMALL_NT) {
+        const cplx z = green(o, n);
+        gl(s)[o] = z.re;
+        gl(s)[c + o] = z.im;
+      }
+    }
+  }
+  __syncthreads();
+  // the first spin's walker and E, and what the weight update needs, while the fields form
+  if (a.reuse || a.nspin > 1) stage_walker(0);
+  for (int e = t; e < N * N; e += SMALL_NT) E[e] = a.E[0][e];
+  const cplx oold = a.tail.overlaps[w];
+  const double wold = a.tail.weights[w], pcs = a.tail.scalars[1];
+
+  // ---- force bias and fields (fields_kernel's formulas)
+  cplx st = {0.0, 0.0}, ft = {0.0, 0.0};
+  for (int g0 = 0; g0 < G; g0 += SMALL_NT / 4) {
+    const int g = g0 + (t >> 2), gc = min(g, G - 1);
+    const cplx m = a.mf[gc];
+    const double xv = a.fields[(int64_t)w * G + gc];
+    double fr = 0.0, fi = 0.0;
+    for (int s = 0; s < a.nspin; ++s) {
+      const int c = N * a.n[s];
+      const double* r = a.rot[s] + (int64_t)gc * c;
+#pragma unroll 8
+      for (int e = q4; e < c; e += 4) {
+        const double v = r[e];
+        fr = fma(v, gl(s)[e], fr);
+        fi = fma(v, gl(s)[c + e], fi);
+      }
+    }
+    const cplx f = {a.mult * quad_sum(fr), a.mult * quad_sum(fi)};
+    if (g < G && q4 == 0) {
+      const cplx fs = {-a.sqdt * (-f.im - m.re), -a.sqdt * (f.re - m.im)};
+      const cplx xt = {xv - fs.re, -fs.im};
+      const cplx fs2 = cmul(fs, fs);
+      st = cadd(st, cmul(xt, m));
+      ft = cadd(ft, cplx{xv * fs.re - fs2.re / 2.0, xv * fs.im - fs2.im / 2.0});
+      xr[g] = -a.sqdt * xt.im;
+      xi[g] = a.sqdt * xt.re;
+    }
+  }
+  {
+    double v[4] = {st.re, st.im, ft.re, ft.im};
+#pragma unroll
+    for (int off = 32; off >= 4; off >>= 1)  // (lanes 4 i carry the sums)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[c] += __shfl_down(v[c], off, 64);
+    if (lane == 0)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) red[wave * 4 + c] = v[c];
+  }
+  __syncthreads();
+
+  for (int s = 0; s < a.nspin; ++s) {
+    const int n = a.n[s], c = N * n;
+    if (s) {  // (the last spin's Green's function is done with y)
+      stage_walker(s);
+      for (int e = t; e < N * N; e += SMALL_NT) E[e] = a.E[s][e];
+    }
+    stage_trial(s);
+    // ---- V (as N x N, from the packed upper triangle too)
+    if (s == 0 || a.chol_spins == 2) {
+      const double* L = a.chol_t + (int64_t)(a.chol_spins == 2 ? s : 0) * a.nv * G;
+      const bool packed = a.nv != N * N;
+      for (int e0 = 0; e0 < a.nv; e0 += SMALL_NT / 4) {
+        const int e = e0 + (t >> 2);
+        const double* r = L + (int64_t)min(e, a.nv - 1) * G;
+        double vr = 0.0, vi = 0.0;
+#pragma unroll 8
+        for (int g = q4; g < G; g += 4) {
+          const double l = r[g];
+          vr = fma(l, xr[g], vr);
+          vi = fma(l, xi[g], vi);
+        }
+        vr = quad_sum(vr);
+        vi = quad_sum(vi);
+        if (e < a.nv && q4 == 0) {
+          if (packed) {
+            // row p of the triangle starts at p N - p (p - 1) / 2
+            const float b = (float)(2 * N + 1);
+            int p = (int)((b - sqrtf(b * b - 8.0f * (float)e)) * 0.5f);
+            if (p * N - p * (p - 1) / 2 > e) --p;
+            if ((p + 1) * N - (p + 1) * p / 2 <= e) ++p;
+            const int k = p + e - (p * N - p * (p - 1) / 2);
+            V[p * N + k] = V[k * N + p] = cplx{vr, vi};
+          } else {
+            V[e] = cplx{vr, vi};
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // ---- w <- E (t0 + V t0 + V V t0 / 2 + ...), t0 = E w, in Horner form; the lane of
+    // number j mod 4 of a quad stores its sum j
+    int prow[SMALL_R], pcol[SMALL_R];
+    cplx t0[SMALL_R], u[SMALL_R];
+#pragma unroll
+    for (int j = 0; j < SMALL_R; ++j) {
+      const int o = min((t >> 2) + SMALL_NT / 4 * j, c - 1);
+      prow[j] = o / n;
+      pcol[j] = o - prow[j] * n;
+      t0[j] = u[j] = cplx{0.0, 0.0};
+    }
+    auto real_product = [&](cplx (&out)[SMALL_R]) {  // out = E y
+#pragma unroll
+      for (int j = 0; j < SMALL_R; ++j) {
+        if (SMALL_NT / 4 * j >= c) continue;
+        cplx x = {0.0, 0.0};
+#pragma unroll 4
+        for (int q = q4; q < N; q += 4) {
+          const double v = E[prow[j] * N + q];
+          const cplx z = y[q * n + pcol[j]];
+          x.re = fma(v, z.re, x.re);
+          x.im = fma(v, z.im, x.im);
+        }
+        out[j] = cplx{quad_sum(x.re), quad_sum(x.im)};
+      }
+    };
+    auto put = [&](const cplx (&v)[SMALL_R]) {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < SMALL_R; ++j) {
+        const int o = (t >> 2) + SMALL_NT / 4 * j;
+        if (o < c && q4 == (j & 3)) y[o] = v[j];
+      }
+      __syncthreads();
+    };
+    real_product(t0);
+    put(t0);
+    for (int k = a.terms_k; k >= 1; --k) {
+      const double dk = (double)k, rk = 1.0 / dk;
+#pragma unroll
+      for (int j = 0; j < SMALL_R; ++j) {
+        if (SMALL_NT / 4 * j >= c) continue;
+        cplx x0 = {0.0, 0.0}, x1 = {0.0, 0.0};
+#pragma unroll 4
+        for (int q = q4; q < N; q += 4) {
+          const cplx v = V[prow[j] * N + q], z = y[q * n + pcol[j]];
+          x0.re = fma(v.re, z.re, x0.re);
+          x0.im = fma(v.re, z.im, x0.im);
+          x1.re = fma(-v.im, z.im, x1.re);
+          x1.im = fma(v.im, z.re, x1.im);
+        }
+        // x / k: the product with 1 / k corrected by its residual
+        const double sr = quad_sum(x0.re + x1.re), si = quad_sum(x0.im + x1.im);
+        const double qr = sr * rk, qi = si * rk;
+        u[j] = cplx{t0[j].re + fma(fma(-qr, dk, sr), rk, qr),
+                    t0[j].im + fma(fma(-qi, dk, si), rk, qi)};
+      }
+      put(u);
+    }
+    real_product(u);
+    put(u);
+    cplx* phi = a.walkers[s] + (int64_t)w * c;
+    for (int o = t; o < c; o += SMALL_NT) phi[o] = y[o];
+
+    // ---- new overlaps; one wave updates the weight, the others form the Green's function
+    // for the next step
+    overlap(n);
+    __syncthreads();
+    if (wave == 0) {
+      const cplx det = small_invert(O, X, n, a.keep, lane);
+      if (lane == 0) dets[s] = det;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      if (s + 1 == a.nspin) {
+        const cplx onew = cmul(dets[0], dets[s]);
+        double v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (red[i] + red[4 + i]) + (red[8 + i] + red[12 + i]);
+        small_weight(a.tail, pcs, w, onew, cplx{v[0], v[1]}, cplx{v[2], v[3]}, oold, wold, lane);
+      }
+    } else if (a.keep) {
+      double* gw = a.green[s] + (int64_t)w * 2 * c;
+      for (int o = t - 64; o < c; o += SMALL_NT - 64) {
+        const cplx z = green(o, n);
+        gw[o] = z.re;
+        gw[c + o] = z.im;
+      }
+    }
+    __syncthreads();
+  }
+
+  // ---- population-control shift (propagation.py:161-164) by the last workgroup to arrive.
+  // Nothing but the weights is read across workgroups: they are written through, and the
+  // wait puts a weight in place before its workgroup arrives (a release at agent scope would
+  // write the whole L2 back: 3 us).  Every workgroup has read the old shift by then.
+  if (t == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(a.arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           a.W - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  double part = 0.0;
+  for (int i = t; i < a.W; i += SMALL_NT)
+    part += __hip_atomic_load(a.tail.weights + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const double total = block_sum<SMALL_NT>(part, red);
+  if (t == 0) {
+    a.tail.scalars[1] = a.tail.scalars[0] - 0.1 * (log(total / (double)a.W) / a.dt);
+    *a.arrived = 0;
+  }
+}
+
+}  // namespace
+
+// Where one launch is the better step (five steps, separate launches against one, us):
+//   - every workgroup resident at once, two to a CU: norb 16, n = 4, 64 vectors: 272 : 196 at
+//     500 walkers, 289 : 321 at 1000;
+//   - the entries of the Cholesky vectors (V's and the half-rotated ones) that each workgroup
+//     runs through by itself: 27000 and less (norb 10, 16, 20) gain a third to a half, 43000
+//     (norb 24, n = 6, 96 vectors, 200 walkers) 297 : 249, 100000 (norb 32, n = 8, 128
+//     vectors) 339 : 393.
+constexpr int SMALL_MAX_W = 512;
+constexpr int64_t SMALL_MAX_ENTRIES = 50000;
+bool small_step_fits(const afqmc_ctx* c, int W) {
+  if (c->mixed || c->f32 || W > SMALL_MAX_W || c->d.norb > SMALL_MAX_N) return false;
+  int64_t rows = (int64_t)c->chol_spins * c->vhs_nv;
+  for (int s = 0; s < c->nspin; ++s) {
+    if (c->nocc[s] < 1 || c->nocc[s] > SMALL_MAX_OCC) return false;
+    rows += c->kdim[s];
+  }
+  return rows * c->d.nchol <= SMALL_MAX_ENTRIES;
+}
+
+int launch_small_step(afqmc_ctx* c, int W, cplx* wup, cplx* wdn, const double* fields,
+                      const WeightsArgs& tail, bool reuse, bool keep) {
+  SmallStep a{};
+  a.W = W;
+  a.N = c->d.norb;
+  a.G = c->d.nchol;
+  a.nspin = c->nspin;
+  a.chol_spins = c->chol_spins;
+  a.terms_k = c->d.n_exp_terms - 1;
+  a.nv = c->vhs_nv;
+  a.mult = c->mult;
+  a.reuse = reuse;
+  a.keep = keep;
+  a.dt = c->d.dt;
+  a.sqdt = sqrt(c->d.dt);
+  for (int s = 0; s < c->nspin; ++s) {
+    a.n[s] = c->nocc[s];
+    a.trial[s] = c->trial[s];
+    a.rot[s] = c->rot_chol[s];
+    a.E[s] = c->exp_h1[s];
+    a.walkers[s] = s ? wdn : wup;
+    a.green[s] = c->green[s];
+  }
+  a.chol_t = c->chol_t;
+  a.mf = c->mf_shifts;
+  a.fields = fields;
+  a.tail = tail;
+  a.arrived = c->step_arrived;
+  const size_t shm = sizeof(double) * (size_t)small_doubles(a.N, a.n[0], a.n[1], a.G);
+  static int lds_limit = 0;
+  const int rc = ensure_dyn_lds((const void*)small_step_kernel, shm, &lds_limit);
+  if (rc) return rc;
+  hipLaunchKernelGGL(small_step_kernel, dim3(W), dim3(SMALL_NT), shm, c->stream, a);
+  LAUNCH_CHECK();
+  return AFQMC_OK;
+}

@@ -218,7 +218,8 @@ AFQMC_API int afqmc_estimate_mix(afqmc_ctx* ctx, double* scalars, const double* 
  * measurement for benchmarks).  While enabled, each phase of afqmc_propagate and the
  * block entry points records an event pair; afqmc_prof_collect (after the stream
  * has drained) adds the elapsed milliseconds and launch counts per phase into
- * ms[AFQMC_NPHASE] / counts[AFQMC_NPHASE] and clears the record. */
+ * ms[AFQMC_NPHASE] / counts[AFQMC_NPHASE] and clears the record.  Steps of small float64
+ * problems, otherwise one launch, run as a launch per phase while enabled. */
 enum {
   AFQMC_PH_GREEN = 0,    /* Green's function of the current walkers   */
   AFQMC_PH_FB_GEMM = 1,  /* force-bias contraction                    */

@@ -155,3 +155,40 @@ def test_energy_at_each_exchange_tile(gpu, norb, nelec, nchol, W, precision, tol
                                       near=wd["mo_coeff"], noise=0.1)
     got = trial.calc_energy(to_dev(walkers, gpu), hdat, wave)
     assert rel(got, o.calc_energy("uhf", walkers, oh, wd)) < tol
+
+
+@pytest.mark.parametrize("asym", [0.0, 1e-7])
+@pytest.mark.parametrize("wt,norb,nelec,nchol,W", [
+    ("rhf", 1, (1, 1), 1, 1), ("rhf", 10, (5, 5), 27, 200), ("uhf", 9, (8, 1), 33, 65),
+    ("uhf", 17, (8, 7), 65, 300), ("rhf", 32, (8, 8), 63, 9), ("uhf", 31, (7, 3), 5, 512)])
+def test_step_in_one_launch_matches_separate_launches(gpu, wt, norb, nelec, nchol, W, asym):
+    """Steps of small problems run as one launch, or as one launch per phase while phases are
+    timed: the same walkers, weights, overlaps and shift over steps that reuse the Green's
+    function and one that does not, for V kept whole and as its upper triangle."""
+    print(f"one launch {wt} N={norb} nelec={nelec} G={nchol} W={W} asym={asym}", flush=True)
+    hd, wd, nelec = problem(wt, norb, nelec, nchol)
+    chol = np.array(hd["chol"]).reshape(nchol, norb, norb)
+    skew = np.random.default_rng(5).uniform(-1.0, 1.0, (norb, norb))
+    chol += asym * np.max(np.abs(chol)) * np.triu(skew, 1)[None]
+    hd = dict(hd, chol=chol.reshape(nchol, norb * norb))
+    trial, prop, hdat, wave, _ = make(wt, norb, nelec, nchol, W, hd, wd)
+    dev = hdat["_afqmc_device"]
+    rng = np.random.default_rng(3)
+    walkers = problems.random_walkers(wt, norb, nelec, W, rng, near=wd["mo_coeff"], noise=0.1)
+    fields = to_dev(rng.standard_normal((4, W, nchol)), gpu)
+    got = []
+    for timed in (False, True):
+        dev.prof_enable(timed)
+        w = to_dev(walkers, gpu)
+        weights = torch.ones(W, dtype=torch.float64, device=gpu)
+        overlaps = dev.overlap(w)
+        scalars = torch.tensor([-0.5, -0.5], dtype=torch.float64, device=gpu)
+        for s in range(4):
+            dev.propagate(w, weights, overlaps, fields[s], scalars, reuse_green=s in (1, 3),
+                          keep_green=s != 1)
+        got.append((w, weights, overlaps, scalars))
+    dev.prof_enable(False)
+    one, many = got
+    for a, b in zip(one, many):
+        b = [x.cpu().numpy() for x in b] if isinstance(b, list) else b.cpu().numpy()
+        assert rel(a, b) < TOL
