@@ -801,37 +801,38 @@ int launch_bf_ct(afqmc_ctx* c, int W, int n, cplx* wk, int s) {
 
 // ------------------------------------------------------------------------------------
 // Split-bf16 streaming form for the mixed mode beyond the register kernel's range
-// (N <= 256, n <= 64).  One workgroup per walker of one spin; wave r owns RT 16-row
-// output tiles starting at row 16 RT r, and every column.  y = [yr | yi] (N x 2 n, each
-// half padded to 16 CT columns) lives in LDS as hi / lo bf16 planes stored [column][k]
-// with k contiguous, so a lane's B operand (8 consecutive k of one column) is one 16-byte
-// read; k is padded with zeros to 32 ceil(N / 32).  V streams from global memory as
-// float32 rows, 32 k at a time with the next block in flight while the current one
-// multiplies, and is split into bf16 planes in registers.  The complex product is four
-// real products,
+// (N <= 256, n <= 64).  One workgroup per walker of one spin; wave r owns output rows
+// [16 r, 16 r + 16) and every column.  y = [yr | yi] (N x 2 n, each half padded to 16 CT
+// columns) lives in LDS as hi / lo bf16 planes stored [column][k] with k contiguous, so a
+// lane's B operand (8 consecutive k of one column) is one 16-byte read; k is padded with
+// zeros to 32 ceil(N / 32).  V streams from global memory as float32 rows, 32 k at a time
+// with the next block in flight while the current one multiplies, and is split into bf16
+// planes in registers.  The complex product is four real products,
 //   ur = Vr yr - Vi yi,  ui = Vr yi + Vi yr,
 // each as three bf16 products (al bh + ah bl + ah bh) on v_mfma_f32_16x16x32_bf16 with
 // float32 accumulation; the planes of -Vi are those of Vi with the sign bits flipped
 // (round-to-nearest-even is symmetric).  E y = y + (E - I) y uses the split planes of
 // E - I (rows of 32 ceil(N / 32) entries) as the register form does, and the Horner
-// recursion y <- t0 + V y / k runs in float32 registers.  The body takes RT 16-row tiles
-// per wave (RT = 2 shares each B operand between two tiles at 256 registers per lane);
-// one tile per wave, up to 16 waves at 128 registers, is what runs: with the packed-V
-// gathers it measured faster for three and four column tiles despite spilling 25-48
-// registers around the Horner steps (UHF N = 200: 2.21 -> 2.04 ms per step).
+// recursion y <- t0 + V y / k runs in float32 registers.
+//
+// What it is shaped by: LDS holds one workgroup of up to 16 waves per CU, so a wave has 128
+// registers and little else to hide its loads.  The next block's loads must not be touched
+// before its split (a select or copy of a loaded value waits for it in the step that
+// asked for it), and nothing may spill: constant LDS strides, byte offsets to uniform bases,
+// and blocks of one kind per branch.  Masked loads, copied at once, with 25 to 48 registers
+// spilled: 2.00 ms for both spins at norb 200, n = 40, 2048 walkers; now 1.50.
 typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));  // dword-aligned rows
 
-inline int bfs_ldk(int N) { return 32 * ((N + 31) / 32) + 16; }
+// LDS columns of y: k padded to 32 ceil(N / 32), a stride fixed for N up to 128 or 256 so
+// that every operand's place is an immediate offset
+constexpr int bfs_ldk(bool small) { return small ? 144 : 272; }
+inline bool bfs_small(int N, int ct) { return N <= 128 && ct >= 3; }  // (else N > 128)
 inline size_t bfs_shm(int N, int ct) {
-  return (size_t)2 * 32 * ct * bfs_ldk(N) * sizeof(uint16_t);
+  return (size_t)2 * 32 * ct * bfs_ldk(bfs_small(N, ct)) * sizeof(uint16_t);
 }
-constexpr int bfs_rt(int) { return 1; }
-inline int bfs_threads(int N, int ct) {
-  const int rows = 16 * bfs_rt(ct);
-  return 64 * ((N + rows - 1) / rows);
-}
+inline int bfs_threads(int N) { return 64 * ((N + 15) / 16); }
 
-template <int CT, int RT>
+template <int CT, bool SMALL>
 __device__ __forceinline__ void taylor_bfs_body(int N, int n, int n_terms_k,
                                                 cplx* __restrict__ walkers,
                                                 const uint16_t* __restrict__ emi_hi,
@@ -839,281 +840,271 @@ __device__ __forceinline__ void taylor_bfs_body(int N, int n, int n_terms_k,
                                                 const float* __restrict__ vhs, int nv,
                                                 const int w) {
   constexpr int NC = 32 * CT;  // LDS columns: CT tiles of yr, then CT tiles of yi
+  constexpr int LDK = bfs_ldk(SMALL);  // rows and chunk swizzle as in the register form
   const int KBk = (N + 31) >> 5;
-  const int LDK = 32 * KBk + 16;  // rows and chunk swizzle as in the register form
   const int np32 = 32 * KBk;
   extern __shared__ uint16_t YB[];  // [2 planes][NC][LDK]
-  uint16_t* Yh = YB;
-  uint16_t* Yl = YB + NC * LDK;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rb = wave * 16 * RT;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rb = wave * 16;
   const int q4 = lane >> 4, col = lane & 15;
   const int sw = (col >> 2) & 1;  // chunk swizzle of this lane's LDS columns
-  const int q4s = q4 ^ sw;
-  // uniform bases with 32-bit lane offsets (saddr + voffset addressing)
   cplx* phi = walkers + (int64_t)w * N * n;
   // V planes: all N^2 entries row-major, or (nv = N(N+1)/2, symmetric V) the upper
   // triangle row by row, entry (a, b), a <= b, at a N - a (a - 1) / 2 + b - a
   const bool packed = nv != N * N;
   const float* Vr = vhs + (int64_t)w * 2 * nv;
   const float* Vi = Vr + nv;
-  bool prow[RT];
-  int prw[RT], voff[RT], eoff[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    const int p = rb + 16 * t + col;  // A row of this lane in tile t
-    prow[t] = p < N;
-    prw[t] = prow[t] ? p : 0;
-    // start of row p (packed: of its upper part, entry (p, p))
-    voff[t] = packed ? prw[t] * N - (prw[t] * (prw[t] - 1)) / 2 : prw[t] * N;
-    eoff[t] = prw[t] * np32;
-  }
+  const int p = min(rb + col, N - 1);  // A row of this lane
+  const bool prow = rb + col < N;
+  const bool tail = rb + 16 > N;  // the wave holds rows past N: zeros
+  // start of row p (packed: of its upper part, entry (p, p))
+  const int voff = packed ? p * N - (p * (p - 1)) / 2 : p * N;
 
   {
     u32x4_t* z = reinterpret_cast<u32x4_t*>(YB);
     const int nz = 2 * NC * LDK / 8;
     for (int e = threadIdx.x; e < nz; e += blockDim.x) z[e] = u32x4_t{0u, 0u, 0u, 0u};
   }
+
+  // walker (float64) -> float32 D layout, the loads all in flight
+  float4_t t0r[CT], t0i[CT], ur[CT], ui[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    cplx z[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      z[r] = phi[min(rb + 4 * q4 + r, N - 1) * n + min(ct * 16 + col, n - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const bool ok = rb + 4 * q4 + r < N && ct * 16 + col < n;
+      t0r[ct][r] = ok ? (float)z[r].re : 0.f;
+      t0i[ct][r] = ok ? (float)z[r].im : 0.f;
+    }
+  }
   __syncthreads();
 
   // D layout (rows 4 (l / 16) + r of a tile, column l % 16) -> LDS planes: four
   // consecutive k of one column, 8-byte stores.  Rows >= N and columns >= n carry zeros
   // (their A rows / B columns are zero), which keeps the padding zero.
-  auto put = [&](const float4_t (*yr)[CT], const float4_t (*yi)[CT]) {
+  uint16_t* yput = YB + col * LDK + rb + 8 * ((q4 >> 1) ^ sw) + 4 * (q4 & 1);
+  auto put = [&](const float4_t (&yr)[CT], const float4_t (&yi)[CT]) {
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          const float4_t v = h ? yi[t][ct] : yr[t][ct];
-          const int off = (h * 16 * CT + ct * 16 + col) * LDK + rb + 16 * t + 8 * ((q4 >> 1) ^ sw) + 4 * (q4 & 1);
-          const uint32_t h01 = pack_bf16x2(v[0], v[1]);
-          const uint32_t h23 = pack_bf16x2(v[2], v[3]);
-          const uint32_t l01 = pack_bf16x2(v[0] - bf16_lo_val(h01), v[1] - bf16_hi_val(h01));
-          const uint32_t l23 = pack_bf16x2(v[2] - bf16_lo_val(h23), v[3] - bf16_hi_val(h23));
-          *reinterpret_cast<u32x2_t*>(Yh + off) = u32x2_t{h01, h23};
-          *reinterpret_cast<u32x2_t*>(Yl + off) = u32x2_t{l01, l23};
-        }
-  };
-  auto bload = [&](const uint16_t* plane, int c0, int kb) {
-    return __builtin_bit_cast(
-        bf16x8_t, *reinterpret_cast<const u32x4_t*>(plane + (c0 + col) * LDK + kb * 32 + 8 * q4s));
-  };
-  auto zero = [&](float4_t (*a)[CT]) {
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) a[t][ct] = float4_t{0.f, 0.f, 0.f, 0.f};
-  };
-  // acc = (E - I) y, a real operator on both halves
-  auto e_product = [&](float4_t (*ar)[CT], float4_t (*ai)[CT]) {
-    zero(ar);
-    zero(ai);
-#pragma unroll 1
-    for (int kb = 0; kb < KBk; ++kb) {
-      bf16x8_t a_h[RT], a_l[RT];
-#pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        u32x4_t ah = {0, 0, 0, 0}, al = {0, 0, 0, 0};
-        if (prow[t]) {
-          ah = *reinterpret_cast<const u32x4_t*>(emi_hi + (eoff[t] + kb * 32 + 8 * q4));
-          al = *reinterpret_cast<const u32x4_t*>(emi_lo + (eoff[t] + kb * 32 + 8 * q4));
-        }
-        a_h[t] = __builtin_bit_cast(bf16x8_t, ah);
-        a_l[t] = __builtin_bit_cast(bf16x8_t, al);
-      }
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const bf16x8_t rh = bload(Yh, ct * 16, kb), rl = bload(Yl, ct * 16, kb);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          ar[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_l[t], rh, ar[t][ct], 0, 0, 0);
-          ar[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_h[t], rl, ar[t][ct], 0, 0, 0);
-          ar[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_h[t], rh, ar[t][ct], 0, 0, 0);
-        }
-        const bf16x8_t ih = bload(Yh, (CT + ct) * 16, kb), il = bload(Yl, (CT + ct) * 16, kb);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          ai[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_l[t], ih, ai[t][ct], 0, 0, 0);
-          ai[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_h[t], il, ai[t][ct], 0, 0, 0);
-          ai[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_h[t], ih, ai[t][ct], 0, 0, 0);
-        }
+        const float4_t v = h ? yi[ct] : yr[ct];
+        const int off = (h * 16 * CT + ct * 16) * LDK;
+        const uint32_t h01 = pack_bf16x2(v[0], v[1]);
+        const uint32_t h23 = pack_bf16x2(v[2], v[3]);
+        const uint32_t l01 = pack_bf16x2(v[0] - bf16_lo_val(h01), v[1] - bf16_hi_val(h01));
+        const uint32_t l23 = pack_bf16x2(v[2] - bf16_lo_val(h23), v[3] - bf16_hi_val(h23));
+        *reinterpret_cast<u32x2_t*>(yput + off) = u32x2_t{h01, h23};
+        *reinterpret_cast<u32x2_t*>(yput + NC * LDK + off) = u32x2_t{l01, l23};
       }
-    }
   };
-  // 8 consecutive k of a V row, for chunks that start inside the row (others are zero).
-  // A chunk on or right of the diagonal is contiguous in the stored row: two 16-byte
-  // loads.  A chunk that straddles k = N reads at most 7 floats past the row end, into the
-  // next row or, for the last row of the last walker, into the 8 floats of tail padding
-  // of the VHS buffer, and is masked after the load.  In the packed layout a chunk left
-  // of the diagonal reads entries (k, p) of rows k < p one by one; for a fixed k the 16
-  // rows of a lane group are consecutive floats of one stored row.
-  auto vload = [&](int kb, float (*r)[8], float (*i)[8]) {
-    const int k0 = kb * 32 + 8 * q4;
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-      f4u_t r0 = {0.f, 0.f, 0.f, 0.f}, r1 = r0, i0 = r0, i1 = r0;
-      const int p = prw[t];
-      if (prow[t] && k0 < N && (!packed || k0 >= p)) {
-        const int base = voff[t] + (packed ? k0 - p : k0);
-        r0 = *reinterpret_cast<const f4u_t*>(Vr + base);
-        r1 = *reinterpret_cast<const f4u_t*>(Vr + (base + 4));
-        i0 = *reinterpret_cast<const f4u_t*>(Vi + base);
-        i1 = *reinterpret_cast<const f4u_t*>(Vi + (base + 4));
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        r[t][e] = r0[e];
-        r[t][4 + e] = r1[e];
-        i[t][e] = i0[e];
-        i[t][4 + e] = i1[e];
-      }
-      if (packed && prow[t] && k0 < p) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int k = k0 + e < N ? k0 + e : N - 1;
-          const int a = k < p ? k : p, b = k < p ? p : k;
-          const int idx = a * N - (a * (a - 1)) / 2 + (b - a);
-          r[t][e] = Vr[idx];
-          i[t][e] = Vi[idx];
-        }
-      }
-      if (k0 + 8 > N) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (k0 + e >= N) r[t][e] = i[t][e] = 0.f;
-      }
-    }
+  // B operand: 8 consecutive k of column 16 c + col (c: CT tiles of yr, then of yi)
+  const uint16_t* yget = YB + col * LDK + 8 * (q4 ^ sw);
+  auto bload = [&](const uint16_t* yk, int plane, int c) {
+    return __builtin_bit_cast(
+        bf16x8_t, *reinterpret_cast<const u32x4_t*>(yk + (plane * NC + 16 * c) * LDK));
   };
-  auto v_product = [&](float4_t (*ur)[CT], float4_t (*ui)[CT]) {
-    zero(ur);
-    zero(ui);
-    float rr[RT][8], ri[RT][8];
-    vload(0, rr, ri);
+  auto bf = [](const u32x4_t& x) { return __builtin_bit_cast(bf16x8_t, x); };
+  // acc = (E - I) y, a real operator on both halves; the next block's E in flight
+  auto e_product = [&](float4_t (&ar)[CT], float4_t (&ai)[CT]) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) ar[ct] = ai[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const uint16_t* eh = emi_hi + p * np32 + 8 * q4;
+    const uint16_t* el = emi_lo + p * np32 + 8 * q4;
+    u32x4_t nh = *reinterpret_cast<const u32x4_t*>(eh), nl = *reinterpret_cast<const u32x4_t*>(el);
+    const uint16_t* yk = yget;
 #pragma unroll 1
-    for (int kb = 0; kb < KBk; ++kb) {
-      u32x4_t rh[RT], rl[RT], ih[RT], il[RT];
+    for (int kb = 0; kb < KBk; ++kb, yk += 32) {
+      u32x4_t ah = nh, al = nl;
+      const int kn = kb + 1 < KBk ? 32 * (kb + 1) : 0;
+      nh = *reinterpret_cast<const u32x4_t*>(eh + kn);
+      nl = *reinterpret_cast<const u32x4_t*>(el + kn);
+      if (tail && !prow) ah = al = u32x4_t{0, 0, 0, 0};
 #pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        split8(rr[t], rh[t], rl[t]);
-        split8(ri[t], ih[t], il[t]);
+      for (int ct = 0; ct < CT; ++ct) {
+        const bf16x8_t rh = bload(yk, 0, ct), rl = bload(yk, 1, ct);
+        ar[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(al), rh, ar[ct], 0, 0, 0);
+        ar[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ah), rl, ar[ct], 0, 0, 0);
+        ar[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ah), rh, ar[ct], 0, 0, 0);
+        const bf16x8_t ih = bload(yk, 0, CT + ct), il = bload(yk, 1, CT + ct);
+        ai[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(al), ih, ai[ct], 0, 0, 0);
+        ai[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ah), il, ai[ct], 0, 0, 0);
+        ai[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ah), ih, ai[ct], 0, 0, 0);
       }
-      if (kb + 1 < KBk) vload(kb + 1, rr, ri);  // next block in flight
-      auto bf = [](const u32x4_t& x) { return __builtin_bit_cast(bf16x8_t, x); };
+    }
+  };
+  // 8 consecutive k of the lane's V row (those past N, or of a row past N, are zeroed at the
+  // split).  Right of the diagonal, or in whole rows, a chunk is contiguous: two 16-byte loads
+  // (one that straddles k = N reads at most 7 floats past the row end, into the next row or,
+  // for the last row of the last walker, into the 8 floats of tail padding of the VHS
+  // buffer).  Left of the diagonal of the packed layout it is the entries (k, p) of rows
+  // k < p, each N - 1 - k after the last; for a fixed k the 16 rows of a lane group are
+  // consecutive floats of one stored row.  Which of the two a block is holds for the whole
+  // wave but for the one or two blocks on the diagonal, so the branches are scalar and the
+  // loads unconditional, from clamped k.
+  struct Vops {
+    f4u_t r0, r1, i0, i1;
+  };
+  auto load1 = [](const float* base, uint32_t o) {  // uniform base, byte offset
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + o);
+  };
+  auto load4 = [](const float* base, uint32_t o) {
+    return *reinterpret_cast<const f4u_t*>(reinterpret_cast<const char*>(base) + o);
+  };
+  auto vload = [&](int kb, Vops& v) {
+    const int k0 = kb * 32 + 8 * q4;
+    if (!packed || 32 * kb >= rb + 15) {
+      // (chunks past N: the row's first one)
+      const uint32_t o = 4 * (voff + (k0 < N ? (packed ? k0 - p : k0) : 0));
+      v.r0 = load4(Vr, o);
+      v.r1 = load4(Vr, o + 16);
+      v.i0 = load4(Vi, o);
+      v.i1 = load4(Vi, o + 16);
+    } else if (32 * kb + 31 <= rb) {
+      uint32_t x = 4 * (k0 * N - (k0 * (k0 - 1)) / 2 + p - k0);  // entry (k0, p)
+      uint32_t d = 4 * (N - 1 - k0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (e < 4) {
+          v.r0[e & 3] = load1(Vr, x);
+          v.i0[e & 3] = load1(Vi, x);
+        } else {
+          v.r1[e & 3] = load1(Vr, x);
+          v.i1[e & 3] = load1(Vi, x);
+        }
+        x += d;
+        d -= 4;
+      }
+    } else {
+      const int kc = min(k0, N - 1);
+      uint32_t x = 4 * (kc * N - (kc * (kc - 1)) / 2 + p - kc);  // entry (k, p), for k <= p
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int k = min(k0 + e, N - 1);
+        const uint32_t o = k <= p ? x : 4 * (uint32_t)(voff + (k - p));
+        if (e < 4) {
+          v.r0[e & 3] = load1(Vr, o);
+          v.i0[e & 3] = load1(Vi, o);
+        } else {
+          v.r1[e & 3] = load1(Vr, o);
+          v.i1[e & 3] = load1(Vi, o);
+        }
+        x += 4 * (N - 1 - k);
+      }
+    }
+  };
+  auto v_product = [&]() {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) ur[ct] = ui[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
+    Vops v;
+    int first = 0;  // (opaque: the block's 16 addresses would be kept, spilled, across the terms)
+    asm volatile("" : "+s"(first));
+    vload(first, v);
+    const uint16_t* yk = yget;
+#pragma unroll 1
+    for (int kb = 0; kb < KBk; ++kb, yk += 32) {
+      u32x4_t rh, rl, ih, il;
+      {
+        float r[8], i[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          r[e] = v.r0[e];
+          r[4 + e] = v.r1[e];
+          i[e] = v.i0[e];
+          i[4 + e] = v.i1[e];
+        }
+        if (tail || 32 * kb + 32 > N) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (!prow || kb * 32 + 8 * q4 + e >= N) r[e] = i[e] = 0.f;
+        }
+        split8(r, rh, rl);
+        split8(i, ih, il);
+      }
+      if (kb + 1 < KBk) vload(kb + 1, v);  // next block in flight
       // rows of yr: ur += Vr yr, ui += Vi yr
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const bf16x8_t yh = bload(Yh, ct * 16, kb), yl = bload(Yl, ct * 16, kb);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rl[t]), yh, ur[t][ct], 0, 0, 0);
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh[t]), yl, ur[t][ct], 0, 0, 0);
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh[t]), yh, ur[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(il[t]), yh, ui[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih[t]), yl, ui[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih[t]), yh, ui[t][ct], 0, 0, 0);
-        }
+        const bf16x8_t yh = bload(yk, 0, ct), yl = bload(yk, 1, ct);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rl), yh, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(il), yh, ui[ct], 0, 0, 0);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh), yl, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih), yl, ui[ct], 0, 0, 0);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh), yh, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih), yh, ui[ct], 0, 0, 0);
       }
       // rows of yi: ur += (-Vi) yi, ui += Vr yi (Vi's planes negated in place)
       const u32x4_t sg = {0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
-#pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        ih[t] ^= sg;
-        il[t] ^= sg;
-      }
+      ih ^= sg;
+      il ^= sg;
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const bf16x8_t yh = bload(Yh, (CT + ct) * 16, kb), yl = bload(Yl, (CT + ct) * 16, kb);
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(il[t]), yh, ur[t][ct], 0, 0, 0);
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih[t]), yl, ur[t][ct], 0, 0, 0);
-          ur[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih[t]), yh, ur[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rl[t]), yh, ui[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh[t]), yl, ui[t][ct], 0, 0, 0);
-          ui[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh[t]), yh, ui[t][ct], 0, 0, 0);
-        }
+        const bf16x8_t yh = bload(yk, 0, CT + ct), yl = bload(yk, 1, CT + ct);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(il), yh, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rl), yh, ui[ct], 0, 0, 0);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih), yl, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh), yl, ui[ct], 0, 0, 0);
+        ur[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(ih), yh, ur[ct], 0, 0, 0);
+        ui[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(rh), yh, ui[ct], 0, 0, 0);
       }
     }
   };
 
-  // walker (float64) -> float32 D layout -> LDS
-  float4_t t0r[RT][CT], t0i[RT][CT], ur[RT][CT], ui[RT][CT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = rb + 16 * t + 4 * q4 + r;
-        const int c = ct * 16 + col;
-        float re = 0.f, im = 0.f;
-        if (row < N && c < n) {
-          const cplx z = phi[row * n + c];
-          re = (float)z.re;
-          im = (float)z.im;
-        }
-        t0r[t][ct][r] = re;
-        t0i[t][ct][r] = im;
-      }
   put(t0r, t0i);
   __syncthreads();
   e_product(ur, ui);
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      t0r[t][ct] += ur[t][ct];
-      t0i[t][ct] += ui[t][ct];
-    }
+  for (int ct = 0; ct < CT; ++ct) {
+    t0r[ct] += ur[ct];
+    t0i[ct] += ui[ct];
+  }
   __syncthreads();
   put(t0r, t0i);
   __syncthreads();
+#pragma unroll 1
   for (int k = n_terms_k; k >= 1; --k) {
-    v_product(ur, ui);
+    v_product();
     __syncthreads();
     const float rk = 1.0f / (float)k;
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        ur[t][ct] = t0r[t][ct] + ur[t][ct] * rk;
-        ui[t][ct] = t0i[t][ct] + ui[t][ct] * rk;
-      }
+    for (int ct = 0; ct < CT; ++ct) {
+      ur[ct] = t0r[ct] + ur[ct] * rk;
+      ui[ct] = t0i[ct] + ui[ct] * rk;
+    }
     put(ur, ui);
     __syncthreads();
   }
-  float4_t ar[RT][CT], ai[RT][CT];
-  e_product(ar, ai);
+  e_product(t0r, t0i);
 #pragma unroll
-  for (int t = 0; t < RT; ++t)
+  for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = rb + 16 * t + 4 * q4 + r;
-        const int c = ct * 16 + col;
-        if (row < N && c < n)
-          phi[row * n + c] = cplx{(double)(ur[t][ct][r] + ar[t][ct][r]),
-                                  (double)(ui[t][ct][r] + ai[t][ct][r])};
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int row = rb + 4 * q4 + r;
+      const int c = ct * 16 + col;
+      if (row < N && c < n)
+        phi[row * n + c] =
+            cplx{(double)(ur[ct][r] + t0r[ct][r]), (double)(ui[ct][r] + t0i[ct][r])};
+    }
 }
 
-template <int CT>
-__global__ __launch_bounds__(1024 / bfs_rt(CT)) void taylor_bfs_kernel(
+template <int CT, bool SMALL>
+__global__ __launch_bounds__(SMALL ? 512 : 1024, 4) void taylor_bfs_kernel(
     int N, int n, int n_terms_k, cplx* __restrict__ walkers, const uint16_t* __restrict__ emi_hi,
     const uint16_t* __restrict__ emi_lo, const float* __restrict__ vhs, int nv) {
-  taylor_bfs_body<CT, bfs_rt(CT)>(N, n, n_terms_k, walkers, emi_hi, emi_lo, vhs, nv,
+  taylor_bfs_body<CT, SMALL>(N, n, n_terms_k, walkers, emi_hi, emi_lo, vhs, nv,
                                   blockIdx.x);
 }
 
-template <int CT>
-__global__ __launch_bounds__(1024 / bfs_rt(CT)) void taylor_bfs_grouped_kernel(
+template <int CT, bool SMALL>
+__global__ __launch_bounds__(SMALL ? 512 : 1024, 4) void taylor_bfs_grouped_kernel(
     const TaylorArgs* __restrict__ args, const int* __restrict__ start, int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
   const TaylorArgs a = args[p];
-  taylor_bfs_body<CT, bfs_rt(CT)>(
+  taylor_bfs_body<CT, SMALL>(
       a.N, a.n, a.K, a.walkers, static_cast<const uint16_t*>(a.E),
       static_cast<const uint16_t*>(a.E2), static_cast<const float*>(a.vhs), a.nv,
       blockIdx.x - start[p]);
@@ -1124,8 +1115,8 @@ __global__ __launch_bounds__(1024 / bfs_rt(CT)) void taylor_bfs_grouped_kernel(
 // blocks are dealt round-robin to the 8 XCDs (block b on XCD b % 8), so the two blocks
 // of a walker run on the same XCD, one dispatch round apart, and the second one's V
 // rows mostly come from that XCD's L2 instead of HBM.
-template <int CT>
-__global__ __launch_bounds__(1024 / bfs_rt(CT)) void taylor_bfs_spins_kernel(
+template <int CT, bool SMALL>
+__global__ __launch_bounds__(SMALL ? 512 : 1024, 4) void taylor_bfs_spins_kernel(
     int N, int n0, int n1, int n_terms_k, int W, cplx* __restrict__ w0, cplx* __restrict__ w1,
     const uint16_t* __restrict__ e0h, const uint16_t* __restrict__ e0l,
     const uint16_t* __restrict__ e1h, const uint16_t* __restrict__ e1l,
@@ -1133,21 +1124,21 @@ __global__ __launch_bounds__(1024 / bfs_rt(CT)) void taylor_bfs_spins_kernel(
   const int b = blockIdx.x;
   const int s = (b >> 3) & 1, w = 8 * (b >> 4) + (b & 7);
   if (w >= W) return;  // (whole workgroup: the tail of the last group of 8 walkers)
-  taylor_bfs_body<CT, bfs_rt(CT)>(N, s ? n1 : n0, n_terms_k, s ? w1 : w0, s ? e1h : e0h,
+  taylor_bfs_body<CT, SMALL>(N, s ? n1 : n0, n_terms_k, s ? w1 : w0, s ? e1h : e0h,
                                   s ? e1l : e0l, vhs, nv, w);
 }
 
-template <int CT>
+template <int CT, bool SMALL>
 int launch_bfs_spins(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
   const int N = c->d.norb;
   if (N > 256 || c->nocc[0] > 16 * CT || c->nocc[1] > 16 * CT || 32 * ((N + 31) / 32) != c->Np32)
     return afqmc_set_error(AFQMC_ERR_ARG, "taylor bf16x3 streaming: N %d column tiles %d", N, CT);
   const size_t shm = bfs_shm(N, CT);
   static int lds_limit = 0;
-  const int rc = ensure_dyn_lds((const void*)taylor_bfs_spins_kernel<CT>, shm, &lds_limit);
+  const int rc = ensure_dyn_lds((const void*)taylor_bfs_spins_kernel<CT, SMALL>, shm, &lds_limit);
   if (rc) return rc;
   const int groups = (W + 7) / 8;
-  hipLaunchKernelGGL((taylor_bfs_spins_kernel<CT>), dim3(16 * groups), dim3(bfs_threads(N, CT)),
+  hipLaunchKernelGGL((taylor_bfs_spins_kernel<CT, SMALL>), dim3(16 * groups), dim3(bfs_threads(N)),
                      shm, c->stream, N, c->nocc[0], c->nocc[1], c->d.n_exp_terms - 1, W, wup,
                      wdn, c->emi_bf[0][0], c->emi_bf[0][1], c->emi_bf[1][0], c->emi_bf[1][1],
                      vhs_f32_of(c, 0), c->vhs_nv);
@@ -1155,7 +1146,7 @@ int launch_bfs_spins(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
   return AFQMC_OK;
 }
 
-template <int CT>
+template <int CT, bool SMALL>
 int launch_bfs(afqmc_ctx* c, int W, int n, cplx* wk, int s) {
   const int N = c->d.norb;
   if (N > 256 || n > 16 * CT || 32 * ((N + 31) / 32) != c->Np32)
@@ -1163,9 +1154,9 @@ int launch_bfs(afqmc_ctx* c, int W, int n, cplx* wk, int s) {
                            N, n, CT);
   const size_t shm = bfs_shm(N, CT);
   static int lds_limit = 0;
-  const int rc = ensure_dyn_lds((const void*)taylor_bfs_kernel<CT>, shm, &lds_limit);
+  const int rc = ensure_dyn_lds((const void*)taylor_bfs_kernel<CT, SMALL>, shm, &lds_limit);
   if (rc) return rc;
-  hipLaunchKernelGGL((taylor_bfs_kernel<CT>), dim3(W), dim3(bfs_threads(N, CT)), shm, c->stream,
+  hipLaunchKernelGGL((taylor_bfs_kernel<CT, SMALL>), dim3(W), dim3(bfs_threads(N)), shm, c->stream,
                      N, n, c->d.n_exp_terms - 1, wk, c->emi_bf[s][0], c->emi_bf[s][1],
                      vhs_f32_of(c, s), c->vhs_nv);
   LAUNCH_CHECK();
@@ -1202,9 +1193,10 @@ void taylor_plan(const afqmc_ctx* c, int s, TaylorPlan* pl) {
       pl->shm = (size_t)2 * ctp * 16 * bf_ldk(kb) * sizeof(uint16_t);
     } else {  // N <= AFQMC_MAX_NORB = 256, n <= AFQMC_MAX_NOCC = 64
       pl->kind = TAYLOR_STREAM_BF16X3;
-      pl->ct = (n + 15) / 16;
-      pl->nthreads = bfs_threads(N, pl->ct);
-      pl->shm = bfs_shm(N, pl->ct);
+      const int ct = (n + 15) / 16;
+      pl->ct = ct + (bfs_small(N, ct) ? 4 : 0);
+      pl->nthreads = bfs_threads(N);
+      pl->shm = bfs_shm(N, ct);
     }
   } else if (N <= 128 && c->nocc[0] <= 32 && c->nocc[1] <= 32) {
     pl->kind = TAYLOR_REG_F64;
@@ -1225,10 +1217,14 @@ int launch_taylor(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
       (c->nocc[0] + 15) / 16 == (c->nocc[1] + 15) / 16) {
     // both spins streaming with one shared V: one launch, the spins of a walker side by side
     switch ((c->nocc[0] + 15) / 16) {
-      case 1: return launch_bfs_spins<1>(c, W, wup, wdn);
-      case 2: return launch_bfs_spins<2>(c, W, wup, wdn);
-      case 3: return launch_bfs_spins<3>(c, W, wup, wdn);
-      default: return launch_bfs_spins<4>(c, W, wup, wdn);
+      case 1: return launch_bfs_spins<1, false>(c, W, wup, wdn);
+      case 2: return launch_bfs_spins<2, false>(c, W, wup, wdn);
+      case 3:
+        return N <= 128 ? launch_bfs_spins<3, true>(c, W, wup, wdn)
+                        : launch_bfs_spins<3, false>(c, W, wup, wdn);
+      default:
+        return N <= 128 ? launch_bfs_spins<4, true>(c, W, wup, wdn)
+                        : launch_bfs_spins<4, false>(c, W, wup, wdn);
     }
   }
   if (c->taylor_bf) {
@@ -1249,10 +1245,16 @@ int launch_taylor(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
         }
       } else {
         switch ((n + 15) / 16) {
-          case 1: rc = launch_bfs<1>(c, W, n, wk, s); break;
-          case 2: rc = launch_bfs<2>(c, W, n, wk, s); break;
-          case 3: rc = launch_bfs<3>(c, W, n, wk, s); break;
-          default: rc = launch_bfs<4>(c, W, n, wk, s); break;
+          case 1: rc = launch_bfs<1, false>(c, W, n, wk, s); break;
+          case 2: rc = launch_bfs<2, false>(c, W, n, wk, s); break;
+          case 3:
+            rc = N <= 128 ? launch_bfs<3, true>(c, W, n, wk, s)
+                          : launch_bfs<3, false>(c, W, n, wk, s);
+            break;
+          default:
+            rc = N <= 128 ? launch_bfs<4, true>(c, W, n, wk, s)
+                          : launch_bfs<4, false>(c, W, n, wk, s);
+            break;
         }
       }
       if (rc) return rc;
@@ -1343,14 +1345,17 @@ int launch_taylor_grouped(hipStream_t st, int kind, int nkgv, int ct, const Tayl
     return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: k blocks %d, column tiles %d", nkgv, ct);
   }
   if (kind == TAYLOR_STREAM_BF16X3) {
-    static int lim[4] = {};
+    static int lim[6] = {};
+#define BFS_CASE(CASE, C, SMALL, I)                                                            \
+  case CASE:                                                                                   \
+    return launch_grouped_fn(taylor_bfs_grouped_kernel<C, SMALL>, st, args, start, nprob,      \
+                             nblocks, nthreads, shm, &lim[I]);
     switch (ct) {
-      case 1: return launch_grouped_fn(taylor_bfs_grouped_kernel<1>, st, args, start, nprob, nblocks, nthreads, shm, &lim[0]);
-      case 2: return launch_grouped_fn(taylor_bfs_grouped_kernel<2>, st, args, start, nprob, nblocks, nthreads, shm, &lim[1]);
-      case 3: return launch_grouped_fn(taylor_bfs_grouped_kernel<3>, st, args, start, nprob, nblocks, nthreads, shm, &lim[2]);
-      case 4: return launch_grouped_fn(taylor_bfs_grouped_kernel<4>, st, args, start, nprob, nblocks, nthreads, shm, &lim[3]);
+      BFS_CASE(1, 1, false, 0) BFS_CASE(2, 2, false, 1) BFS_CASE(3, 3, false, 2)
+      BFS_CASE(4, 4, false, 3) BFS_CASE(7, 3, true, 4) BFS_CASE(8, 4, true, 5)
       default: return afqmc_set_error(AFQMC_ERR_ARG, "grouped taylor: column tiles %d", ct);
     }
+#undef BFS_CASE
   }
   static int lim64[2] = {};
   if (nthreads <= 64 * STREAM_SMALL)
