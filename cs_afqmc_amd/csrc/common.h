@@ -555,5 +555,5 @@ int launch_gemm_bf16x3_grouped(hipStream_t s, int bm, int out, const GemmArgs* a
                                const int* start, int nprob, int nblocks);
 int launch_gemm_f64_grouped(hipStream_t s, int bm, const GemmArgs* args, const int* start,
                             int nprob, int nblocks);
-int launch_gemm_f32_grouped(hipStream_t s, int bm, bool vec2, const GemmArgs* args,
+int launch_gemm_f32_grouped(hipStream_t s, int bm, const GemmArgs* args,
                             const int* start, int nprob, int nblocks);

@@ -12,43 +12,42 @@
 //   B operand: lane l holds B[l / 16][l % 16]   (B as k x n)
 //   D (float4): lane l, element r holds D[4 (l / 16) + r][l % 16]
 //
-// Tiles of BM x BN with BK = 16, four waves (2 x 2), float operands k-major in LDS
-// (double buffered, register prefetch of the next k-tile).  Split-K as in the float64
-// GEMM: grid.y splits K and split z writes alpha * its partial product to
-// C + z * c_split_stride (beta must be 0); consumers add the slices in order.
+// Tiles of BM x BN with BK = 16, four waves (2 x 2), float operands in LDS (double buffered,
+// register prefetch of the next k-tile).  Split-K as in the float64 GEMM: grid.y splits K and
+// split z writes alpha * its partial product to C + z * c_split_stride (beta must be 0);
+// consumers add the slices in order.
+//
+// As in the float64 GEMM, operand loads are 16 bytes and unconditional, from clamped rows and
+// k at any 8-byte boundary (masked loads waited one by one, and odd K read 8 bytes at a
+// time), and k past the range is zeroed as the registers go to LDS.  An LDS row of 16 floats
+// is four 16-byte chunks, element e of chunk c being k = 4 e + c, so one read per lane and
+// row feeds the four MFMAs of a k-tile, each of four consecutive k; chunk c of row r sits at
+// c ^ ((r >> 1) & 3), under which the sixteen rows of a chunk meet no bank twice.
+// A step's two, 1200 x 2701 x 301 and 1200 x 301 x 1241: 62 -> 29 us on average.
 #include "common.h"
 
 namespace {
 
 constexpr int F32_BK = 16;
-constexpr int F32_PAD = 16;  // row stride == 16 (mod 32) floats: rows k, k+1 use disjoint banks
-// Element (k, m) of a k-major LDS tile sits at column m ^ f32_swz<VEC>(k).  The MFMA
-// operand reads (16 consecutive m at k = 4 s .. 4 s + 3 per wave) share the swizzle and
-// see the same banks as without it; the staging stores (16 or 8 k rows x 4 or 8 m per
-// wave) without it put four k rows on one bank, a 4-way conflict, and with it the 64
-// lanes meet 64 banks.
-template <int VEC>
-__device__ inline int f32_swz(int k) { return ((k >> 2) & 3) << (VEC == 2 ? 3 : 2); }
+constexpr int F32_RCH = F32_BK / 4;  // chunks per LDS row
+// 16 bytes at any 8-byte boundary (rows of odd length)
+typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
+typedef double d2_t __attribute__((ext_vector_type(2)));
 
-template <int BM, int BN, int WM, int WN, int VEC>
+template <int BM, int BN, int WM, int WN>
 __device__ __forceinline__ void gemm_nt_f32_body(
     int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
     const double* __restrict__ B, int ldb, double beta, double* __restrict__ C, int ldc,
     int tiles_m, int tiles_n, int k_per_split, int64_t c_split_stride, const int bx,
     const int by) {
-  constexpr int NT = 256;
-  constexpr int BK = F32_BK;
+  constexpr int BK = F32_BK, RCH = F32_RCH;
   constexpr int TM = BM / WM / 16;
   constexpr int TN = BN / WN / 16;
-  constexpr int KT = BK / VEC;
-  constexpr int RSTEP = NT / KT;
-  constexpr int A_LD = BM / RSTEP;
-  constexpr int B_LD = BN / RSTEP;
+  constexpr int A_LD = BM / 32, B_LD = BN / 32;  // 8 threads to a row
   static_assert(WM * WN == 4, "four waves");
-  static_assert(A_LD >= 1 && B_LD >= 1, "tile too small");
 
-  __shared__ float As[2][BK][BM + F32_PAD];
-  __shared__ float Bs[2][BK][BN + F32_PAD];
+  __shared__ float4_t As[2][BM * RCH];
+  __shared__ float4_t Bs[2][BN * RCH];
 
   int tile_m, tile_n;
   const bool m_major = M > N;
@@ -62,48 +61,44 @@ __device__ __forceinline__ void gemm_nt_f32_body(
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave % WM, wn = wave / WM;
-  const int lk = (t % KT) * VEC, lr = t / KT;
+  const int lch = t & 7, lr = t >> 3;
 
-  float ra[A_LD][VEC], rb[B_LD][VEC];
+  // rows past M or N read the last row: their products are never stored
+  const double* Ab = A + (int64_t)m0 * lda;
+  const double* Bb = B + (int64_t)n0 * ldb;
+  int aoff[A_LD], boff[B_LD];
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) aoff[i] = min(lr + i * 32, M - 1 - m0) * lda;
+#pragma unroll
+  for (int i = 0; i < B_LD; ++i) boff[i] = min(lr + i * 32, N - 1 - n0) * ldb;
+  d2_t ra[A_LD], rb[B_LD];
+  // pairs past kend read elements kend - 1 and kend (the operands' allocations end with at
+  // least one element of padding)
   auto load_tile = [&](int k0) {
-    const int k = k0 + lk;
-    const bool kok = k < kend;  // VEC == 2 needs even k ranges (checked at launch)
+    const int k = min(k0 + 2 * lch, kend - 1);
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) ra[i] = *reinterpret_cast<const d2u_t*>(Ab + (aoff[i] + k));
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) rb[i] = *reinterpret_cast<const d2u_t*>(Bb + (boff[i] + k));
+  };
+  // the places of k = 2 lch and 2 lch + 1 in a row's floats (32-row steps keep them)
+  const int c0 = (2 * lch) & 3, rsw = (lr >> 1) & 3;
+  const int s0 = (lr * RCH + (c0 ^ rsw)) * 4 + (lch >> 1);
+  const int s1 = (lr * RCH + ((c0 + 1) ^ rsw)) * 4 + (lch >> 1);
+  auto store_tile = [&](int buf, int k0) {
+    const bool ok0 = k0 + 2 * lch < kend, ok1 = k0 + 2 * lch + 1 < kend;
+    float* a = reinterpret_cast<float*>(As[buf]);
+    float* b = reinterpret_cast<float*>(Bs[buf]);
 #pragma unroll
     for (int i = 0; i < A_LD; ++i) {
-      const int r = m0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < M && kok) v = *reinterpret_cast<const double2*>(A + (int64_t)r * lda + k);
-        ra[i][0] = (float)v.x;
-        ra[i][VEC - 1] = (float)v.y;
-      } else {
-        ra[i][0] = (r < M && kok) ? (float)A[(int64_t)r * lda + k] : 0.0f;
-      }
+      a[s0 + i * 32 * BK] = ok0 ? (float)ra[i].x : 0.f;
+      a[s1 + i * 32 * BK] = ok1 ? (float)ra[i].y : 0.f;
     }
 #pragma unroll
     for (int i = 0; i < B_LD; ++i) {
-      const int r = n0 + lr + i * RSTEP;
-      if (VEC == 2) {
-        double2 v = make_double2(0.0, 0.0);
-        if (r < N && kok) v = *reinterpret_cast<const double2*>(B + (int64_t)r * ldb + k);
-        rb[i][0] = (float)v.x;
-        rb[i][VEC - 1] = (float)v.y;
-      } else {
-        rb[i][0] = (r < N && kok) ? (float)B[(int64_t)r * ldb + k] : 0.0f;
-      }
+      b[s0 + i * 32 * BK] = ok0 ? (float)rb[i].x : 0.f;
+      b[s1 + i * 32 * BK] = ok1 ? (float)rb[i].y : 0.f;
     }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < A_LD; ++i)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        As[buf][lk + v][(lr + i * RSTEP) ^ f32_swz<VEC>(lk + v)] = ra[i][v];
-#pragma unroll
-    for (int i = 0; i < B_LD; ++i)
-#pragma unroll
-      for (int v = 0; v < VEC; ++v)
-        Bs[buf][lk + v][(lr + i * RSTEP) ^ f32_swz<VEC>(lk + v)] = rb[i][v];
   };
 
   float4_t acc[TM][TN];
@@ -115,30 +110,29 @@ __device__ __forceinline__ void gemm_nt_f32_body(
   const int nk = (kend - kbeg + BK - 1) / BK;
   if (nk > 0) {
     load_tile(kbeg);
-    store_tile(0);
+    store_tile(0, kbeg);
   }
   __syncthreads();
-  const int am = wm * (BM / WM) + (lane & 15);
-  const int bn = wn * (BN / WN) + (lane & 15);
-  const int kq = lane >> 4;
+  const int co = (lane >> 4) ^ ((lane >> 1) & 3);
+  const int am = (wm * (BM / WM) + (lane & 15)) * RCH + co;
+  const int bn = (wn * (BN / WN) + (lane & 15)) * RCH + co;
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    if (kt + 1 < nk) load_tile(kbeg + (kt + 1) * BK);
+    const int knext = kbeg + (kt + 1) * BK;
+    if (kt + 1 < nk) load_tile(knext);
+    float4_t af[TM], bf[TN];
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      float af[TM], bf[TN];
-      const int sw = f32_swz<VEC>(ks * 4 + kq);
+    for (int i = 0; i < TM; ++i) af[i] = As[cur][am + i * 16 * RCH];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = As[cur][ks * 4 + kq][(am + i * 16) ^ sw];
+    for (int j = 0; j < TN; ++j) bf[j] = Bs[cur][bn + j * 16 * RCH];
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = Bs[cur][ks * 4 + kq][(bn + j * 16) ^ sw];
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-    }
-    if (kt + 1 < nk) store_tile(cur ^ 1);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][e], bf[j][e], acc[i][j], 0, 0, 0);
+    if (kt + 1 < nk) store_tile(cur ^ 1, knext);
     __syncthreads();
   }
 
@@ -159,24 +153,24 @@ __device__ __forceinline__ void gemm_nt_f32_body(
     }
 }
 
-template <int BM, int BN, int VEC>
-__global__ __launch_bounds__(256) void gemm_nt_f32_kernel(
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_nt_f32_kernel(
     int M, int N, int K, double alpha, const double* __restrict__ A, int lda,
     const double* __restrict__ B, int ldb, double beta, double* __restrict__ C, int ldc,
     int tiles_m, int tiles_n, int k_per_split, int64_t c_split_stride) {
-  gemm_nt_f32_body<BM, BN, 2, 2, VEC>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles_m,
+  gemm_nt_f32_body<BM, BN, 2, 2>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles_m,
                                       tiles_n, k_per_split, c_split_stride, blockIdx.x,
                                       blockIdx.y);
 }
 
 // grouped: problem p owns tiles [start[p], start[p + 1]), no split-K, beta = 0
-template <int BM, int BN, int VEC>
-__global__ __launch_bounds__(256) void gemm_f32_grouped_kernel(const GemmArgs* __restrict__ args,
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_grouped_kernel(const GemmArgs* __restrict__ args,
                                                                const int* __restrict__ start,
                                                                int nprob) {
   const int p = group_of(start, nprob, blockIdx.x);
   const GemmArgs a = args[p];
-  gemm_nt_f32_body<BM, BN, 2, 2, VEC>(a.M, a.N, a.K, (double)a.alpha,
+  gemm_nt_f32_body<BM, BN, 2, 2>(a.M, a.N, a.K, (double)a.alpha,
                                       static_cast<const double*>(a.A), (int)a.lda,
                                       static_cast<const double*>(a.B), (int)a.ldb, 0.0,
                                       static_cast<double*>(a.C), (int)a.ldc, a.tiles_m, a.tiles_n,
@@ -187,21 +181,13 @@ __global__ __launch_bounds__(256) void gemm_f32_grouped_kernel(const GemmArgs* _
 template <int BM, int BN>
 int launch_f32_tiles(hipStream_t s, int M, int N, int K, double alpha, const double* A, int lda,
                      const double* B, int ldb, double beta, double* C, int ldc, int splits,
-                     int k_per_split, int64_t c_split_stride, bool vec2) {
+                     int k_per_split, int64_t c_split_stride) {
   const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   dim3 grid(tm * tn, splits);
-  if (vec2)
-    hipLaunchKernelGGL((gemm_nt_f32_kernel<BM, BN, 2>), grid, dim3(256), 0, s, M, N, K, alpha,
-                       A, lda, B, ldb, beta, C, ldc, tm, tn, k_per_split, c_split_stride);
-  else
-    hipLaunchKernelGGL((gemm_nt_f32_kernel<BM, BN, 1>), grid, dim3(256), 0, s, M, N, K, alpha,
-                       A, lda, B, ldb, beta, C, ldc, tm, tn, k_per_split, c_split_stride);
+  hipLaunchKernelGGL((gemm_nt_f32_kernel<BM, BN>), grid, dim3(256), 0, s, M, N, K, alpha, A, lda,
+                     B, ldb, beta, C, ldc, tm, tn, k_per_split, c_split_stride);
   LAUNCH_CHECK();
   return AFQMC_OK;
-}
-
-bool f32_vec2(int lda, int ldb, int K, const double* A, const double* B) {
-  return ((lda | ldb | K) % 2 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0);
 }
 
 }  // namespace
@@ -214,45 +200,32 @@ int launch_gemm_nt_f32_split(hipStream_t s, int M, int N, int K, double alpha, c
   if (splits < 1) splits = 1;
   int kps = (K + splits - 1) / splits;
   kps = (kps + F32_BK - 1) / F32_BK * F32_BK;
-  const bool vec2 = f32_vec2(lda, ldb, K, A, B);
   const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
   if (big_tiles * splits >= 512)
     return launch_f32_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits,
-                                      kps, c_split_stride, vec2);
+                                      kps, c_split_stride);
   return launch_f32_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits, kps,
-                                  c_split_stride, vec2);
+                                  c_split_stride);
 }
 
 int launch_gemm_nt_f32(hipStream_t s, int M, int N, int K, double alpha, const double* A,
                        int lda, const double* B, int ldb, double beta, double* C, int ldc) {
   if (M <= 0 || N <= 0) return AFQMC_OK;
   if (K <= 0) return afqmc_set_error(AFQMC_ERR_ARG, "gemm: K=%d", K);
-  const bool vec2 = f32_vec2(lda, ldb, K, A, B);
   const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
   if (big_tiles >= 512)
-    return launch_f32_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0,
-                                      vec2);
-  return launch_f32_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0,
-                                  vec2);
+    return launch_f32_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
+  return launch_f32_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
 }
 
-int launch_gemm_f32_grouped(hipStream_t s, int bm, bool vec2, const GemmArgs* args,
-                            const int* start, int nprob, int nblocks) {
-  if (bm == 128) {
-    if (vec2)
-      hipLaunchKernelGGL((gemm_f32_grouped_kernel<128, 128, 2>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-    else
-      hipLaunchKernelGGL((gemm_f32_grouped_kernel<128, 128, 1>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-  } else {
-    if (vec2)
-      hipLaunchKernelGGL((gemm_f32_grouped_kernel<64, 64, 2>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-    else
-      hipLaunchKernelGGL((gemm_f32_grouped_kernel<64, 64, 1>), dim3(nblocks), dim3(256), 0, s,
-                         args, start, nprob);
-  }
+int launch_gemm_f32_grouped(hipStream_t s, int bm, const GemmArgs* args, const int* start,
+                            int nprob, int nblocks) {
+  if (bm == 128)
+    hipLaunchKernelGGL((gemm_f32_grouped_kernel<128, 128>), dim3(nblocks), dim3(256), 0, s, args,
+                       start, nprob);
+  else
+    hipLaunchKernelGGL((gemm_f32_grouped_kernel<64, 64>), dim3(nblocks), dim3(256), 0, s, args,
+                       start, nprob);
   LAUNCH_CHECK();
   return AFQMC_OK;
 }

@@ -48,7 +48,6 @@ struct afqmc_group {
   bool f32 = false;           // FP32 mode: the float64 operands on float32 MFMA
   int fb_bm = 0, vhs_bm = 0;  // GEMM tile edge (0: heuristic)
   int cg_bm = 0;              // tile edge of the energy's float64 c_g product (0: heuristic)
-  bool f32_vec2 = true;       // every FP32-mode product has an even K
   // built tables
   std::vector<Launch> meas, taylor;
   Launch fb{}, vhs{}, fields{}, weights{};
@@ -94,7 +93,6 @@ int heuristic_bm(int64_t tiles128) { return tiles128 >= 512 ? 128 : 64; }
 
 int build(afqmc_group* g) {
   g->host_tab.clear();
-  g->f32_vec2 = true;
   g->meas.clear();
   g->taylor.clear();
   std::vector<unsigned char>& tab = g->host_tab;
@@ -172,7 +170,6 @@ int build(afqmc_group* g) {
           a.K = c->kdim[s];
           a.A = c->green[s];
           a.B = c->rot_chol[s];
-          if (a.K % 2) g->f32_vec2 = false;
         }
         a.lda = a.ldb = a.K;
         a.tiles_m = (a.M + bm - 1) / bm;
@@ -248,7 +245,6 @@ int build(afqmc_group* g) {
           a.A = c->xs;
           a.B = chol_t_of(c, cs);
           a.C = vhs_of(c, cs);
-          if (a.K % 2) g->f32_vec2 = false;
         }
         a.lda = a.ldb = a.K;
         a.tiles_m = (a.M + bm - 1) / bm;
@@ -644,7 +640,7 @@ int run_gemm(afqmc_group* g, const Launch& L, int out_f32) {
     return launch_gemm_bf16x3_grouped(g->stream, L.k0, out_f32, targs<GemmArgs>(g, L),
                                       tstart(g, L), L.nprob, L.nblocks);
   if (g->f32)
-    return launch_gemm_f32_grouped(g->stream, L.k0, g->f32_vec2, targs<GemmArgs>(g, L),
+    return launch_gemm_f32_grouped(g->stream, L.k0, targs<GemmArgs>(g, L),
                                    tstart(g, L), L.nprob, L.nblocks);
   return launch_gemm_f64_grouped(g->stream, L.k0, targs<GemmArgs>(g, L),
                                  tstart(g, L), L.nprob, L.nblocks);
