@@ -514,6 +514,11 @@ int launch_energy_finish_grouped(hipStream_t st, const FinishArgs* args, const i
 // vectors the QR keeps in LDS, and their bytes
 int qr_slots(int m, int n);
 size_t qr_lds_bytes(int m, int n);
+// qr_lds.hip: the other form (slots unused), and whether a context takes it
+bool qr_in_lds(const afqmc_ctx* c);
+int launch_qr_lds(hipStream_t st, int m, int n, cplx* walkers, int W);
+int launch_qr_lds_grouped(hipStream_t st, const QrArgs* args, const int* start, int nprob,
+                          int nblocks, size_t shm);
 int launch_qr_grouped(hipStream_t st, const QrArgs* args, const int* start, int nprob,
                       int nblocks, size_t shm, int max_m, int max_n);
 int launch_overlap_combine_grouped(hipStream_t st, const OvcArgs* args, const int* start,

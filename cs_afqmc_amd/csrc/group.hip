@@ -65,7 +65,7 @@ struct afqmc_group {
   bool side_ready = false;
   // block ends (afqmc_group_orthonormalize / _overlap / _energy): tables built with the
   // step's; en_ptrs are the energies outputs the finishing table was built for
-  Launch qr{}, ovc{}, fb64{}, fin{};
+  Launch qr[2]{}, ovc{}, fb64{}, fin{};  // qr: register form, LDS form
   std::vector<Launch> meas_ov, meas_en, exch;
   std::vector<void*> en_ptrs;
   // block fields draws (afqmc_group_fields_normal_key), keys the table was built for
@@ -347,35 +347,38 @@ int build(afqmc_group* g) {
 
   // ---- block ends
   {
-    // QR: one block per walker and spin
-    std::vector<QrArgs> qa;
-    std::vector<int> qs;
-    size_t qshm = 0;
-    int b = 0, max_m = 0, max_n = 0;
-    for (const Member& m : g->mem) {
-      afqmc_ctx* c = m.c;
-      for (int s = 0; s < c->nspin; ++s) {
-        const size_t lb = qr_lds_bytes(c->d.norb, c->nocc[s]);
-        QrArgs a{};
-        a.m = c->d.norb;
-        a.n = c->nocc[s];
-        a.slots = qr_slots(a.m, a.n);
-        a.walkers = s == 0 ? m.wup : m.wdn;
-        qshm = std::max(qshm, lb);
-        max_m = std::max(max_m, a.m);
-        max_n = std::max(max_n, a.n);
-        qa.push_back(a);
-        qs.push_back(b);
-        b += c->d.n_walkers;
+    // QR: one block per walker and spin, one launch per form
+    for (int form = 0; form < 2; ++form) {
+      std::vector<QrArgs> qa;
+      std::vector<int> qs;
+      size_t qshm = 0;
+      int b = 0, max_m = 0, max_n = 0;
+      for (const Member& m : g->mem) {
+        afqmc_ctx* c = m.c;
+        if (qr_in_lds(c) != (form == 1)) continue;
+        for (int s = 0; s < c->nspin; ++s) {
+          QrArgs a{};
+          a.m = c->d.norb;
+          a.n = c->nocc[s];
+          a.slots = form == 1 ? a.n : qr_slots(a.m, a.n);
+          a.walkers = s == 0 ? m.wup : m.wdn;
+          qshm = std::max(qshm, qr_lds_bytes(a.m, a.n));
+          max_m = std::max(max_m, a.m);
+          max_n = std::max(max_n, a.n);
+          qa.push_back(a);
+          qs.push_back(b);
+          b += c->d.n_walkers;
+        }
       }
+      g->qr[form] = Launch{};
+      if (qa.empty()) continue;
+      g->qr[form].shm = qshm;
+      g->qr[form].k0 = max_m;
+      g->qr[form].k1 = max_n;
+      g->qr[form].nprob = (int)qa.size();
+      g->qr[form].nblocks = b;
+      put_table(tab, g->qr[form], qa, qs);
     }
-    g->qr = Launch{};
-    g->qr.shm = qshm;
-    g->qr.k0 = max_m;
-    g->qr.k1 = max_n;
-    g->qr.nprob = (int)qa.size();
-    g->qr.nblocks = b;
-    put_table(tab, g->qr, qa, qs);
   }
   {
     // overlaps (determinants only) and Green's functions for the energy (float64, plus
@@ -819,8 +822,14 @@ extern "C" int afqmc_group_orthonormalize(afqmc_group* g) {
   int rc = group_ready(g);
   if (rc) return rc;
   PhaseTimer t(&g->prof, g->stream, AFQMC_PH_QR);
-  return launch_qr_grouped(g->stream, targs<QrArgs>(g, g->qr), tstart(g, g->qr), g->qr.nprob,
-                           g->qr.nblocks, g->qr.shm, g->qr.k0, g->qr.k1);
+  const Launch &reg = g->qr[0], &lds = g->qr[1];
+  if (reg.nprob)
+    rc = launch_qr_grouped(g->stream, targs<QrArgs>(g, reg), tstart(g, reg), reg.nprob,
+                           reg.nblocks, reg.shm, reg.k0, reg.k1);
+  if (!rc && lds.nprob)
+    rc = launch_qr_lds_grouped(g->stream, targs<QrArgs>(g, lds), tstart(g, lds), lds.nprob,
+                               lds.nblocks, lds.shm);
+  return rc;
 }
 
 extern "C" int afqmc_group_overlap(afqmc_group* g) {

@@ -338,9 +338,13 @@ int launch_qr(afqmc_ctx* c, int W, cplx* wup, cplx* wdn) {
   const int N = c->d.norb;
   for (int s = 0; s < c->nspin; ++s) {
     const int n = c->nocc[s];
-    const int rc = qr_select(N, n, [&](auto nwv, auto cpw, auto rpl) {
-      return launch_qr_t<nwv, cpw, rpl>(c->stream, N, n, s == 0 ? wup : wdn, W, qr_slots(N, n));
-    });
+    cplx* walkers = s == 0 ? wup : wdn;
+    const int rc =
+        qr_in_lds(c) ? launch_qr_lds(c->stream, N, n, walkers, W)
+                     : qr_select(N, n, [&](auto nwv, auto cpw, auto rpl) {
+                         return launch_qr_t<nwv, cpw, rpl>(c->stream, N, n, walkers, W,
+                                                           qr_slots(N, n));
+                       });
     if (rc) return rc;
   }
   return AFQMC_OK;

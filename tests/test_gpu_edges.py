@@ -192,3 +192,16 @@ def test_step_in_one_launch_matches_separate_launches(gpu, wt, norb, nelec, ncho
     for a, b in zip(one, many):
         b = [x.cpu().numpy() for x in b] if isinstance(b, list) else b.cpu().numpy()
         assert rel(a, b) < TOL
+
+
+@pytest.mark.parametrize("norb,n", [(1, 1), (9, 9), (64, 16), (65, 17), (128, 64)])
+def test_orthonormalize_mixed(gpu, norb, n):
+    """The mixed mode's QR of up to 128 orbitals; the bound of the test above."""
+    print(f"qr mixed N={norb} n={n}", flush=True)
+    hd, wd, nelec = problem("rhf", norb, (n, n), 1)
+    trial, prop, hdat, wave, _ = make("rhf", norb, nelec, 1, 3, hd, wd, "bf16x3")
+    rng = np.random.default_rng(17)
+    w = rng.standard_normal((3, norb, n)) + 1j * rng.standard_normal((3, norb, n))
+    got = hdat["_afqmc_device"].orthonormalize(to_dev(w, gpu))
+    assert np.max(np.linalg.cond(w)) < 1e4
+    assert rel(got, np.array([np.linalg.qr(x)[0] for x in w])) < 1e-11
