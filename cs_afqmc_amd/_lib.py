@@ -30,6 +30,7 @@ EXPORTS = (
     "afqmc_overlap",
     "afqmc_force_bias",
     "afqmc_energy",
+    "afqmc_energy_overlap",
     "afqmc_orthonormalize",
     "afqmc_sr",
     "afqmc_sr_key",
@@ -118,6 +119,7 @@ def _declare(lib):
     lib.afqmc_overlap.argtypes = [_vp, _i32, _vp, _vp, _vp]
     lib.afqmc_force_bias.argtypes = [_vp, _i32, _vp, _vp, _vp]
     lib.afqmc_energy.argtypes = [_vp, _i32, _vp, _vp, _vp]
+    lib.afqmc_energy_overlap.argtypes = [_vp, _i32, _vp, _vp, _vp, _vp]
     lib.afqmc_orthonormalize.argtypes = [_vp, _i32, _vp, _vp]
     lib.afqmc_sr.argtypes = [_vp, _i32, _vp, _vp, _vp, ctypes.c_double, _vp, _i32]
     lib.afqmc_sr_key.argtypes = [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _i32]

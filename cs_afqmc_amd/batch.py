@@ -105,8 +105,7 @@ class Fragment:
         self.slot, SR, overlaps, e_estimate mix.  Host bookkeeping is in record()."""
         pd = self.prop_data
         self.dev.orthonormalize(pd["walkers"])
-        self.dev.overlap(pd["walkers"], out=pd["overlaps"])
-        self.dev.energy(pd["walkers"], out=self.energies)
+        self.dev.energy(pd["walkers"], out=self.energies, overlaps=pd["overlaps"])
         self.end_block_tail()
         self.dev.overlap(pd["walkers"], out=pd["overlaps"])
 

@@ -38,8 +38,7 @@ def _field_block_end(sy):
     """corr_sample.py:541-548: QR, overlaps, block energy -> population-control shift."""
     pd = sy.pd
     sy.dev.orthonormalize(pd["walkers"])
-    sy.dev.overlap(pd["walkers"], out=pd["overlaps"])
-    en = sy.dev.energy(pd["walkers"], out=sy.energies)
+    en = sy.dev.energy(pd["walkers"], out=sy.energies, overlaps=pd["overlaps"])
     st = torch.zeros(_lib.BLOCK_STATS_LEN, dtype=torch.float64, device=sy.dev.device)
     sy.dev.block_stats(en, pd["weights"], sy.scalars, st)  # pcs <- 0.9 pcs + 0.1 E_block
     return en

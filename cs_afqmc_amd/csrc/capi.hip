@@ -546,23 +546,37 @@ extern "C" int afqmc_force_bias(afqmc_ctx* c, int32_t W, const void* walkers_up,
   return launch_fb_out(c, W, static_cast<cplx*>(force_bias));
 }
 
-extern "C" int afqmc_energy(afqmc_ctx* c, int32_t W, const void* walkers_up,
-                            const void* walkers_dn, void* energies) {
+// energies, and the walkers' overlaps where overlaps is given (the Green's function forms
+// their determinants anyway)
+static int energy_of(afqmc_ctx* c, int32_t W, const void* walkers_up, const void* walkers_dn,
+                     void* energies, void* overlaps) {
   int rc = check_w(c, W);
   if (rc) return rc;
   if ((rc = check_walkers(c, walkers_up, walkers_dn))) return rc;
   if (!energies) return afqmc_set_error(AFQMC_ERR_ARG, "null energies");
   if ((rc = set_device(c))) return rc;
   c->green_src = nullptr;
-  // Green's function in float64 (one-body term, c_g), plus split-bf16 planes for the
+  // Green's function in float64 (one-body term, c_g), plus its split-bf16 form for the
   // exchange contraction of the mixed mode
   if ((rc = launch_measure(c, W, static_cast<const cplx*>(walkers_up),
                            static_cast<const cplx*>(walkers_dn), true, c->mixed)))
     return rc;
+  if (overlaps && (rc = launch_overlap_combine(c, W, static_cast<cplx*>(overlaps)))) return rc;
   PhaseTimer t(c, AFQMC_PH_ENERGY);
   // c_g = force bias, always contracted in float64
   if ((rc = force_bias_gemm(c, W, FB_F64))) return rc;
   return launch_energy(c, W, static_cast<cplx*>(energies));
+}
+
+extern "C" int afqmc_energy(afqmc_ctx* c, int32_t W, const void* walkers_up,
+                            const void* walkers_dn, void* energies) {
+  return energy_of(c, W, walkers_up, walkers_dn, energies, nullptr);
+}
+
+extern "C" int afqmc_energy_overlap(afqmc_ctx* c, int32_t W, const void* walkers_up,
+                                    const void* walkers_dn, void* energies, void* overlaps) {
+  if (!overlaps) return afqmc_set_error(AFQMC_ERR_ARG, "null overlaps");
+  return energy_of(c, W, walkers_up, walkers_dn, energies, overlaps);
 }
 
 extern "C" int afqmc_orthonormalize(afqmc_ctx* c, int32_t W, void* walkers_up,

@@ -249,12 +249,17 @@ class DeviceStep:
         _lib.check(self._lib.afqmc_force_bias(self._h, W, _dptr(up), _dptr(dn), _dptr(out)))
         return out
 
-    def energy(self, walkers, out=None):
+    def energy(self, walkers, out=None, overlaps=None):
+        """overlaps: also receives the walkers' overlaps, as overlap(out=overlaps)."""
         up, dn, W = self._walkers(walkers)
         if out is None:
             out = torch.empty(W, dtype=torch.complex128, device=up.device)
         self._prep()
-        _lib.check(self._lib.afqmc_energy(self._h, W, _dptr(up), _dptr(dn), _dptr(out)))
+        if overlaps is None:
+            _lib.check(self._lib.afqmc_energy(self._h, W, _dptr(up), _dptr(dn), _dptr(out)))
+        else:
+            _lib.check(self._lib.afqmc_energy_overlap(self._h, W, _dptr(up), _dptr(dn),
+                                                      _dptr(out), _dptr(overlaps)))
         return out
 
     def orthonormalize(self, walkers):

@@ -59,8 +59,7 @@ class _BlockState:
             dev.propagate(self.walkers, self.weights, self.overlaps, self.fields[s], self.scalars,
                           reuse_green=s > 0, keep_green=s + 1 < self.n_prop_steps)
         dev.orthonormalize(self.walkers)
-        dev.overlap(self.walkers, out=self.overlaps)
-        en = dev.energy(self.walkers, out=self.energies)
+        en = dev.energy(self.walkers, out=self.energies, overlaps=self.overlaps)
         dev.block_stats(en, self.weights, self.scalars, self.slot)
 
     def _sr(self):

@@ -140,6 +140,11 @@ AFQMC_API int afqmc_overlap(afqmc_ctx* ctx, int32_t n_walkers, const void* walke
 AFQMC_API int afqmc_force_bias(afqmc_ctx* ctx, int32_t n_walkers, const void* walkers_up,
                      const void* walkers_dn, void* force_bias);
 
+/* afqmc_energy and afqmc_overlap of the same walkers, as a sampler block ends
+ * (sampling.py:71-73), from one evaluation of the overlap matrices; the same results. */
+AFQMC_API int afqmc_energy_overlap(afqmc_ctx* ctx, int32_t n_walkers, const void* walkers_up,
+                                   const void* walkers_dn, void* energies, void* overlaps);
+
 /* trial.calc_energy (wavefunctions.py:225-241 / :203-223) -> rhf._calc_energy_restricted
  * (wavefunctions.py:529-541) / uhf._calc_energy (:711-743): energies (W) complex128. */
 AFQMC_API int afqmc_energy(afqmc_ctx* ctx, int32_t n_walkers, const void* walkers_up,

@@ -205,3 +205,19 @@ def test_orthonormalize_mixed(gpu, norb, n):
     got = hdat["_afqmc_device"].orthonormalize(to_dev(w, gpu))
     assert np.max(np.linalg.cond(w)) < 1e4
     assert rel(got, np.array([np.linalg.qr(x)[0] for x in w])) < 1e-11
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("wt,norb,nelec,W", [("rhf", 10, (5, 5), 7), ("uhf", 30, (27, 8), 5)])
+def test_energy_with_overlaps_matches_both(gpu, wt, norb, nelec, W, precision):
+    """The block end's combined call gives the bits of the separate ones."""
+    print(f"energy with overlaps {wt} N={norb} {precision}", flush=True)
+    hd, wd, nelec = problem(wt, norb, nelec, 9)
+    trial, prop, hdat, wave, _ = make(wt, norb, nelec, 9, W, hd, wd, precision)
+    dev = hdat["_afqmc_device"]
+    w = to_dev(problems.random_walkers(wt, norb, nelec, W, np.random.default_rng(3),
+                                       near=wd["mo_coeff"], noise=0.1), gpu)
+    overlaps = torch.zeros(W, dtype=torch.complex128, device=gpu)
+    energies = dev.energy(w, overlaps=overlaps)
+    assert torch.equal(overlaps, dev.overlap(w))
+    assert torch.equal(energies, dev.energy(w))
