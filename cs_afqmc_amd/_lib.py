@@ -25,6 +25,7 @@ EXPORTS = (
     "afqmc_set_stream",
     "afqmc_ctx_device_bytes",
     "afqmc_ctx_vhs_entries",
+    "afqmc_step_plan",
     "afqmc_last_error",
     "afqmc_propagate",
     "afqmc_overlap",
@@ -113,6 +114,7 @@ def _declare(lib):
     lib.afqmc_ctx_device_bytes.restype = ctypes.c_int64
     lib.afqmc_ctx_vhs_entries.argtypes = [_vp]
     lib.afqmc_ctx_vhs_entries.restype = ctypes.c_int64
+    lib.afqmc_step_plan.argtypes = [_vp, _i32, _vp]
     lib.afqmc_last_error.argtypes = []
     lib.afqmc_last_error.restype = ctypes.c_char_p
     lib.afqmc_propagate.argtypes = [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32]

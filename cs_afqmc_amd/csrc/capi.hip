@@ -377,6 +377,14 @@ extern "C" int64_t afqmc_ctx_vhs_entries(const afqmc_ctx* ctx) {
   return ctx ? ctx->vhs_nv : 0;
 }
 
+extern "C" int afqmc_step_plan(const afqmc_ctx* ctx, int32_t W, int32_t* one_launch) {
+  const int rc = check_w(ctx, W);
+  if (rc) return rc;
+  if (!one_launch) return afqmc_set_error(AFQMC_ERR_ARG, "null plan");
+  *one_launch = small_step_fits(ctx, W) ? 1 : 0;
+  return AFQMC_OK;
+}
+
 extern "C" int afqmc_propagate(afqmc_ctx* c, int32_t W, void* walkers_up, void* walkers_dn,
                                double* weights, void* overlaps, const double* fields,
                                double* scalars, void* force_bias_out, int32_t flags) {

@@ -1372,8 +1372,15 @@ __global__ __launch_bounds__(SMALL_NT, 2) void small_step_kernel(SmallStep a) {
 //     runs through by itself: 27000 and less (norb 10, 16, 20) gain a third to a half, 43000
 //     (norb 24, n = 6, 96 vectors, 200 walkers) 297 : 249, 100000 (norb 32, n = 8, 128
 //     vectors) 339 : 393.
+// LDS grows with the vectors (two doubles each, 400 KB at norb 1 with the 25000 vectors those
+// entries allow): what one workgroup can have, or half of a CU's where two have to share it.
 constexpr int SMALL_MAX_W = 512;
 constexpr int64_t SMALL_MAX_ENTRIES = 50000;
+constexpr size_t SMALL_LDS_ONE = 156 * 1024, SMALL_LDS_TWO = 78 * 1024;
+size_t small_step_lds(const afqmc_ctx* c) {
+  return sizeof(double) * (size_t)small_doubles(c->d.norb, c->nocc[0],
+                                                c->nspin > 1 ? c->nocc[1] : 0, c->d.nchol);
+}
 bool small_step_fits(const afqmc_ctx* c, int W) {
   if (c->mixed || c->f32 || W > SMALL_MAX_W || c->d.norb > SMALL_MAX_N) return false;
   int64_t rows = (int64_t)c->chol_spins * c->vhs_nv;
@@ -1381,7 +1388,8 @@ bool small_step_fits(const afqmc_ctx* c, int W) {
     if (c->nocc[s] < 1 || c->nocc[s] > SMALL_MAX_OCC) return false;
     rows += c->kdim[s];
   }
-  return rows * c->d.nchol <= SMALL_MAX_ENTRIES;
+  if (rows * c->d.nchol > SMALL_MAX_ENTRIES) return false;
+  return small_step_lds(c) <= (W > 256 ? SMALL_LDS_TWO : SMALL_LDS_ONE);
 }
 
 int launch_small_step(afqmc_ctx* c, int W, cplx* wup, cplx* wdn, const double* fields,
@@ -1412,7 +1420,7 @@ int launch_small_step(afqmc_ctx* c, int W, cplx* wup, cplx* wdn, const double* f
   a.fields = fields;
   a.tail = tail;
   a.arrived = c->step_arrived;
-  const size_t shm = sizeof(double) * (size_t)small_doubles(a.N, a.n[0], a.n[1], a.G);
+  const size_t shm = small_step_lds(c);
   static int lds_limit = 0;
   const int rc = ensure_dyn_lds((const void*)small_step_kernel, shm, &lds_limit);
   if (rc) return rc;

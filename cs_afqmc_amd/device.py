@@ -180,6 +180,14 @@ class DeviceStep:
         """Entries of one stored VHS plane (N*N, or N(N+1)/2 for the upper triangle)."""
         return int(self._lib.afqmc_ctx_vhs_entries(self._h))
 
+    def step_in_one_launch(self, n_walkers=None):
+        """Whether a step of n_walkers walkers (default: the capacity) is one launch."""
+        one = ctypes.c_int32()
+        _lib.check(self._lib.afqmc_step_plan(
+            self._h, self.n_walkers if n_walkers is None else int(n_walkers),
+            ctypes.byref(one)))
+        return bool(one.value)
+
     def _prep(self):
         _lib.check(self._lib.afqmc_set_stream(self._h, _stream()))
 

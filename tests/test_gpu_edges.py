@@ -221,3 +221,26 @@ def test_energy_with_overlaps_matches_both(gpu, wt, norb, nelec, W, precision):
     energies = dev.energy(w, overlaps=overlaps)
     assert torch.equal(overlaps, dev.overlap(w))
     assert torch.equal(energies, dev.energy(w))
+
+
+@pytest.mark.parametrize("wt,nchol,W,one", [
+    ("rhf", 9800, 5, True), ("rhf", 10400, 5, False), ("rhf", 25000, 3, False),
+    ("uhf", 16666, 3, False), ("rhf", 4800, 300, True), ("rhf", 5200, 300, False)])
+def test_step_with_few_orbitals_and_many_vectors(gpu, wt, nchol, W, one):
+    """One orbital with as many vectors as a workgroup's LDS holds, or half of it where two
+    workgroups share a CU, takes one launch, more vectors the separate ones."""
+    print(f"vectors {wt} G={nchol} W={W}", flush=True)
+    make_problem = problems.synthetic_rhf if wt == "rhf" else problems.synthetic_uhf
+    occ = (1,) if wt == "rhf" else (1, 1)
+    # sum_g L_g^2 of order one, without decay: every vector counts
+    hd, wd, nelec = make_problem(1, *occ, nchol, seed=11, decay=1e9, chol_std=0.5 / nchol**0.5)
+    trial, prop, hdat, wave, oh = make(wt, 1, nelec, nchol, W, hd, wd)
+    assert hdat["_afqmc_device"].step_in_one_launch() == one
+    rng = np.random.default_rng(3)
+    walkers = problems.random_walkers(wt, 1, nelec, W, rng, near=wd["mo_coeff"], noise=0.1)
+    fields = rng.standard_normal((W, nchol))
+    pd, od = one_step(wt, trial, prop, hdat, wave, oh, wd, walkers, fields, gpu, 1)
+    assert np.all(od["weights"] > 0.0)
+    assert rel(pd["walkers"], od["walkers"]) < TOL
+    assert rel(pd["overlaps"], od["overlaps"]) < TOL
+    assert rel(pd["weights"], od["weights"]) < TOL
