@@ -262,6 +262,8 @@ class DeviceStep:
         up, dn, W = self._walkers(walkers)
         if out is None:
             out = torch.empty(W, dtype=torch.complex128, device=up.device)
+        if overlaps is not None:
+            self._vec(overlaps, W, torch.complex128, "overlaps")
         self._prep()
         if overlaps is None:
             _lib.check(self._lib.afqmc_energy(self._h, W, _dptr(up), _dptr(dn), _dptr(out)))
