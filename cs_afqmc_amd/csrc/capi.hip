@@ -1,6 +1,7 @@
 // C ABI of the gfx950 AFQMC step library: context lifetime, error reporting and the
 // entry points declared in include/cs_afqmc_amd.h.
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -124,7 +125,8 @@ int symmetric_vectors(afqmc_ctx* c, const double* chol, int64_t count) {
   double asym, amax;
   std::memcpy(&asym, &st[0], sizeof(double));
   std::memcpy(&amax, &st[1], sizeof(double));
-  if (asym <= (c->mixed ? 1e-12 : 0x1p-50) * amax) c->vhs_nv = N * (N + 1) / 2;
+  if (std::isfinite(amax) && asym <= (c->mixed ? 1e-12 : 0x1p-50) * amax)
+    c->vhs_nv = N * (N + 1) / 2;
   return AFQMC_OK;
 }
 

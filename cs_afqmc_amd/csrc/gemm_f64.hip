@@ -289,8 +289,9 @@ __global__ __launch_bounds__(256) void transpose_f64_kernel(int rows, int cols, 
 }
 
 // Symmetry of count n x n matrices: out[0] = max |L[p][k] - L[k][p]| and out[1] = max |L|
-// as the bit patterns of non-negative doubles (ordered like the values, so atomicMax
-// applies).  A block takes one pair (I, J), I <= J, of 32 x 32 tiles of one matrix, both
+// as the bit patterns of non-negative doubles (ordered like the values, so integer maxima
+// apply, and NaN, which fmax would drop, is the largest: vectors with an entry that is not
+// finite never count as symmetric).  A block takes one pair (I, J), I <= J, of 32 x 32 tiles of one matrix, both
 // read along rows, the second one compared through LDS.
 __global__ __launch_bounds__(256) void sym_check_kernel(int n, int nt,
                                                         const double* __restrict__ L,
@@ -301,34 +302,33 @@ __global__ __launch_bounds__(256) void sym_check_kernel(int n, int nt,
   J += I;
   const double* m = L + (int64_t)blockIdx.y * n * n;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  double asym = 0.0, amax = 0.0;
+  unsigned long long asym = 0ull, amax = 0ull;
+  auto bits = [](double x) { return (unsigned long long)__double_as_longlong(fabs(x)); };
   for (int j = ty; j < 32; j += 8) {
     const int r = J * 32 + j, c = I * 32 + tx;
     const double v = (r < n && c < n) ? m[(int64_t)r * n + c] : 0.0;
     tile[j][tx] = v;
-    amax = fmax(amax, fabs(v));
+    amax = max(amax, bits(v));
   }
   __syncthreads();
   for (int j = ty; j < 32; j += 8) {
     const int r = I * 32 + j, c = J * 32 + tx;
     if (r < n && c < n) {
       const double v = m[(int64_t)r * n + c];
-      amax = fmax(amax, fabs(v));
-      asym = fmax(asym, fabs(v - tile[tx][j]));
+      amax = max(amax, bits(v));
+      asym = max(asym, bits(v - tile[tx][j]));
     }
   }
   for (int off = 32; off > 0; off >>= 1) {
-    asym = fmax(asym, __shfl_xor(asym, off, 64));
-    amax = fmax(amax, __shfl_xor(amax, off, 64));
+    asym = max(asym, __shfl_xor(asym, off, 64));
+    amax = max(amax, __shfl_xor(amax, off, 64));
   }
   if ((threadIdx.x & 63) == 0) {
     // (a wave below the maximum so far leaves it alone: 10^5 waves share the two words)
-    const double v[2] = {asym, amax};
+    const unsigned long long v[2] = {asym, amax};
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const auto bits = (unsigned long long)__double_as_longlong(v[i]);
-      if (bits > __atomic_load_n(&out[i], __ATOMIC_RELAXED)) atomicMax(&out[i], bits);
-    }
+    for (int i = 0; i < 2; ++i)
+      if (v[i] > __atomic_load_n(&out[i], __ATOMIC_RELAXED)) atomicMax(&out[i], v[i]);
   }
 }
 

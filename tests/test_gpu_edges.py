@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from cs_afqmc_amd import hamiltonian, problems, propagation, wavefunctions
+from cs_afqmc_amd.device import DeviceStep
 from oracle import afqmc_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -244,3 +245,25 @@ def test_step_with_few_orbitals_and_many_vectors(gpu, wt, nchol, W, one):
     assert rel(pd["walkers"], od["walkers"]) < TOL
     assert rel(pd["overlaps"], od["overlaps"]) < TOL
     assert rel(pd["weights"], od["weights"]) < TOL
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+@pytest.mark.parametrize("entries", [
+    {(40, 3): np.nan}, {(3, 40): np.nan}, {(7, 7): np.nan}, {(40, 3): np.inf},
+    {(3, 40): np.inf, (40, 3): np.inf}, {(7, 7): -np.inf}])
+def test_vectors_that_are_not_finite_keep_v_whole(gpu, entries, precision):
+    """An entry that is not finite has no mirror image to stand for it, nor does it widen
+    the asymmetry that counts as rounding: V is kept whole."""
+    norb, nchol, W = 41, 5, 3
+    hd, wd, nelec = problem("rhf", norb, (4, 4), nchol)
+    trial, prop, hdat, wave, oh = make("rhf", norb, nelec, nchol, W, hd, wd, precision)
+    dev = hdat["_afqmc_device"]
+    assert dev.vhs_entries() == norb * (norb + 1) // 2
+    chol = np.array(hd["chol"]).reshape(nchol, norb, norb)
+    for at, value in entries.items():
+        chol[(2,) + at] = value
+    zeros = np.zeros
+    ctx = DeviceStep("rhf", norb, nelec, W, DT, 6, 0.0, 0.0, chol, wd["mo_coeff"],
+                     zeros((4, norb)), zeros((nchol, 4, norb)), zeros(nchol), np.eye(norb),
+                     precision=precision)
+    assert ctx.vhs_entries() == norb * norb
