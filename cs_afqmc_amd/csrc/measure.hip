@@ -989,8 +989,8 @@ struct SmallStep {
   int* arrived;  // workgroups done, 0 between launches
 };
 
-constexpr int SMALL_NT = 256, SMALL_MAX_N = 32, SMALL_MAX_OCC = 8;
-constexpr int SMALL_R = SMALL_MAX_N * SMALL_MAX_OCC * 4 / SMALL_NT;  // sums per quad
+constexpr int SMALL_NT = 256, SMALL_MAX_N = 28, SMALL_MAX_OCC = 8;
+constexpr int SMALL_R = (SMALL_MAX_N * SMALL_MAX_OCC * 4 + SMALL_NT - 1) / SMALL_NT;  // sums per quad
 
 // lane ^ 1 and lane ^ 2 of a quad
 template <int CTRL>
@@ -1365,17 +1365,30 @@ __global__ __launch_bounds__(SMALL_NT, 2) void small_step_kernel(SmallStep a) {
 
 }  // namespace
 
-// Where one launch is the better step (five steps, separate launches against one, us):
-//   - every workgroup resident at once, two to a CU: norb 16, n = 4, 64 vectors: 272 : 196 at
-//     500 walkers, 289 : 321 at 1000;
-//   - the entries of the Cholesky vectors (V's and the half-rotated ones) that each workgroup
-//     runs through by itself: 27000 and less (norb 10, 16, 20) gain a third to a half, 43000
-//     (norb 24, n = 6, 96 vectors, 200 walkers) 297 : 249, 100000 (norb 32, n = 8, 128
-//     vectors) 339 : 393.
+// Where one launch is the better step.  A workgroup runs through a walker's sums by itself, on
+// vector instructions: the entries of the Cholesky vectors (V's and the half-rotated ones),
+// one product each, and the Taylor terms, N^2 n products each on four lanes' chains, which
+// weigh four times as much a term.  Separate launches take a spin's part as often as there are
+// spins.  Hence the cost per spin, entries + 4 terms N^2 n; separate against one launch, us a
+// step (graph of 20 steps), five terms:
+//   W <= 256, a CU to a workgroup: norb 10, n = 5, 27 vectors (cost 12800) 31.3 : 19.8; norb
+//     24, n = 6, 96 vectors (112000) 40.6 : 37.6; two spins of norb 24, n = 8, 70 vectors
+//     (116000) 70.9 : 63.5; norb 26, n = 8, 40 vectors (131000) 43.0 : 42.4; norb 28, n = 7,
+//     50 vectors (140000) 43.3 : 43.7; norb 30, n = 8, 5 vectors (148000) 42.4 : 45.8
+//   to 512, two workgroups to a CU: norb 16, n = 4, 250 vectors (70500) 44.2 : 41.6; two
+//     spins of norb 20, n = 8 + 7, a set of 69 vectors each (84800) 80.9 : 78.7, n = 8 + 8,
+//     94 vectors (88900) 75.4 : 78.7; norb 20, n = 5, 100 vectors, V whole (90000) 44.1 : 45.2
+//   more walkers: norb 16, n = 4, 64 vectors, five steps 272 : 196 at 500, 289 : 321 at 1000
+// Past norb 28 a step may lose below those lines (norb 29, n = 5, 70 vectors, 122000: 41.1 :
+// 45.3; norb 31, n = 3, 40 vectors, 512 walkers, 81000: 40.5 : 42.6; two spins of norb 31, n =
+// 8 + 1, 60 vectors, 110000: 64.0 : 68.6; norb 30, n = 5 + 5, a set of 30 vectors each,
+// 108000: 70.2 : 79.7), past 50000 entries the Cholesky vectors alone are too many (norb 32,
+// n = 8, 128 vectors, five steps: 339 : 393).
 // LDS grows with the vectors (two doubles each, 400 KB at norb 1 with the 25000 vectors those
 // entries allow): what one workgroup can have, or half of a CU's where two have to share it.
 constexpr int SMALL_MAX_W = 512;
 constexpr int64_t SMALL_MAX_ENTRIES = 50000;
+constexpr int64_t SMALL_COST_ONE = 125000, SMALL_COST_TWO = 85000;
 constexpr size_t SMALL_LDS_ONE = 156 * 1024, SMALL_LDS_TWO = 78 * 1024;
 size_t small_step_lds(const afqmc_ctx* c) {
   return sizeof(double) * (size_t)small_doubles(c->d.norb, c->nocc[0],
@@ -1383,13 +1396,17 @@ size_t small_step_lds(const afqmc_ctx* c) {
 }
 bool small_step_fits(const afqmc_ctx* c, int W) {
   if (c->mixed || c->f32 || W > SMALL_MAX_W || c->d.norb > SMALL_MAX_N) return false;
-  int64_t rows = (int64_t)c->chol_spins * c->vhs_nv;
+  int64_t rows = (int64_t)c->chol_spins * c->vhs_nv, taylor = 0;
   for (int s = 0; s < c->nspin; ++s) {
     if (c->nocc[s] < 1 || c->nocc[s] > SMALL_MAX_OCC) return false;
     rows += c->kdim[s];
+    taylor += (int64_t)c->kdim[s] * c->d.norb;
   }
-  if (rows * c->d.nchol > SMALL_MAX_ENTRIES) return false;
-  return small_step_lds(c) <= (W > 256 ? SMALL_LDS_TWO : SMALL_LDS_ONE);
+  const int64_t entries = rows * c->d.nchol;
+  const int64_t cost = (entries + 4 * (c->d.n_exp_terms - 1) * taylor) / c->nspin;
+  const bool two = W > 256;  // workgroups on a CU
+  return entries <= SMALL_MAX_ENTRIES && cost <= (two ? SMALL_COST_TWO : SMALL_COST_ONE) &&
+         small_step_lds(c) <= (two ? SMALL_LDS_TWO : SMALL_LDS_ONE);
 }
 
 int launch_small_step(afqmc_ctx* c, int W, cplx* wup, cplx* wdn, const double* fields,

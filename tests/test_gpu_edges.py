@@ -9,6 +9,8 @@ import torch
 
 from cs_afqmc_amd import hamiltonian, problems, propagation, wavefunctions
 from cs_afqmc_amd.device import DeviceStep
+from cs_afqmc_amd.prop_unrestricted import propagation as spin_propagation
+from cs_afqmc_amd.prop_unrestricted import wavefunctions_unrestricted as spin_wavefunctions
 from oracle import afqmc_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -267,3 +269,62 @@ def test_vectors_that_are_not_finite_keep_v_whole(gpu, entries, precision):
                      zeros((4, norb)), zeros((nchol, 4, norb)), zeros(nchol), np.eye(norb),
                      precision=precision)
     assert ctx.vhs_entries() == norb * norb
+
+
+# both sides of the rule's lines: the cost per spin is entries + 20 norb^2 n against 125000, or
+# 85000 past 256 walkers
+@pytest.mark.parametrize("wt,norb,nelec,nchol,W,asym,one", [
+    ("rhf", 28, (7, 7), 20, 256, 0.0, True), ("rhf", 28, (7, 7), 30, 256, 0.0, False),
+    ("rhf", 28, (7, 7), 20, 257, 0.0, False), ("rhf", 24, (5, 5), 40, 512, 0.0, True),
+    ("rhf", 24, (5, 5), 70, 512, 0.0, False), ("rhf", 24, (5, 5), 40, 513, 0.0, False),
+    ("rhf", 29, (1, 1), 5, 9, 0.0, False), ("rhf", 10, (9, 9), 5, 9, 0.0, False),
+    ("rhf", 28, (4, 4), 55, 9, 1e-7, True), ("rhf", 28, (4, 4), 58, 9, 1e-7, False),
+    ("uhf", 28, (8, 1), 60, 33, 0.0, True), ("uhf", 29, (1, 1), 5, 9, 0.0, False),
+    ("uhf", 24, (8, 8), 70, 200, 0.0, True),
+    ("spin", 20, (8, 7), 69, 300, 0.0, True), ("spin", 20, (8, 7), 45, 300, 1e-7, True)])
+def test_step_route_follows_size(gpu, wt, norb, nelec, nchol, W, asym, one):
+    """Steps take one launch up to the sizes where it is the better way, and there agree
+    with the launches of the separate phases (which steps that are timed take)."""
+    print(f"route {wt} N={norb} nelec={nelec} G={nchol} W={W} asym={asym}", flush=True)
+    cs = 0.5 / np.sqrt(norb)
+    if wt == "spin":
+        hd, wd, nelec = problems.synthetic_uhf_spin(norb, *nelec, nchol, seed=11, chol_std=cs)
+    else:
+        hd, wd, nelec = problem(wt, norb, nelec, nchol)
+    chol = np.array(hd["chol"]).reshape(-1, norb, norb)
+    skew = np.random.default_rng(5).uniform(-1.0, 1.0, (norb, norb))
+    chol += asym * np.max(np.abs(chol)) * np.triu(skew, 1)[None]
+    hd = dict(hd, chol=chol.reshape(np.shape(hd["chol"])))
+    if wt == "spin":
+        trial, prop = spin_wavefunctions.uhf(norb, nelec), spin_propagation.propagator_unrestricted(
+            DT, W, precision="fp64")
+        ham = hamiltonian.hamiltonian(norb)
+        hdat = ham.build_measurement_intermediates(hd, trial, wd)
+        hdat = ham.build_propagation_intermediates(hdat, prop, trial, wd)
+    else:
+        trial, prop, hdat, _, _ = make(wt, norb, nelec, nchol, W, hd, wd)
+    dev = hdat["_afqmc_device"]
+    assert dev.vhs_entries() == (norb * norb if asym else norb * (norb + 1) // 2)
+    assert dev.step_in_one_launch() == one
+    if not one:
+        return
+    rng = np.random.default_rng(3)
+    walkers = problems.random_walkers("rhf" if wt == "rhf" else "uhf", norb, nelec, W, rng,
+                                      near=wd["mo_coeff"], noise=0.1)
+    fields = to_dev(rng.standard_normal((3, W, nchol)), gpu)
+    got = []
+    for timed in (False, True):
+        dev.prof_enable(timed)
+        w = to_dev(walkers, gpu)
+        weights = torch.ones(W, dtype=torch.float64, device=gpu)
+        overlaps = dev.overlap(w)
+        scalars = torch.tensor([-0.5, -0.5], dtype=torch.float64, device=gpu)
+        for s in range(3):
+            dev.propagate(w, weights, overlaps, fields[s], scalars, reuse_green=s > 0,
+                          keep_green=s < 2)
+        got.append((w, weights, overlaps, scalars))
+    dev.prof_enable(False)
+    assert float(got[1][1].sum()) > 0.0
+    for a, b in zip(*got):
+        b = [x.cpu().numpy() for x in b] if isinstance(b, list) else b.cpu().numpy()
+        assert rel(a, b) < TOL
