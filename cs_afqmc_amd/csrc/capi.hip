@@ -379,11 +379,13 @@ extern "C" int64_t afqmc_ctx_vhs_entries(const afqmc_ctx* ctx) {
   return ctx ? ctx->vhs_nv : 0;
 }
 
-extern "C" int afqmc_step_plan(const afqmc_ctx* ctx, int32_t W, int32_t* one_launch) {
+extern "C" int afqmc_step_plan(const afqmc_ctx* ctx, int32_t W, int32_t* plan) {
   const int rc = check_w(ctx, W);
   if (rc) return rc;
-  if (!one_launch) return afqmc_set_error(AFQMC_ERR_ARG, "null plan");
-  *one_launch = small_step_fits(ctx, W) ? 1 : 0;
+  if (!plan) return afqmc_set_error(AFQMC_ERR_ARG, "null plan");
+  plan[0] = small_step_fits(ctx, W) ? 1 : 0;
+  const auto tile = ctx->mixed ? gemm_bf16x3_tile : ctx->f32 ? gemm_f32_tile : gemm_f64_tile;
+  plan[1] = tile(2 * W, ctx->vhs_nv, 1);
   return AFQMC_OK;
 }
 

@@ -364,6 +364,10 @@ int launch_gemm_nt_f64_split(hipStream_t s, int M, int N, int K, double alpha, c
                              int lda, const double* B, int ldb, double* C, int ldc, int splits,
                              int64_t c_split_stride);
 int gemm_f64_splits(int M, int N, int K);
+// tile edge (64 or 128) of a product in `splits` splits, by precision
+int gemm_f64_tile(int M, int N, int splits);
+int gemm_f32_tile(int M, int N, int splits);
+int gemm_bf16x3_tile(int M, int N, int splits);
 // gemm_f32.hip: the same products on float32 MFMA (float64 operands rounded as staged,
 // float32 accumulation, float64 C)
 int launch_gemm_nt_f32(hipStream_t s, int M, int N, int K, double alpha, const double* A,

@@ -201,14 +201,18 @@ int gemm_bf16x3(hipStream_t s, int M, int N, int K, float alpha, const uint16_t*
   if (K <= 0 || K % BK) return afqmc_set_error(AFQMC_ERR_ARG, "bf16x3 gemm: K=%d", K);
   if (splits < 1) splits = 1;
   int kps = (K / BK + splits - 1) / splits * BK;
-  const int64_t big = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big * splits >= 512)
+  if (gemm_bf16x3_tile(M, N, splits) == 128)
     return launch_bf<128, 128, OutT>(s, M, N, K, alpha, A, B, C, ldc, splits, kps,
                                      c_split_stride);
   return launch_bf<64, 64, OutT>(s, M, N, K, alpha, A, B, C, ldc, splits, kps, c_split_stride);
 }
 
 }  // namespace
+
+// 128-wide tiles where they make two rounds of the 256 CUs
+int gemm_bf16x3_tile(int M, int N, int splits) {
+  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) * splits >= 512 ? 128 : 64;
+}
 
 int launch_split_bf16(hipStream_t s, int rows, int cols, const double* x, int64_t ld_src,
                       uint16_t* hi, uint16_t* lo, int64_t ld_dst) {

@@ -192,6 +192,11 @@ int launch_f32_tiles(hipStream_t s, int M, int N, int K, double alpha, const dou
 
 }  // namespace
 
+// 128-wide tiles where they make two rounds of the 256 CUs
+int gemm_f32_tile(int M, int N, int splits) {
+  return (int64_t)((M + 127) / 128) * ((N + 127) / 128) * splits >= 512 ? 128 : 64;
+}
+
 int launch_gemm_nt_f32_split(hipStream_t s, int M, int N, int K, double alpha, const double* A,
                              int lda, const double* B, int ldb, double* C, int ldc, int splits,
                              int64_t c_split_stride) {
@@ -200,8 +205,7 @@ int launch_gemm_nt_f32_split(hipStream_t s, int M, int N, int K, double alpha, c
   if (splits < 1) splits = 1;
   int kps = (K + splits - 1) / splits;
   kps = (kps + F32_BK - 1) / F32_BK * F32_BK;
-  const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big_tiles * splits >= 512)
+  if (gemm_f32_tile(M, N, splits) == 128)
     return launch_f32_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits,
                                       kps, c_split_stride);
   return launch_f32_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, 0.0, C, ldc, splits, kps,
@@ -212,8 +216,7 @@ int launch_gemm_nt_f32(hipStream_t s, int M, int N, int K, double alpha, const d
                        int lda, const double* B, int ldb, double beta, double* C, int ldc) {
   if (M <= 0 || N <= 0) return AFQMC_OK;
   if (K <= 0) return afqmc_set_error(AFQMC_ERR_ARG, "gemm: K=%d", K);
-  const int64_t big_tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (big_tiles >= 512)
+  if (gemm_f32_tile(M, N, 1) == 128)
     return launch_f32_tiles<128, 128>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
   return launch_f32_tiles<64, 64>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 1, K, 0);
 }

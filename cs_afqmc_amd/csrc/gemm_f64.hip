@@ -197,6 +197,8 @@ int launch_tiles(hipStream_t s, int M, int N, int K, double alpha, const double*
   return AFQMC_OK;
 }
 
+}  // namespace
+
 // Tile edge: a 128-wide tile runs at 65 TFLOP/s against 61 of a 64-wide one (8192 x 4096 x
 // 4096), but in rounds of 256 tiles (one per CU) a partly filled last round weighs more.
 // 128 where it has two rounds and still does more per round (measured at 2048 x 10000 x
@@ -209,8 +211,6 @@ int gemm_f64_tile(int M, int N, int splits) {
   const double e64 = (double)t64 / (double)((t64 + 255) / 256);
   return 65.0 * e128 > 61.0 * e64 ? 128 : 64;
 }
-
-}  // namespace
 
 int gemm_f64_splits(int M, int N, int K) {
   // split K only when the 64x64 tile grid cannot fill the 256 CUs twice over

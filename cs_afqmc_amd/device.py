@@ -182,11 +182,17 @@ class DeviceStep:
 
     def step_in_one_launch(self, n_walkers=None):
         """Whether a step of n_walkers walkers (default: the capacity) is one launch."""
-        one = ctypes.c_int32()
+        return bool(self._step_plan(n_walkers)[0])
+
+    def vhs_gemm_tile(self, n_walkers=None):
+        """Tile edge of the VHS product of a step of n_walkers walkers."""
+        return int(self._step_plan(n_walkers)[1])
+
+    def _step_plan(self, n_walkers):
+        plan = (ctypes.c_int32 * 2)()
         _lib.check(self._lib.afqmc_step_plan(
-            self._h, self.n_walkers if n_walkers is None else int(n_walkers),
-            ctypes.byref(one)))
-        return bool(one.value)
+            self._h, self.n_walkers if n_walkers is None else int(n_walkers), plan))
+        return plan
 
     def _prep(self):
         _lib.check(self._lib.afqmc_set_stream(self._h, _stream()))

@@ -106,10 +106,11 @@ AFQMC_API int64_t afqmc_ctx_device_bytes(const afqmc_ctx* ctx);
  * No counterpart in the reference: a layout query for measurement tools. */
 AFQMC_API int64_t afqmc_ctx_vhs_entries(const afqmc_ctx* ctx);
 
-/* How afqmc_propagate runs steps of n_walkers walkers on this context: *one_launch is 1
- * when a whole step is one launch (small float64 problems; steps that are timed by phase
- * or write out the force bias are separate launches all the same), else 0. */
-AFQMC_API int afqmc_step_plan(const afqmc_ctx* ctx, int32_t n_walkers, int32_t* one_launch);
+/* How afqmc_propagate runs steps of n_walkers walkers on this context: plan[0] is 1 when a
+ * whole step is one launch (small float64 problems; steps that are timed by phase or write
+ * out the force bias are separate launches all the same), else 0; plan[1] is the tile edge
+ * of the VHS product of separate launches. */
+AFQMC_API int afqmc_step_plan(const afqmc_ctx* ctx, int32_t n_walkers, int32_t plan[2]);
 AFQMC_API const char* afqmc_last_error(void);
 
 /* One phaseless step, propagator.propagate (propagation.py:100-165) with

@@ -328,3 +328,30 @@ def test_step_route_follows_size(gpu, wt, norb, nelec, nchol, W, asym, one):
     for a, b in zip(*got):
         b = [x.cpu().numpy() for x in b] if isinstance(b, list) else b.cpu().numpy()
         assert rel(a, b) < TOL
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", TOL), ("fp32", 2e-5), ("bf16x3", 1e-4)])
+@pytest.mark.parametrize("norb,n,nchol,W", [(115, 9, 37, 850), (115, 9, 32, 896)])
+def test_step_with_128_wide_gemm_tiles(gpu, norb, n, nchol, W, precision, tol):
+    """V from 128-wide GEMM tiles with partly filled last tiles in all three directions (and
+    with whole ones in rows and k), the first and last walkers against the oracle.  The
+    bounds of the reduced precisions are those their steps are held to elsewhere."""
+    print(f"128-wide tiles N={norb} n={n} G={nchol} W={W} {precision}", flush=True)
+    hd, wd, nelec = problem("rhf", norb, (n, n), nchol)
+    trial, prop, hdat, wave, oh = make("rhf", norb, nelec, nchol, W, hd, wd, precision)
+    assert hdat["_afqmc_device"].vhs_gemm_tile() == 128
+    rng = np.random.default_rng(3)
+    walkers = problems.random_walkers("rhf", norb, nelec, W, rng, near=wd["mo_coeff"], noise=0.1)
+    fields = rng.standard_normal((W, nchol))
+    pd = {"walkers": to_dev(walkers, gpu),
+          "weights": torch.ones(W, dtype=torch.float64, device=gpu),
+          "e_estimate": torch.tensor(-0.5, dtype=torch.float64, device=gpu),
+          "pop_control_ene_shift": torch.tensor(-0.5, dtype=torch.float64, device=gpu)}
+    pd["overlaps"] = trial.calc_overlap(pd["walkers"], wave)
+    pd = prop.propagate(trial, hdat, pd, to_dev(fields, gpu), wave)
+    some = np.r_[0:4, 60:68, W - 40:W]  # walkers do not depend on one another
+    od = {"walkers": walkers[some], "weights": np.ones(len(some)), "e_estimate": -0.5,
+          "overlaps": o.calc_overlap("rhf", walkers[some], wd), "pop_control_ene_shift": -0.5}
+    od = o.propagate("rhf", "rhf", oh, od, fields[some], wd, DT, 6, norb)
+    for name in ("walkers", "overlaps", "weights"):
+        assert rel(pd[name][torch.as_tensor(some, device=gpu)], od[name]) < tol
