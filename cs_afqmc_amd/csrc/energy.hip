@@ -66,6 +66,7 @@ inline int exchange_chunk(int g_tiles, int64_t tile_bytes) {
 // (tiles of more walkers, n <= 7, add up per pass instead).  Sums over threads: wave tree,
 // then the waves in order.
 constexpr int EX_NT = 256, EX_FR = 64, EX_MAXW = 8, EX_WMAX = 64;
+static_assert(2 * EX_MAXW == 16, "exchange_wave_sums");
 
 // (i, j), i <= j, of pair q = j (j + 1) / 2 + i
 struct PairTable {
@@ -83,6 +84,31 @@ __device__ inline int exchange_col_row(int col, int n) {
   const int w = (int)(((float)col + 0.5f) * (1.0f / (float)(2 * n)));
   const int e = col - w * 2 * n;
   return w * 2 * n + (e & 1) * n + (e >> 1);
+}
+
+// Sum over the wave of each of 16 values, value l / 4 in lane l: a lane adds its partner's
+// half of the values to its own and passes on the other half, 17 exchanges where a tree for
+// each value takes 96, with the same additions in the same order.  Those trees were most of
+// the reduction where a thread has few items and a tile many walkers.  Energies, us, with a
+// tree for each value and so: one vector, n = 1, 64 walkers, split-bf16, 42.6 -> 27.7; norb
+// 40, n = 6, 160 vectors, 512 walkers, split-bf16, 58.1 -> 47.0; norb 100, n = 20, 400
+// vectors, 1024 walkers, float64 1649 -> 1591, split-bf16 524 -> 447.
+template <int HALF>
+__device__ __forceinline__ void exchange_halve(double (&v)[16], int lane) {
+  const bool up = lane & (4 * HALF);
+#pragma unroll
+  for (int k = 0; k < HALF; ++k) {
+    const double mine = up ? v[HALF + k] : v[k], give = up ? v[k] : v[HALF + k];
+    v[k] = mine + __shfl_xor(give, 4 * HALF, 64);
+  }
+}
+__device__ __forceinline__ double exchange_wave_sums(double (&v)[16], int lane) {
+  exchange_halve<8>(v, lane);
+  exchange_halve<4>(v, lane);
+  exchange_halve<2>(v, lane);
+  exchange_halve<1>(v, lane);
+  v[0] += __shfl_xor(v[0], 2, 64);
+  return v[0] + __shfl_xor(v[0], 1, 64);
 }
 
 template <typename T, typename WriteF>
@@ -129,19 +155,18 @@ __device__ __forceinline__ void exchange_reduce(T* Fs, int ldf, int n, int g_use
           }
       }
       if (!persist || last) {
+        double v[2 * EX_MAXW];
 #pragma unroll
-        for (int k = 0; k < EX_MAXW; ++k)
-          if (wb + k < w_used) {
-            double vr = xr[k], vi = xi[k];
-            for (int off = 32; off > 0; off >>= 1) {
-              vr += __shfl_down(vr, off, 64);
-              vi += __shfl_down(vi, off, 64);
-            }
-            if (lane == 0) {
-              cplx* p = parts + wave * EX_WMAX + wb + k;
-              *p = g0 == 0 || persist ? cplx{vr, vi} : cplx{p->re + vr, p->im + vi};
-            }
-          }
+        for (int k = 0; k < EX_MAXW; ++k) {
+          v[k] = xr[k];
+          v[EX_MAXW + k] = xi[k];
+        }
+        const double sum = exchange_wave_sums(v, lane);
+        const int k = (lane >> 2) & (EX_MAXW - 1);
+        if ((lane & 3) == 0 && wb + k < w_used) {
+          double* p = reinterpret_cast<double*>(parts + wave * EX_WMAX + wb + k) + (lane >> 5);
+          *p = g0 == 0 || persist ? sum : *p + sum;
+        }
       }
     }
   }

@@ -355,3 +355,18 @@ def test_step_with_128_wide_gemm_tiles(gpu, norb, n, nchol, W, precision, tol):
     od = o.propagate("rhf", "rhf", oh, od, fields[some], wd, DT, 6, norb)
     for name in ("walkers", "overlaps", "weights"):
         assert rel(pd[name][torch.as_tensor(some, device=gpu)], od[name]) < tol
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", TOL), ("fp32", 2e-5), ("bf16x3", 1e-4)])
+@pytest.mark.parametrize("norb,nelec,nchol,W", [(4, (1, 1), 150, 131), (7, (2, 1), 140, 70),
+                                                (9, (4, 3), 53, 41), (12, (7, 5), 40, 65)])
+def test_energy_of_few_electrons(gpu, norb, nelec, nchol, W, precision, tol):
+    """Exchange tiles of more than eight walkers, whose sums add up over the passes, with
+    partly filled last groups of eight."""
+    print(f"exchange N={norb} nelec={nelec} G={nchol} W={W} {precision}", flush=True)
+    hd, wd, nelec = problem("uhf", norb, nelec, nchol)
+    trial, prop, hdat, wave, oh = make("uhf", norb, nelec, nchol, W, hd, wd, precision)
+    walkers = problems.random_walkers("uhf", norb, nelec, W, np.random.default_rng(3),
+                                      near=wd["mo_coeff"], noise=0.1)
+    got = trial.calc_energy(to_dev(walkers, gpu), hdat, wave)
+    assert rel(got, o.calc_energy("uhf", walkers, oh, wd)) < tol
