@@ -102,9 +102,11 @@ def phase_kernel(precision, phase, norb, nelec):
     if phase in ("overlap", "green"):
         return "measure_kernel"
     if phase == "energy":
-        return {"fp64": "exchange_f64_kernel", "fp32": "exchange_f64_kernel<F32>"}.get(
+        return {"fp64": "exchange_f64_kernel", "fp32": "exchange_f64_kernel<true"}.get(
             precision, "exchange_bf16x3_kernel")
-    return {"fields": "fields_kernel", "weights": "pcs_kernel", "qr": "qr_kernel",
+    if phase == "qr":
+        return "qr_lds_kernel" if precision == "bf16x3" and norb <= 128 else "qr_kernel"
+    return {"fields": "fields_kernel", "weights": "pcs_kernel",
             "sr": "sr_index_kernel", "rng": "normal_key_kernel"}.get(phase, phase)
 
 
@@ -629,6 +631,9 @@ def run_h10(precision, n_calls):
     timed_ph = dev.prof_collect()
     dev.prof_enable(False, phases=None)
     _, roof = dominant_roofline(precision, {dom: timed_ph[dom]}, fl, by, kern, H10_WORKLOAD)
+    if roof is not None and dev.step_in_one_launch():
+        roof["note"] = ("of a step run as separate launches, as steps timed by phase are; the "
+                        "timed calls run each step as one launch of small_step_kernel")
     return {"stats": np.concatenate(rows), "sr_idx": idx, "nchol": setup["nchol"],
             "e_hf": setup["e_hf"], "roofline": roof,
             "value": 200 * 50 * (n_calls - 2) / (ms / 1e3)}

@@ -545,7 +545,10 @@ enum TaylorKind {
 };
 
 struct TaylorPlan {
-  int kind, nkgv, ct, nthreads;
+  int kind;
+  int nkgv;  // the kernel's template key: waves (float64 register form) or k blocks of the
+             // packed [Vr | Vi] axis (split-bf16 register form)
+  int ct, nthreads;
   int nblocks;  // over the context's walker capacity
   size_t shm;
 };

@@ -3,10 +3,12 @@
 //
 // Why both stay: the next step of the mixed mode rounds Q to float32, and over the tens of
 // steps of a block a last-bit difference of Q that crosses such a rounding grows to 1e-6 of a
-// walker.  The two forms sum rows in different orders, so mixed runs of these sizes keep the
-// order they have always had; the register form would save them 22 of 1216 us at norb 100, n =
-// 20, 1024 walkers (five steps and a QR), 0.5 of 85 ms in a block of 64 fragments.  Past 128
-// orbitals it saves 1.2 of 2.1 ms a launch and more, and is used in every mode.
+// walker.  The two forms sum rows in different orders, and this one keeps the digits that
+// mixed runs of these sizes have always had, for little: the register form would save 22 of
+// 1216 us at norb 100, n = 20, 1024 walkers (five steps and a QR), 0.5 of 85 ms in a block of
+// 64 fragments.  The line is drawn by that saving, not by accuracy: past 128 orbitals it is
+// 1.2 of 2.1 ms a launch and more, the register form is used in every mode, and mixed runs
+// took on other last digits with it.
 //
 // One workgroup of four waves per (walker, spin), the walker column-major in LDS.
 #include "common.h"

@@ -1350,8 +1350,8 @@ int reg_grouped(int ct, hipStream_t st, const TaylorArgs* args, const int* start
 
 }  // namespace
 
-// Grouped Taylor launch for problems of one kernel kind and template key (nkgv bucket,
-// column tiles ct) and one block size nthreads = 64 * ceil(N / 16).
+// Grouped Taylor launch for problems of one kernel kind and template key (nkgv, column
+// tiles ct) and one block size nthreads = 64 * ceil(N / 16).
 int launch_taylor_grouped(hipStream_t st, int kind, int nkgv, int ct, const TaylorArgs* args,
                           const int* start, int nprob, int nblocks, int nthreads, size_t shm) {
   if (kind == TAYLOR_REG_F64) {
