@@ -591,9 +591,9 @@ __device__ __forceinline__ void measure_narrow_body(
 //     exchanged and the first negated.  One 16-byte load of the walker feeds both.
 // Per walker at norb 200, n = 40 and two walkers per CU, in cycles (MFMA alone in brackets):
 // overlaps 44k (13k), inversion 82k, Green's function 55k (26k); with the operands read as
-// they came (X through both maps for each tile) it was 42k, 83k and 108k.  2048 walkers:
-// 442 -> 330 us; norb 131, n = 29, 777 walkers: 124 -> 85 us; norb 250, n = 50, 512: 310 ->
-// 170 us.
+// they came (X through both maps for each tile) it was 42k, 83k and 108k.  A launch with the
+// float64 Green's function, 2048 walkers: 455 -> 335 us; norb 131, n = 29, 777 walkers: 131 ->
+// 75 us; norb 250, n = 50, 512: 321 -> 184 us.
 constexpr int MW_KC = 16;  // rows per chunk of the overlap product
 // doubles per LDS row: 16 T2 columns, == 16 (mod 32), so rows k and k + 1 meet different
 // bank halves
